@@ -61,10 +61,10 @@ typedef enum ckan_input_map {
  * batch of `batch` rows (kan/layers/chebykan.py:21-22,64).
  * Degrees 0..16 run on the MFMA kernels in the compute precision.  Degrees
  * 17..1024 (the reference layer takes any degree, kan/layers/chebykan.py:21-51)
- * run on vector-ALU kernels in fp32 whatever `compute` asks, with either input
- * map; their packed buffer is C widened to fp32 in its own [in, out, D]
- * layout followed by the basis recurrence block, and they need no workspace
- * (the size queries return 0). */
+ * run on the general kernels (fp32 matrix instructions) in fp32 whatever
+ * `compute` asks, with either input map; their packed buffer is C widened to
+ * fp32 in its own [in, out, D] layout followed by the basis recurrence block,
+ * and they need no workspace (the size queries return 0). */
 typedef struct ckan_desc {
   int64_t batch;        /* B: rows of x after x.view(-1, in_dim)          */
   int32_t in_dim;       /* I                                               */
@@ -154,7 +154,7 @@ int ckan_backward(const ckan_desc* desc, const float* t_cache, const void* packe
  * The reference layer computes in fp64 when its parameter is fp64
  * (kan/layers/chebykan.py:48-51 after .double(); kan/basis/chebyshev.py:78-101
  * then runs in fp64).  These entry points run that case in fp64 end to end
- * (fp64 FMA on the vector ALU).  x, coeffs [in, out, D], y, t_cache [B, in],
+ * (fp64 matrix instructions).  x, coeffs [in, out, D], y, t_cache [B, in],
  * dy, dx and dcoeffs are fp64; desc->compute and desc->coeff_dtype must be 0.
  * No packing and no workspace: coeffs are read in their own layout.
  * Same formulas, NULL rules and accumulate semantics as ckan_forward /
@@ -192,7 +192,7 @@ int ckan_backward_f64_basis(const ckan_desc* desc, const double* rec, const doub
  * ChebyKAN layer's with C'.  So ckan_pack_coeffs_basis + ckan_forward +
  * ckan_backward (into dC') + ckan_coeff_grad_from_chebyshev run such a layer
  * (ckan_backward_basis: the last two in one call).
- * Above degree 16 (the vector-ALU kernels) the packed buffer carries the
+ * Above degree 16 (the general kernels) the packed buffer carries the
  * family's recurrence instead of C M: the kernels evaluate P_n(s u) by the
  * recurrence and differentiate it, ckan_backward's dC is already the family
  * coefficients' gradient and ckan_coeff_grad_from_chebyshev is the identity
@@ -373,7 +373,7 @@ int ckan_exec_create(const ckan_exec_config* cfg, ckan_exec** out, void* stream)
  * coefficients (ckan_exec_set/get_coeffs, Adam state) are those of its own
  * basis.  Family layers up to degree 16 train through the change of basis
  * into Chebyshev coefficients (gradient mapped back by the transpose before
- * the optimizer step); above it, on the vector-ALU recurrence. */
+ * the optimizer step); above it, on the family's recurrence. */
 int ckan_exec_create_basis(const ckan_exec_config* cfg, const struct ckan_basis_spec* bases,
                            const float* affine, ckan_exec** out, void* stream);
 int ckan_exec_destroy(ckan_exec* ex);

@@ -75,9 +75,9 @@ int validate_desc(const ckan_desc* d) {
   if (d->in_dim < 1) return fail(CKAN_ERR_INVALID_ARG, "in_dim must be >= 1 (got %d)", d->in_dim);
   if (d->out_dim < 1) return fail(CKAN_ERR_INVALID_ARG, "out_dim must be >= 1 (got %d)", d->out_dim);
   if (d->degree < 0) return fail(CKAN_ERR_INVALID_ARG, "degree must be >= 0 (got %d)", d->degree);
-  if (d->degree > kValuMaxDegree)
+  if (d->degree > kGeneralMaxDegree)
     return fail(CKAN_ERR_UNSUPPORTED, "degree %d > %d is not supported by this build", d->degree,
-                kValuMaxDegree);
+                kGeneralMaxDegree);
   if (d->compute != CKAN_COMPUTE_FP32 && d->compute != CKAN_COMPUTE_BF16)
     return fail(CKAN_ERR_INVALID_ARG, "unknown compute mode %d", d->compute);
   if (d->coeff_dtype != CKAN_DTYPE_F32 && d->coeff_dtype != CKAN_DTYPE_BF16)
@@ -108,29 +108,39 @@ Plan plan_of(const ckan_desc* d) {
   return p;
 }
 
-// Layers above the MFMA kernels' degree limit run on the vector-ALU kernels
+// Layers above the packed kernels' degree limit run on the general kernels
 // in fp32 (whatever desc->compute asks).  Their packed buffer is C copied to
 // fp32 in its own [I, O, D] layout, then (at the next 256-byte boundary) the
 // basis recurrence block; the input-map cache has row pitch I.
-inline bool valu_route(const ckan_desc* d) { return d->degree > kMfmaMaxDegree; }
-inline int64_t valu_coeffs(const ckan_desc* d) {
+inline bool general_route(const ckan_desc* d) { return d->degree > kMfmaMaxDegree; }
+inline int64_t general_coeffs(const ckan_desc* d) {
   return (int64_t)d->in_dim * d->out_dim * (d->degree + 1);
 }
-inline size_t valu_rec_offset(const ckan_desc* d) {
-  return align256((size_t)valu_coeffs(d) * sizeof(float));
+inline size_t general_rec_offset(const ckan_desc* d) {
+  return align256((size_t)general_coeffs(d) * sizeof(float));
 }
-inline float* valu_rec(const ckan_desc* d, void* packed) {
-  return reinterpret_cast<float*>(static_cast<char*>(packed) + valu_rec_offset(d));
+inline float* general_rec(const ckan_desc* d, void* packed) {
+  return reinterpret_cast<float*>(static_cast<char*>(packed) + general_rec_offset(d));
 }
-inline const float* valu_rec(const ckan_desc* d, const void* packed) {
-  return reinterpret_cast<const float*>(static_cast<const char*>(packed) + valu_rec_offset(d));
+inline const float* general_rec(const ckan_desc* d, const void* packed) {
+  return reinterpret_cast<const float*>(static_cast<const char*>(packed) + general_rec_offset(d));
 }
 
-// The vector-ALU dx launch puts 8 inputs per block on grid y (at most 65535).
-int valu_backward_shape_ok(const ckan_desc* d) {
+// The dimensions that the general kernels take: their 32-bit byte offsets
+// span a few rows of t and dy.
+int general_forward_shape_ok(const ckan_desc* d) {
+  if (d->out_dim > 64 * 65535)
+    return fail(CKAN_ERR_UNSUPPORTED, "out_dim %d above %d is not supported by the general "
+                "forward (degree above 16 or fp64)", d->out_dim, 64 * 65535);
+  return CKAN_OK;
+}
+int general_backward_shape_ok(const ckan_desc* d) {
   if ((d->in_dim + 7) / 8 > 65535)
-    return fail(CKAN_ERR_UNSUPPORTED, "in_dim %d above 524280 is not supported by the vector-ALU "
+    return fail(CKAN_ERR_UNSUPPORTED, "in_dim %d above 524280 is not supported by the general "
                 "backward (degree above 16 or fp64)", d->in_dim);
+  if (d->out_dim > 128 * 65535)
+    return fail(CKAN_ERR_UNSUPPORTED, "out_dim %d above %d is not supported by the general "
+                "backward (degree above 16 or fp64)", d->out_dim, 128 * 65535);
   return CKAN_OK;
 }
 
@@ -208,25 +218,25 @@ int backward_core(const ckan_desc* desc, const float* t_cache, const void* packe
   const bool need_dx = dx != nullptr, need_dc = dcoeffs != nullptr;
   if (!need_dx && !need_dc) return CKAN_OK;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (valu_route(desc)) {
-    if ((rc = valu_backward_shape_ok(desc))) return rc;
+  if (general_route(desc)) {
+    if ((rc = general_backward_shape_ok(desc))) return rc;
     if (desc->batch == 0) {
       if (need_dc && om.mode >= kDcSgd)
         return fail(CKAN_ERR_UNSUPPORTED, "backward: an optimizer-applying call needs batch >= 1");
       if (need_dc && om.mode == kDcStore) {
-        launch_zero_f32(dcoeffs, valu_coeffs(desc), s);
+        launch_zero_f32(dcoeffs, general_coeffs(desc), s);
         return check_launch("zero dcoeffs");
       }
       return CKAN_OK;
     }
     // packed carries the basis recurrence: required for dC as well
     if (!t_cache || !dy || !packed) return fail(CKAN_ERR_INVALID_ARG, "t_cache/dy/packed is NULL");
-    ProfScope ps("bwd_valu", s);
-    launch_backward_valu<float>(t_cache, static_cast<const float*>(packed), dy, dx, dcoeffs, om,
+    ProfScope ps("bwd_general", s);
+    launch_backward_general<float>(t_cache, static_cast<const float*>(packed), dy, dx, dcoeffs, om,
                                 desc->batch, desc->in_dim, desc->out_dim, desc->degree, s,
-                                packed ? valu_rec(desc, packed) : nullptr, desc->input_map,
+                                packed ? general_rec(desc, packed) : nullptr, desc->input_map,
                                 desc->in_scale);
-    return check_launch("backward (vector ALU)");
+    return check_launch("backward (general)");
   }
   const Plan p = plan_of(desc);
   if (p.B == 0) {
@@ -313,27 +323,27 @@ const char* ckan_version(void) { return "kan_amd-chebykan 0.1.0 (gfx950)"; }
 
 size_t ckan_packed_bytes(const ckan_desc* desc) {
   if (validate_desc(desc) != CKAN_OK) return 0;
-  if (valu_route(desc))
-    return valu_rec_offset(desc) + align256((size_t)recur_floats(desc->degree) * sizeof(float));
+  if (general_route(desc))
+    return general_rec_offset(desc) + align256((size_t)recur_floats(desc->degree) * sizeof(float));
   return packed_bytes(plan_of(desc));
 }
 
 size_t ckan_tcache_elems(const ckan_desc* desc) {
   if (validate_desc(desc) != CKAN_OK) return 0;
-  if (valu_route(desc)) return (size_t)desc->batch * desc->in_dim;
+  if (general_route(desc)) return (size_t)desc->batch * desc->in_dim;
   const Plan p = plan_of(desc);
   return (size_t)p.B * p.I_sg;
 }
 
 size_t ckan_fwd_workspace_bytes(const ckan_desc* desc) {
-  if (validate_desc(desc) != CKAN_OK || valu_route(desc)) return 0;
+  if (validate_desc(desc) != CKAN_OK || general_route(desc)) return 0;
   const Plan p = plan_of(desc);
   if (p.B == 0) return 0;
   return fwd_ws_bytes(p, choose_fwd(p));
 }
 
 size_t ckan_bwd_workspace_bytes(const ckan_desc* desc, int need_dx, int need_dcoeffs) {
-  if (validate_desc(desc) != CKAN_OK || valu_route(desc)) return 0;
+  if (validate_desc(desc) != CKAN_OK || general_route(desc)) return 0;
   const Plan p = plan_of(desc);
   return bwd_layout(p, need_dx != 0, need_dcoeffs != 0).total;
 }
@@ -355,11 +365,11 @@ int ckan_pack_coeffs(const ckan_desc* desc, const void* coeffs, void* packed, vo
   if (!coeffs || !packed) return fail(CKAN_ERR_INVALID_ARG, "coeffs/packed is NULL");
   if (!aligned16(packed)) return fail(CKAN_ERR_INVALID_ARG, "packed buffer must be 16-byte aligned");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (valu_route(desc)) {  // C in fp32 and the Chebyshev recurrence block
+  if (general_route(desc)) {  // C in fp32 and the Chebyshev recurrence block
     ProfScope ps("pack", s);
     launch_to_f32(coeffs, desc->coeff_dtype == CKAN_DTYPE_BF16, static_cast<float*>(packed),
-                  valu_coeffs(desc), s);
-    launch_write_recur(valu_rec(desc, packed), CKAN_BASIS_CHEBYSHEV, 0.0, 0.0, desc->degree, 1.0f, s);
+                  general_coeffs(desc), s);
+    launch_write_recur(general_rec(desc, packed), CKAN_BASIS_CHEBYSHEV, 0.0, 0.0, desc->degree, 1.0f, s);
     return check_launch("pack_coeffs");
   }
   const Plan p = plan_of(desc);
@@ -377,14 +387,15 @@ int ckan_forward(const ckan_desc* desc, const float* x, const void* packed, floa
     return fail(CKAN_ERR_INVALID_ARG, "x/packed/y/t_cache is NULL");
   if (!aligned16(packed) || !aligned16(t_cache))
     return fail(CKAN_ERR_INVALID_ARG, "packed and t_cache must be 16-byte aligned");
-  if (valu_route(desc)) {
+  if (general_route(desc)) {
+    if ((rc = general_forward_shape_ok(desc))) return rc;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    ProfScope ps("fwd_valu", s);
-    launch_forward_valu<float>(x, static_cast<const float*>(packed), y, t_cache, desc->batch,
+    ProfScope ps("fwd_general", s);
+    launch_forward_general<float>(x, static_cast<const float*>(packed), y, t_cache, desc->batch,
                                desc->in_dim, desc->out_dim, desc->degree, s,
-                               valu_rec(desc, packed), desc->input_map, desc->in_scale,
+                               general_rec(desc, packed), desc->input_map, desc->in_scale,
                                desc->in_shift);
-    return check_launch("forward (vector ALU)");
+    return check_launch("forward (general)");
   }
   const Plan p = plan_of(desc);
   const FwdChoice c = choose_fwd(p);
@@ -450,7 +461,7 @@ int pack_forward_impl(const ckan_desc* desc, const ckan_basis_spec* spec, const 
                       size_t ws_bytes, void* stream, bool t_ready, bool out_tanh) {
   int rc = validate_desc(desc);
   if (rc) return rc;
-  if (valu_route(desc)) {
+  if (general_route(desc)) {
     rc = spec ? ckan_pack_coeffs_basis(desc, spec, coeffs, packed, stream)
               : ckan_pack_coeffs(desc, coeffs, packed, stream);
     if (rc) return rc;
@@ -547,9 +558,10 @@ int forward_f64_impl(const ckan_desc* desc, const double* rec, const double* x,
   if ((rc = require_tanh_map(desc, "fp64 path"))) return rc;
   if (desc->batch == 0) return CKAN_OK;
   if (!x || !coeffs || !y || !t_cache) return fail(CKAN_ERR_INVALID_ARG, "x/coeffs/y/t_cache is NULL");
+  if ((rc = general_forward_shape_ok(desc))) return rc;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   ProfScope ps("fwd_f64", s);
-  launch_forward_valu<double>(x, coeffs, y, t_cache, desc->batch, desc->in_dim,
+  launch_forward_general<double>(x, coeffs, y, t_cache, desc->batch, desc->in_dim,
                               desc->out_dim, desc->degree, s, rec);
   return check_launch("forward_f64");
 }
@@ -562,7 +574,7 @@ int backward_f64_impl(const ckan_desc* desc, const double* rec, const double* t_
   if (desc->compute != CKAN_COMPUTE_FP32 || desc->coeff_dtype != CKAN_DTYPE_F32)
     return fail(CKAN_ERR_INVALID_ARG, "fp64 path: desc->compute and desc->coeff_dtype must be 0");
   if ((rc = require_tanh_map(desc, "fp64 path"))) return rc;
-  if ((rc = valu_backward_shape_ok(desc))) return rc;
+  if ((rc = general_backward_shape_ok(desc))) return rc;
   if (!dx && !dcoeffs) return CKAN_OK;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (desc->batch == 0) {
@@ -577,7 +589,7 @@ int backward_f64_impl(const ckan_desc* desc, const double* rec, const double* t_
     return fail(CKAN_ERR_INVALID_ARG, "t_cache/dy/coeffs is NULL");
   ProfScope ps("bwd_f64", s);
   const DcOut om{accumulate ? kDcAccumulate : kDcStore};
-  launch_backward_valu<double>(t_cache, coeffs, dy, dx, dcoeffs, om, desc->batch, desc->in_dim,
+  launch_backward_general<double>(t_cache, coeffs, dy, dx, dcoeffs, om, desc->batch, desc->in_dim,
                                desc->out_dim, desc->degree, s, rec);
   return check_launch("backward_f64");
 }
@@ -610,7 +622,7 @@ int family_of(const ckan_basis_spec* spec, int degree, double* a, double* b, dou
   return CKAN_OK;
 }
 
-// Validates a basis spec of a layer of degree `degree` up to the vector-ALU
+// Validates a basis spec of a layer of degree `degree` up to the general
 // path's limit (the recurrence-block form of the basis has no matrix).
 int family_valid(const ckan_basis_spec* spec, int degree) {
   if (!spec) return fail(CKAN_ERR_INVALID_ARG, "basis spec is NULL");
@@ -640,15 +652,15 @@ int family_xform(const ckan_basis_spec* spec, int degree, BasisXform* xf) {
 }  // namespace
 
 size_t ckan_recurrence_bytes_f64(const ckan_basis_spec* spec) {
-  if (!spec || spec->degree < 0 || spec->degree > kValuMaxDegree) return 0;
+  if (!spec || spec->degree < 0 || spec->degree > kGeneralMaxDegree) return 0;
   return (size_t)(3 * (spec->degree + 1) + 2) * sizeof(double);
 }
 
 int ckan_write_recurrence_f64(const ckan_basis_spec* spec, double* rec, void* stream) {
   if (!spec) return fail(CKAN_ERR_INVALID_ARG, "basis spec is NULL");
-  if (spec->degree < 0 || spec->degree > kValuMaxDegree)
+  if (spec->degree < 0 || spec->degree > kGeneralMaxDegree)
     return fail(spec->degree < 0 ? CKAN_ERR_INVALID_ARG : CKAN_ERR_UNSUPPORTED,
-                "basis degree %d outside 0..%d", spec->degree, kValuMaxDegree);
+                "basis degree %d outside 0..%d", spec->degree, kGeneralMaxDegree);
   int rc = family_valid(spec, spec->degree);
   if (rc) return rc;
   if (!rec) return fail(CKAN_ERR_INVALID_ARG, "rec is NULL");
@@ -685,14 +697,14 @@ int ckan_pack_coeffs_basis(const ckan_desc* desc, const ckan_basis_spec* spec, c
   int rc = validate_desc(desc);
   if (rc) return rc;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (valu_route(desc)) {  // C in fp32 and the family's recurrence block
+  if (general_route(desc)) {  // C in fp32 and the family's recurrence block
     if ((rc = family_valid(spec, desc->degree))) return rc;
     if (!coeffs || !packed) return fail(CKAN_ERR_INVALID_ARG, "coeffs/packed is NULL");
     if (!aligned16(packed)) return fail(CKAN_ERR_INVALID_ARG, "packed buffer must be 16-byte aligned");
     ProfScope ps("pack", s);
     launch_to_f32(coeffs, desc->coeff_dtype == CKAN_DTYPE_BF16, static_cast<float*>(packed),
-                  valu_coeffs(desc), s);
-    launch_write_recur(valu_rec(desc, packed), spec->family, spec->alpha, spec->beta, desc->degree,
+                  general_coeffs(desc), s);
+    launch_write_recur(general_rec(desc, packed), spec->family, spec->alpha, spec->beta, desc->degree,
                        (float)spec->scale, s);
     return check_launch("pack_coeffs_basis");
   }
@@ -711,8 +723,8 @@ int ckan_coeff_grad_from_chebyshev(const ckan_desc* desc, const ckan_basis_spec*
   int rc = validate_desc(desc);
   if (rc) return rc;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (valu_route(desc)) {
-    // the vector-ALU backward already differentiates in the family's basis:
+  if (general_route(desc)) {
+    // the general backward already differentiates in the family's basis:
     // the map is the identity (a copy, an accumulation, or nothing in place)
     if ((rc = family_valid(spec, desc->degree))) return rc;
     if (!dcheb || !dcoeffs) return fail(CKAN_ERR_INVALID_ARG, "dcheb/dcoeffs is NULL");
@@ -720,7 +732,7 @@ int ckan_coeff_grad_from_chebyshev(const ckan_desc* desc, const ckan_basis_spec*
       return fail(CKAN_ERR_INVALID_ARG, "in-place transform (dcheb == dcoeffs) cannot accumulate");
     if (dcheb == dcoeffs) return CKAN_OK;
     ProfScope ps("coeff_from_cheb", s);
-    launch_to_f32(dcheb, false, dcoeffs, valu_coeffs(desc), s, accumulate != 0);
+    launch_to_f32(dcheb, false, dcoeffs, general_coeffs(desc), s, accumulate != 0);
     return check_launch("coeff_grad_from_chebyshev");
   }
   BasisXform xf;
@@ -740,8 +752,8 @@ int ckan_backward_basis(const ckan_desc* desc, const ckan_basis_spec* spec, cons
   int rc = validate_desc(desc);
   if (rc) return rc;
   const DcOut om{kDcStore};
-  if (valu_route(desc)) {
-    // the vector-ALU backward differentiates in the family's basis already
+  if (general_route(desc)) {
+    // the general backward differentiates in the family's basis already
     if ((rc = family_valid(spec, desc->degree))) return rc;
     return backward_impl(desc, t_cache, packed, dy, dx, dcoeffs, om, ws, ws_bytes, stream);
   }
@@ -917,9 +929,9 @@ int ckan_family_basis(const ckan_basis_spec* spec, const float* t, int64_t n, fl
                       void* stream) {
   int rc = family_valid(spec, spec ? spec->degree : 0);
   if (rc) return rc;
-  if (spec->degree < 0 || spec->degree > kValuMaxDegree)
+  if (spec->degree < 0 || spec->degree > kGeneralMaxDegree)
     return fail(spec->degree < 0 ? CKAN_ERR_INVALID_ARG : CKAN_ERR_UNSUPPORTED,
-                "basis degree %d outside 0..%d", spec->degree, kValuMaxDegree);
+                "basis degree %d outside 0..%d", spec->degree, kGeneralMaxDegree);
   if (n < 0) return fail(CKAN_ERR_INVALID_ARG, "n must be >= 0");
   if (n == 0) return CKAN_OK;
   if (!t || !out) return fail(CKAN_ERR_INVALID_ARG, "t/out is NULL");
@@ -933,9 +945,9 @@ int ckan_family_basis_backward(const ckan_basis_spec* spec, const float* t, cons
                                int64_t n, float* dt, void* stream) {
   int rc = family_valid(spec, spec ? spec->degree : 0);
   if (rc) return rc;
-  if (spec->degree < 0 || spec->degree > kValuMaxDegree)
+  if (spec->degree < 0 || spec->degree > kGeneralMaxDegree)
     return fail(spec->degree < 0 ? CKAN_ERR_INVALID_ARG : CKAN_ERR_UNSUPPORTED,
-                "basis degree %d outside 0..%d", spec->degree, kValuMaxDegree);
+                "basis degree %d outside 0..%d", spec->degree, kGeneralMaxDegree);
   if (n < 0) return fail(CKAN_ERR_INVALID_ARG, "n must be >= 0");
   if (n == 0) return CKAN_OK;
   if (!t || !g || !dt) return fail(CKAN_ERR_INVALID_ARG, "t/g/dt is NULL");
@@ -1025,18 +1037,18 @@ size_t ckan_profile_report(char* buf, size_t len) {
 }  // extern "C"
 
 bool ckan::layer_reads_tcache(const ckan_desc* desc) {
-  if (validate_desc(desc) != CKAN_OK || valu_route(desc)) return false;
+  if (validate_desc(desc) != CKAN_OK || general_route(desc)) return false;
   const Plan p = plan_of(desc);
   return p.I == p.I_sg && fwd_reads_tcache(choose_fwd(p));
 }
 
 bool ckan::layer_out_tanh_ok(const ckan_desc* desc) {
-  if (validate_desc(desc) != CKAN_OK || valu_route(desc)) return false;
+  if (validate_desc(desc) != CKAN_OK || general_route(desc)) return false;
   return fwd_out_tanh_ok(plan_of(desc));
 }
 
 bool ckan::pack_pair_fits(const ckan_desc* a, const ckan_desc* b) {
-  if (validate_desc(a) != CKAN_OK || validate_desc(b) != CKAN_OK || valu_route(a) || valu_route(b))
+  if (validate_desc(a) != CKAN_OK || validate_desc(b) != CKAN_OK || general_route(a) || general_route(b))
     return false;
   if (a->coeff_dtype != CKAN_DTYPE_F32 || b->coeff_dtype != CKAN_DTYPE_F32) return false;
   if (a->batch != b->batch || a->out_dim != b->in_dim || a->batch < 1) return false;
@@ -1133,7 +1145,7 @@ bool ckan::self_pack_pair_fits(const ckan_desc* a, const ckan_desc* b) {
 }
 
 int ckan::self_pack_layer(const ckan_desc* desc, const void* C, void* packed, void* stream) {
-  if (validate_desc(desc) != CKAN_OK || valu_route(desc))
+  if (validate_desc(desc) != CKAN_OK || general_route(desc))
     return fail(CKAN_ERR_INVALID_ARG, "self_pack_layer: not a packed-kernel layer");
   if (!C || !packed || !aligned16(packed))
     return fail(CKAN_ERR_INVALID_ARG, "self_pack_layer: NULL or misaligned buffer");
@@ -1208,7 +1220,7 @@ int ckan::pack_forward_ex(const ckan_desc* desc, const void* coeffs, void* packe
                            t_ready, out_tanh);
 }
 
-bool ckan::layer_on_valu(const ckan_desc* desc) { return valu_route(desc); }
+bool ckan::layer_is_general(const ckan_desc* desc) { return general_route(desc); }
 
 int ckan::basis_check(const ckan_basis_spec* spec, int degree, BasisXform* xf) {
   if (degree > kMfmaMaxDegree) return family_valid(spec, degree);

@@ -491,7 +491,7 @@ struct ckan_exec {
     // kMfmaMaxDegree its pack multiplies C by the change of basis M into
     // Chebyshev coefficients C' = C M; its dC kernels then produce dC', and one
     // more launch forms dC = dC' M^T and applies the optimizer step to C.
-    // Above it the vector-ALU backward differentiates in the family's basis
+    // Above it the general backward differentiates in the family's basis
     // and applies the step itself, as for a Chebyshev layer.
     bool family = false;
     ckan_basis_spec spec{};
@@ -738,7 +738,7 @@ int run_step(ckan_exec* ex, const float* x, const void* target, hipStream_t s,
     float* dx = l > 0 ? ex->layers[l - 1].dy : nullptr;
     const DcOut om = step_mode(ex, ly);
     const LossMean* lm = tail && l == L - 1 ? &lm_tail : nullptr;
-    if (ly.family && !layer_on_valu(&ly.desc)) {
+    if (ly.family && !layer_is_general(&ly.desc)) {
       // dC' into gcheb, then dC = dC' M^T and the optimizer step into C
       if ((rc = backward_impl(&ly.desc, ly.t, ly.packed, ly.dy, dx, ex->gcheb, DcOut{kDcStore},
                               ex->bws, ex->bws_bytes, s, lm)))
@@ -817,7 +817,7 @@ int ckan_exec_create_basis(const ckan_exec_config* cfg, const ckan_basis_spec* b
       if (ly.family && (rc = basis_check(&ly.spec, ly.desc.degree, &ly.xf))) break;
     }
     ly.ncoef = (int64_t)ly.desc.in_dim * ly.desc.out_dim * (ly.desc.degree + 1);
-    if (ly.family && !layer_on_valu(&ly.desc) && ly.ncoef > gcheb_elems) gcheb_elems = ly.ncoef;
+    if (ly.family && !layer_is_general(&ly.desc) && ly.ncoef > gcheb_elems) gcheb_elems = ly.ncoef;
     const int64_t ny = cfg->batch * ly.desc.out_dim;
     if ((rc = dev_alloc(ex, (void**)&ly.C, ly.ncoef * 4)) ||
         (rc = dev_alloc(ex, &ly.packed, ly.packed_bytes)) ||

@@ -74,7 +74,7 @@ bool family_recurrence(int family, int degree, double alpha, double beta, double
   return recur_coef(family, 0, alpha, beta, a, b, c);  // also checks the family at degree 0
 }
 
-// The recurrence block of a vector-ALU packed buffer: a[D], b[D], c[D], the
+// The recurrence block of a general-path packed buffer: a[D], b[D], c[D], the
 // basis scale s (P_n is evaluated at s * t) and the kind: 0 for the Chebyshev
 // basis at scale 1 (the kernels' specialised recurrence), 1 otherwise.
 __global__ void k_write_recur(float* __restrict__ rec, int family, double alpha, double beta, int D,
@@ -350,7 +350,7 @@ __device__ __forceinline__ void stage_family(float* ra, float* rb, float* rc, in
 __global__ void __launch_bounds__(256)
 k_basis_family(const float* __restrict__ t, int64_t n, int deg, int family, double alpha,
                double beta, float* __restrict__ out) {
-  __shared__ float ra[kValuMaxDegree + 1], rb[kValuMaxDegree + 1], rc[kValuMaxDegree + 1];
+  __shared__ float ra[kGeneralMaxDegree + 1], rb[kGeneralMaxDegree + 1], rc[kGeneralMaxDegree + 1];
   stage_family(ra, rb, rc, deg, family, alpha, beta);
   for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < n;
        q += (int64_t)gridDim.x * blockDim.x) {
@@ -374,7 +374,7 @@ k_basis_family(const float* __restrict__ t, int64_t n, int deg, int family, doub
 __global__ void __launch_bounds__(256)
 k_basis_family_bwd(const float* __restrict__ t, const float* __restrict__ g, int64_t n, int deg,
                    int family, double alpha, double beta, float* __restrict__ dt) {
-  __shared__ float ra[kValuMaxDegree + 1], rb[kValuMaxDegree + 1], rc[kValuMaxDegree + 1];
+  __shared__ float ra[kGeneralMaxDegree + 1], rb[kGeneralMaxDegree + 1], rc[kGeneralMaxDegree + 1];
   stage_family(ra, rb, rc, deg, family, alpha, beta);
   for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < n;
        q += (int64_t)gridDim.x * blockDim.x) {

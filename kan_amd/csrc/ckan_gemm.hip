@@ -2777,17 +2777,6 @@ k_dc_pipe(const typename Elem<BF>::type* __restrict__ dYc, const float* __restri
 // Host-side configuration and launchers
 // ---------------------------------------------------------------------------
 
-// Raises a kernel's dynamic-LDS limit before its first launch on each device
-// (the attribute is per device).  `done` holds one bit per device.
-static void ensure_lds_limit(const void* fn, int bytes, std::atomic<uint32_t>& done) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 32) dev = 0;
-  const uint32_t bit = 1u << dev;
-  if (done.load(std::memory_order_acquire) & bit) return;
-  (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  done.fetch_or(bit, std::memory_order_acq_rel);
-}
-
 // Number of workgroups that fills the chip once: 256 CUs, one 4-wave block each.
 static constexpr int kChipBlocks = 256;
 

@@ -1,0 +1,900 @@
+// The ChebyKAN layer for any degree, in fp32 or fp64, on the fp32 / fp64
+// matrix instructions (v_mfma_f32_16x16x4_f32, v_mfma_f64_16x16x4_f64):
+//   forward  y[b, o]     = sum_{i, d} P_d(t[b, i]) C[i, o, d],  t = tanh(x)
+//   dx       dx[b, i]    = t'(x) sum_d G[b, i, d] P_d'(t),
+//                          G[b, i, d] = sum_o dy[b, o] C[i, o, d]
+//   dC       dC[i, o, d] = sum_b P_d(t[b, i]) dy[b, o]
+// with P_d = T_d (the Chebyshev layers) or any basis of a three-term
+// recurrence P_d = (a_d u + b_d) P_{d-1} - c_d P_{d-2} at u = s t (the Jacobi
+// and Hermite layers, kan/basis/jacobi.py:131-188,
+// kan/basis/hermite.py:158-233), whose coefficients come from a recurrence
+// block (in fp32, the packed buffer's).  t = tanh(x), or the affine map a x + b
+// of a finite-domain Hermite layer (kan/basis/hermite.py:102-112).
+// It serves the fp64 layer (the reference computes in fp64 when its
+// parameter is fp64: kan/layers/chebykan.py:48-51 after .double()) and fp32
+// layers above the packed kernels' degree 16 (the reference layers take any
+// degree, kan/layers/chebykan.py:21-51).  C is read in its own [I, O, D]
+// layout; t is [B, I].
+//
+// How the contractions meet the 16x16x4 instruction.  Lane l holds row (or
+// column) l % 16 of an operand at reduction slot g = l / 16.  Which reduction
+// index a slot carries is free, so every basis value is made in the register
+// of the lane that feeds it, by that lane's own recurrence, one step per
+// matrix instruction:
+//   forward: slot g of one instruction is input i0 + g at one degree, so lane
+//     (row, g) walks the degrees of its (row, input) pair;
+//   dC: the operand rows are 16 inputs and slot g is batch row b0 + g, so lane
+//     (input, g) walks the degrees of its (input, row) pair, one accumulator
+//     per degree;
+//   dx: the result columns are 16 inputs with one accumulator per degree, so
+//     each lane holds every G[b, i, d] of its own (b, i) pairs and the degree
+//     sum needs no exchange.
+// The basis never passes through LDS or memory, and one or two recurrence
+// FMAs ride beside up to eight matrix instructions; what bounds the kernels is
+// the matrix pipe (64 clk per fp64 instruction, 32 per fp32) and, at small
+// sizes, how far the reduction can be split to fill it.  Against the
+// vector-ALU register tiles that these kernels replaced (which put 64-128
+// blocks on the chip at these sizes), forward / dx / dC:
+//   2048 x 256 -> 256, degree 8, fp64:  483 / 112 / 532 -> 70 / 58 / 51 us
+//   4096 x 256 -> 128, degree 24, fp32: 1013 / 191 / 1534 -> 106 / 82 / 85 us
+// (41 / 49 / 56 TFLOP/s of products in fp64; 63 / 82 / 79 in fp32).
+#include "ckan_kernels.hpp"
+
+#include <math.h>
+
+#include <atomic>
+#include <type_traits>
+
+namespace ckan {
+
+typedef __attribute__((ext_vector_type(4))) double f64x4_t;
+
+template <typename T> __device__ __forceinline__ T vtanh(T x);
+template <> __device__ __forceinline__ float vtanh<float>(float x) { return tanhf(x); }
+template <> __device__ __forceinline__ double vtanh<double>(double x) { return tanh(x); }
+
+// t = tanh(x), or ima x + imb with the affine map.
+template <typename T>
+__global__ void __launch_bounds__(256)
+k_tanh_v(const T* __restrict__ x, T* __restrict__ t, int64_t n, int imap, float ima, float imb) {
+  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < n;
+       q += (int64_t)gridDim.x * blockDim.x)
+    t[q] = imap ? fma((T)ima, x[q], (T)imb) : vtanh<T>(x[q]);
+}
+
+template <typename T>
+__device__ __forceinline__ T buffer_load(__amdgpu_buffer_rsrc_t rs, int voff, int soff) {
+  if constexpr (sizeof(T) == 8)
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(rs, voff, soff, 0));
+  else
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(rs, voff, soff, 0));
+}
+
+// The 16x16x4 matrix instruction of each type, and the result row of
+// accumulator value v in lane group g (the column is lane % 16).
+template <typename T> struct Mx;
+template <> struct Mx<float> {
+  typedef f32x4_t acc_t;
+  static __device__ __forceinline__ acc_t mma(float a, float b, acc_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int v, int g) { return 4 * g + v; }
+};
+template <> struct Mx<double> {
+  typedef f64x4_t acc_t;
+  static __device__ __forceinline__ acc_t mma(double a, double b, acc_t c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int v, int g) { return 4 * v + g; }
+};
+
+// One basis recurrence.  Chebyshev (GEN = false): T_{d+1} = 2t T_d - T_{d-1},
+// w = 2t, started from T_{-1} = t so that the first step gives 2t - t = t =
+// T_1 exactly and every step is the same FMA.  GEN: P_{d+1} = (a_{d+1} w +
+// b_{d+1}) P_d - c_{d+1} P_{d-1}, w = u = s t, started from P_{-1} = 0 (c_1 =
+// 0); rs holds a[D], b[D], c[D], s.  A cleared recurrence stays zero.
+template <typename T, bool GEN> struct Rec {
+  T w, pm, pc;
+  __device__ __forceinline__ void init(T t, const T* rs, int D) {
+    if constexpr (GEN) {
+      w = rs[3 * D] * t;
+      pm = T(0);
+    } else {
+      w = t + t;
+      pm = t;
+    }
+    pc = T(1);
+  }
+  __device__ __forceinline__ void clear() { w = pm = pc = T(0); }
+  // To degree n (n past the layer's last degree reads in-range coefficients
+  // whose result no caller uses).
+  __device__ __forceinline__ void step(const T* rs, int D, int n) {
+    T nx;
+    if constexpr (GEN) {
+      const int k = n < D ? n : D - 1;
+      nx = fma(fma(rs[k], w, rs[D + k]), pc, -rs[2 * D + k] * pm);
+    } else {
+      nx = fma(w, pc, -pm);
+    }
+    pm = pc;
+    pc = nx;
+  }
+  // To degree n + 1 from n - 1, in place (a rolled loop of single steps would
+  // move registers as often as it computes).
+  __device__ __forceinline__ void step2(const T* rs, int D, int n) {
+    if constexpr (GEN) {
+      pm = fma(fma(rs[n], w, rs[D + n]), pc, -rs[2 * D + n] * pm);
+      pc = fma(fma(rs[n + 1], w, rs[D + n + 1]), pm, -rs[2 * D + n + 1] * pc);
+    } else {
+      pm = fma(w, pc, -pm);
+      pc = fma(w, pm, -pc);
+    }
+  }
+};
+
+// The recurrence block in LDS (families only); the kind flag (0: Chebyshev)
+// is uniform over a launch and selects the kernel body.
+template <typename T>
+__device__ __forceinline__ bool stage_rec(T* rs, const T* __restrict__ rec, int D) {
+  if (rec == nullptr || rec[3 * D + 1] == T(0)) return false;
+  for (int k = threadIdx.x; k < 3 * D + 2; k += blockDim.x) rs[k] = rec[k];
+  return true;
+}
+// LDS elements reserved for it (16-byte multiple).
+static int rec_lds_elems(bool has_rec, int D) { return has_rec ? (3 * D + 2 + 3) / 4 * 4 : 0; }
+
+// Blocks are 8 waves.  kWaves = WM * WK: WM waves share a C tile along the
+// rows, WK groups split the reduction and are summed in a fixed order.
+constexpr int kWaves = 8;
+
+// Block -> tile with consecutive tiles on one XCD (workgroups go round-robin
+// over the 8 XCDs), so that tiles sharing operands meet in one L2.
+__device__ __forceinline__ unsigned xcd_tile(unsigned id, unsigned n) {
+  const unsigned per = n / 8, rem = n % 8, x = id % 8, k = id / 8;
+  return x * per + (x < rem ? x : rem) + k;
+}
+
+// 16 bytes of consecutive elements at the elements' own alignment (C's runs
+// start anywhere; the memory system takes unaligned 16-byte loads).
+template <typename T> struct Run {
+  static constexpr int V = 16 / (int)sizeof(T);
+  typedef T vec __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
+};
+// n (uniform, at most MAX) consecutive elements of C from src into dst, 16
+// bytes at a time where that stays inside C (it ends at cend), else one by
+// one.  Whole vectors: elements past n hold what follows in C.  !ok: zeros.
+template <typename T, int MAX>
+__device__ __forceinline__ void load_run(const T* src, const T* cend, int n, bool ok, T* dst) {
+  constexpr int V = Run<T>::V, NV = (MAX + V - 1) / V;
+  if (src + (n + V - 1) / V * V <= cend) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      if (v * V < n) {
+        const typename Run<T>::vec x = *reinterpret_cast<const typename Run<T>::vec*>(src + v * V);
+#pragma unroll
+        for (int e = 0; e < V; ++e)
+          if (v * V + e < MAX) dst[v * V + e] = x[e];
+      }
+    }
+  } else {
+#pragma unroll
+    for (int d = 0; d < MAX; ++d) dst[d] = src[d < n ? d : n - 1];
+  }
+  if (!ok) {
+#pragma unroll
+    for (int d = 0; d < MAX; ++d) dst[d] = T(0);
+  }
+}
+
+// ---- forward ------------------------------------------------------------------
+// Wave tile 16 NM rows x 16 NN outputs.  A step is 4 inputs x one chunk of at
+// most kFwdDC degrees: its C tile goes through registers into one of two LDS
+// buffers while the other one's step runs.  LDS image: element (ii, o, d) at
+// ii * S + o * DP + d with DP odd and S = 16 DP (mod 64), so that the 64 lanes
+// of a read (16 outputs x 4 inputs at one degree) take distinct banks.
+template <typename T> constexpr int kFwdDC = sizeof(T) == 8 ? 9 : 17;
+struct GenFwd {
+  int wk;              // reduction groups
+  int dc, nch;         // degrees per chunk, chunks
+  int dp, s;           // LDS strides (elements)
+  int rec_elems;
+  int mblocks, nblocks;
+};
+template <int NN> __host__ __device__ constexpr int fwd_stride(int dp) {
+  return 16 * NN * dp + (16 * dp * (NN == 4 ? 1 : NN == 2 ? 3 : 0)) % 64;
+}
+
+template <typename T, int NM, int NN, bool GEN>
+__device__ __forceinline__ void gen_fwd_body(const T* __restrict__ t, const T* __restrict__ C,
+                                             T* __restrict__ y, int64_t B, int I, int O, int D,
+                                             const GenFwd f, T* lds, const T* rs) {
+  typedef typename Mx<T>::acc_t acc_t;
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, l15 = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int WM = kWaves / f.wk, wm = wave % WM, wk = wave / WM;
+  const unsigned tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int64_t b0 = ((int64_t)(tile % f.mblocks) * WM + wm) * (16 * NM);
+  const int o0 = (int)(tile / f.mblocks) * (16 * NN);
+  const int stage = 4 * f.s;
+  T* buf = lds + f.rec_elems + wk * stage;
+  const int half = f.wk * stage;  // elements from buffer 0 to buffer 1
+
+  acc_t acc[NM][NN];
+#pragma unroll
+  for (int m = 0; m < NM; ++m)
+#pragma unroll
+    for (int n = 0; n < NN; ++n) acc[m][n] = acc_t{0, 0, 0, 0};
+
+  // this lane's rows, clamped (results of rows past B are not stored)
+  const T* trow[NM];
+#pragma unroll
+  for (int m = 0; m < NM; ++m) {
+    const int64_t b = b0 + 16 * m + l15;
+    trow[m] = t + (b < B ? b : 0) * I;
+  }
+
+  // C's tile is 64 NN runs of dn degrees, (input q / 16 NN, output q % 16 NN);
+  // thread q of the group's first NN waves stages run q (two runs where a
+  // group has NN / 2 waves)
+  constexpr int kRuns = NN > 1 ? 2 : 1;
+  T pre[kRuns][kFwdDC<T>], tn[NM];
+  const T* cend = C + (size_t)I * O * D;
+  auto load_tile = [&](int i0, int d0, int dn) {
+#pragma unroll
+    for (int r = 0; r < kRuns; ++r) {
+      if (r * WM + wm < NN) {
+        const int q = (r * WM + wm) * 64 + lane, i = i0 + q / (16 * NN), o = o0 + q % (16 * NN);
+        const bool ok = i < I && o < O;
+        load_run<T, kFwdDC<T>>(ok ? C + ((size_t)i * O + o) * D + d0 : C, cend, dn, ok, pre[r]);
+      }
+    }
+  };
+  auto store_tile = [&](T* dst, int dn) {
+#pragma unroll
+    for (int r = 0; r < kRuns; ++r) {
+      if (r * WM + wm < NN) {
+        const int q = (r * WM + wm) * 64 + lane;
+        T* run = dst + (q / (16 * NN)) * f.s + (q % (16 * NN)) * f.dp;
+#pragma unroll
+        for (int d = 0; d < kFwdDC<T>; ++d)
+          if (d < dn) run[d] = pre[r][d];
+      }
+    }
+  };
+  auto load_t = [&](int i0) {
+    const int i = i0 + g < I ? i0 + g : 0;
+#pragma unroll
+    for (int m = 0; m < NM; ++m) tn[m] = trow[m][i];
+  };
+
+  const int groups = (I + 3) / 4, iters = (groups + f.wk - 1) / f.wk;
+  Rec<T, GEN> r[NM];
+  load_tile(4 * wk, 0, min(f.dc, D));
+  load_t(4 * wk);
+  store_tile(buf, min(f.dc, D));
+  __syncthreads();
+  int cur = 0;
+  for (int it = 0; it < iters; ++it) {
+    const int i0 = 4 * (it * f.wk + wk);
+#pragma unroll
+    for (int m = 0; m < NM; ++m) r[m].init(tn[m], rs, D);
+    if (i0 + 4 > I) {  // inputs past I meet zero coefficients: keep their basis finite
+#pragma unroll
+      for (int m = 0; m < NM; ++m)
+        if (i0 + g >= I) r[m].clear();
+    }
+    for (int c = 0; c < f.nch; ++c) {
+      const int d0 = c * f.dc, dn = min(f.dc, D - d0);
+      const bool last_c = c + 1 == f.nch, more = !(last_c && it + 1 == iters);
+      const int nd0 = last_c ? 0 : d0 + f.dc, ndn = min(f.dc, D - nd0);
+      const int ni0 = last_c ? i0 + 4 * f.wk : i0;
+      if (more) {
+        load_tile(ni0, nd0, ndn);
+        if (last_c) load_t(ni0);
+      }
+      const T* bp = buf + cur * half + g * f.s + l15 * f.dp;
+      T bv[NN];
+#pragma unroll
+      for (int n = 0; n < NN; ++n) bv[n] = bp[n * 16 * f.dp];
+#pragma unroll 2
+      for (int d = 0; d < dn; ++d) {
+        T bn[NN];  // the next degree's (the last one's read stays inside the LDS tile and is dropped)
+#pragma unroll
+        for (int n = 0; n < NN; ++n) bn[n] = bp[n * 16 * f.dp + (d + 1 < dn ? d + 1 : d)];
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+          for (int n = 0; n < NN; ++n) acc[m][n] = Mx<T>::mma(r[m].pc, bv[n], acc[m][n]);
+#pragma unroll
+        for (int m = 0; m < NM; ++m) r[m].step(rs, D, d0 + d + 1);
+#pragma unroll
+        for (int n = 0; n < NN; ++n) bv[n] = bn[n];
+      }
+      if (more) store_tile(buf + (cur ^ 1) * half, ndn);
+      cur ^= 1;
+      __syncthreads();
+    }
+  }
+  // sum the reduction groups in order through LDS (the tile buffers are done)
+  T* red = lds + f.rec_elems + (size_t)wm * (64 * NM * NN * 4) + lane;
+  for (int k = 1; k < f.wk; ++k) {
+    if (wk == k) {
+#pragma unroll
+      for (int q = 0; q < NM * NN * 4; ++q) red[q * 64] = acc[q / 4 / NN][q / 4 % NN][q % 4];
+    }
+    __syncthreads();
+    if (wk == 0) {
+#pragma unroll
+      for (int q = 0; q < NM * NN * 4; ++q) acc[q / 4 / NN][q / 4 % NN][q % 4] += red[q * 64];
+    }
+    __syncthreads();
+  }
+  if (wk != 0) return;
+#pragma unroll
+  for (int m = 0; m < NM; ++m)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int64_t b = b0 + 16 * m + Mx<T>::row(v, g);
+      if (b >= B) continue;
+#pragma unroll
+      for (int n = 0; n < NN; ++n) {
+        const int o = o0 + 16 * n + l15;
+        if (o < O) y[b * O + o] = acc[m][n][v];
+      }
+    }
+}
+
+template <typename T> __device__ __forceinline__ T* dyn_lds() {
+  extern __shared__ __align__(16) char gen_lds[];
+  return reinterpret_cast<T*>(gen_lds);
+}
+
+template <typename T, int NM, int NN>
+__global__ void __launch_bounds__(512)
+k_gen_fwd(const T* __restrict__ t, const T* __restrict__ C, T* __restrict__ y, int64_t B, int I,
+          int O, int D, GenFwd f, const T* __restrict__ rec) {
+  T* lds = dyn_lds<T>();
+  const bool gen = stage_rec<T>(lds, rec, D);
+  __syncthreads();
+  if (gen) gen_fwd_body<T, NM, NN, true>(t, C, y, B, I, O, D, f, lds, lds);
+  else gen_fwd_body<T, NM, NN, false>(t, C, y, B, I, O, D, f, lds, lds);
+}
+
+// ---- dx -------------------------------------------------------------------------
+// Wave tile 16 rows x 16 inputs, DM degrees at a time with one accumulator per
+// degree; a chunk's G is folded into dx by the lane that holds it before the
+// next chunk starts.  A step is 16 outputs: lane group g takes outputs 4 g ..
+// 4 g + 3 of it, so a lane reads 4 consecutive dy values.  C's tile [16
+// inputs][16 outputs][DM] goes through registers into one of two LDS buffers,
+// one (input, output) run of degrees per thread; element (i, o = 4 g + s, d)
+// at i * S + g * Q + s * DM + d with S odd and Q = 16 S (mod 64): the 64 lanes
+// of a read take distinct banks.  A second row fragment per wave would halve
+// the LDS reads, which are far from the bound (4 per SIMD round of one matrix
+// instruction each), and spills.
+template <int DM> struct GenDxLds {
+  static constexpr int Q = (4 * DM + 15) / 32 * 32 + 16;      // 16 (mod 32), >= 4 DM
+  static constexpr int S = 4 * Q + (Q % 64 == 16 ? 1 : 3);    // odd, 16 S = Q (mod 64)
+  static_assert(Q >= 4 * DM && Q % 32 == 16 && (16 * S - Q) % 64 == 0, "LDS strides");
+  static constexpr int kStage = 16 * S;
+};
+struct GenDx {
+  int wk, nch, rec_elems, mblocks;
+  int imap;
+  float ima;
+};
+
+template <typename T, int DM, bool GEN>
+__device__ __forceinline__ void gen_dx_body(const T* __restrict__ t, const T* __restrict__ C,
+                                            const T* __restrict__ dy, T* __restrict__ dx, int64_t B,
+                                            int I, int O, int D, const GenDx f, T* lds,
+                                            const T* rs) {
+  typedef typename Mx<T>::acc_t acc_t;
+  typedef GenDxLds<DM> L;
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, l15 = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int WM = kWaves / f.wk, wm = wave % WM, wk = wave / WM;
+  const unsigned tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int64_t b0 = ((int64_t)(tile % f.mblocks) * WM + wm) * 16;
+  const int i0 = (int)(tile / f.mblocks) * 16;
+  T* buf = lds + f.rec_elems + wk * L::kStage;
+  const int half = f.wk * L::kStage;
+
+  const T* yrow = dy + (b0 + l15 < B ? b0 + l15 : 0) * O + 4 * g;  // rows past B are not stored
+  // waves 0-3 of a group stage its C tile: thread q the run of degrees of
+  // (input q / 16, output q % 16)
+  const bool stager = wm < 4;
+  const int q = (wm & 3) * 64 + lane;
+  const bool iok = i0 + (q >> 4) < I;
+  const T* crun = C + (size_t)(iok ? i0 + (q >> 4) : 0) * O * D;
+  const T* cend = C + (size_t)I * O * D;
+  T* cdst = buf + (q >> 4) * L::S + ((q >> 2) & 3) * L::Q + (q & 3) * DM;
+
+  T s[4];  // this lane's (b, i) pairs: rows b0 + row(v, g), input i0 + l15
+#pragma unroll
+  for (int v = 0; v < 4; ++v) s[v] = T(0);
+
+  T pre[DM], an[4];
+  auto load_step = [&](int ob, int d0, int dn) {
+    if (stager) {
+      const int o = ob + (q & 15);
+      const bool ok = iok && o < O;
+      load_run<T, DM>(ok ? crun + (size_t)o * D + d0 : C, cend, dn, ok, pre);
+    }
+    if (ob + 16 <= O) {
+      constexpr int V = Run<T>::V;
+#pragma unroll
+      for (int v = 0; v < 4 / V; ++v) {
+        const typename Run<T>::vec x = *reinterpret_cast<const typename Run<T>::vec*>(yrow + ob + v * V);
+#pragma unroll
+        for (int e = 0; e < V; ++e) an[v * V + e] = x[e];
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) an[k] = ob + 4 * g + k < O ? yrow[ob + k] : T(0);
+    }
+  };
+  auto store_step = [&](int b) {
+    if (stager) {
+#pragma unroll
+      for (int k = 0; k < DM; ++k) cdst[b * half + k] = pre[k];
+    }
+  };
+
+  const int osteps = (O + 15) / 16, iters = (osteps + f.wk - 1) / f.wk;
+  load_step(16 * wk, 0, min(DM, D));
+  store_step(0);
+  __syncthreads();
+  int cur = 0;
+  for (int c = 0; c < f.nch; ++c) {
+    const int d0 = c * DM, dn = min(DM, D - d0);
+    acc_t acc[DM];
+#pragma unroll
+    for (int d = 0; d < DM; ++d) acc[d] = acc_t{0, 0, 0, 0};
+    for (int it = 0; it < iters; ++it) {
+      T a[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) a[k] = an[k];
+      const bool last = it + 1 == iters, more = !(last && c + 1 == f.nch);
+      if (more) {
+        const int nd0 = last ? d0 + DM : d0;
+        load_step(16 * (last ? wk : (it + 1) * f.wk + wk), nd0, min(DM, D - nd0));
+      }
+      const T* bp = buf + cur * half + l15 * L::S + g * L::Q;
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int d = 0; d < DM; ++d) acc[d] = Mx<T>::mma(a[k], bp[k * DM + d], acc[d]);
+      if (more) store_step(cur ^ 1);
+      cur ^= 1;
+      __syncthreads();
+    }
+    // s += sum_d G_d P_d'(t) over the chunk (this reduction group's share of G)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int64_t b = b0 + Mx<T>::row(v, g);
+      const T tv = b < B && i0 + l15 < I ? t[b * I + i0 + l15] : T(0);
+      T sum = T(0);
+      if constexpr (GEN) {
+        // (pm, pc) = (P_{n-1}, P_n), (qm, qc) their derivatives in u, from n = 0:
+        // P_n' = a_n P_{n-1} + (a_n u + b_n) P_{n-1}' - c_n P_{n-2}'
+        const T u = rs[3 * D] * tv;
+        T pm = T(0), pc = T(1), qm = T(0), qc = T(0);
+        auto step = [&](int n) {
+          asm volatile("" ::: "memory");  // coefficients read per step, not hoisted
+          const int k = n < D ? n : D - 1;
+          const T a_n = rs[k], fn = fma(a_n, u, rs[D + k]), cn = rs[2 * D + k];
+          const T pn = fma(fn, pc, -cn * pm);
+          const T qn = fma(a_n, pc, fma(fn, qc, -cn * qm));
+          pm = pc;
+          pc = pn;
+          qm = qc;
+          qc = qn;
+        };
+        for (int n = 1; n <= d0; ++n) step(n);
+#pragma unroll
+        for (int d = 0; d < DM; ++d) {
+          if (d < dn) {
+            sum = fma(acc[d][v], qc, sum);
+            step(d0 + d + 1);
+          }
+        }
+      } else {
+        // dT_n/dt = n U_{n-1}: (up, u) = (U_{n-2}, U_{n-1}) at degree n, from
+        // (U_{-1}, U_0) at n = 1; degree 0 has no derivative
+        const T t2 = tv + tv;
+        T up = T(0), u = T(1);
+        for (int n = 1; n < d0; ++n) {
+          const T un = fma(t2, u, -up);
+          up = u;
+          u = un;
+        }
+        T deg = (T)d0;  // counted in T (exact)
+#pragma unroll
+        for (int d = 0; d < DM; ++d) {
+          if (d < dn && (d > 0 || d0 > 0)) {
+            sum = fma(acc[d][v] * deg, u, sum);
+            const T un = fma(t2, u, -up);
+            up = u;
+            u = un;
+          }
+          deg += T(1);
+        }
+      }
+      s[v] += sum;
+    }
+  }
+  // sum the reduction groups in order, apply t'(x), store
+  T* red = lds + f.rec_elems + wm * 256 + lane;
+  for (int k = 1; k < f.wk; ++k) {
+    if (wk == k) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) red[v * 64] = s[v];
+    }
+    __syncthreads();
+    if (wk == 0) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) s[v] += red[v * 64];
+    }
+    __syncthreads();
+  }
+  if (wk != 0 || i0 + l15 >= I) return;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const int64_t b = b0 + Mx<T>::row(v, g);
+    if (b >= B) continue;
+    const T tv = t[b * I + i0 + l15];
+    const T slope = f.imap ? (T)f.ima : T(1) - tv * tv;
+    dx[b * I + i0 + l15] = (GEN ? s[v] * rs[3 * D] : s[v]) * slope;  // du/dt = rs[3 D] for a family
+  }
+}
+
+template <typename T, int DM>
+__global__ void __launch_bounds__(512)
+k_gen_dx(const T* __restrict__ t, const T* __restrict__ C, const T* __restrict__ dy,
+         T* __restrict__ dx, int64_t B, int I, int O, int D, GenDx f, const T* __restrict__ rec) {
+  T* lds = dyn_lds<T>();
+  const bool gen = stage_rec<T>(lds, rec, D);
+  __syncthreads();
+  if (gen) gen_dx_body<T, DM, true>(t, C, dy, dx, B, I, O, D, f, lds, lds);
+  else gen_dx_body<T, DM, false>(t, C, dy, dx, B, I, O, D, f, lds, lds);
+}
+
+// ---- dC ---------------------------------------------------------------------------
+template <typename T> struct DcWrite;
+template <> struct DcWrite<float> {  // the dC write modes of the MFMA kernels
+  static __device__ __forceinline__ void put(float* d, float v, const DcOut& om) { dc_write(d, v, om); }
+};
+template <> struct DcWrite<double> {  // store or accumulate
+  static __device__ __forceinline__ void put(double* d, double v, const DcOut& om) {
+    *d = om.mode == kDcAccumulate ? *d + v : v;
+  }
+};
+
+// Wave tile 16 inputs x 16 NN outputs x DM degrees (one chunk of the degree
+// axis), the reduction over the batch rows split between the WK waves of a
+// block that share the tile.  Both operands come straight from memory: 16
+// lanes read 16 consecutive t (or dy) values of a row, and the waves of a
+// block reuse each other's lines in L1.  The next unit of rows is loaded while
+// one is used.  The WK partial sums meet in LDS by halves (a fixed order).
+struct GenDc {
+  int wk, nch, rec_elems;
+  int iblocks, otiles;   // 16-input blocks, output tiles of 16 NN
+  int64_t units;         // row units per reduction group
+};
+// Rows a wave loads ahead, 4 per matrix instruction: as many as the registers
+// beside the accumulators hold (twice as many on the narrow tiles measured
+// the same).
+template <typename T> constexpr int kDcUnit = sizeof(T) == 8 ? 8 : 16;
+
+template <typename T, int DM, int NN, bool GEN>
+__device__ __forceinline__ void gen_dc_body(const T* __restrict__ t, const T* __restrict__ dy,
+                                            T* __restrict__ dC, int64_t B, int I, int O, int D,
+                                            const GenDc f, const DcOut& om, T* lds, const T* rs) {
+  typedef typename Mx<T>::acc_t acc_t;
+  constexpr int kU = kDcUnit<T>, KU = kU / 4;
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, l15 = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int WT = kWaves / f.wk, wt = wave % WT, wk = wave / WT;
+  // tiles: output tile fastest, then input block, then chunk
+  const unsigned ntiles = (unsigned)f.otiles * f.iblocks * f.nch;
+  const unsigned tile = xcd_tile(blockIdx.x, gridDim.x) * WT + wt;
+  const bool live = tile < ntiles;  // a block's last waves may have no tile
+  const unsigned tl = live ? tile : 0;
+  const int o0 = (int)(tl % f.otiles) * (16 * NN);
+  const int i0 = (int)(tl / f.otiles % f.iblocks) * 16;
+  const int d0 = (int)(tl / f.otiles / f.iblocks) * DM;
+  const int i = i0 + l15;
+  const bool iok = i < I;
+
+  acc_t acc[DM][NN];
+#pragma unroll
+  for (int d = 0; d < DM; ++d)
+#pragma unroll
+    for (int n = 0; n < NN; ++n) acc[d][n] = acc_t{0, 0, 0, 0};
+
+  const int64_t ub = (int64_t)wk * f.units, ue0 = ub + f.units, nu = (B + kU - 1) / kU;
+  const int64_t ue = live ? (ue0 < nu ? ue0 : nu) : 0;
+  // Loads go through a buffer descriptor of the unit's rows, rebuilt in
+  // scalar registers each unit: a lane's byte offset is fixed for the kernel,
+  // the row offset is scalar, and rows past B read as zeros (dy = 0 drops
+  // them).  Inputs and outputs past the layer's read column 0; their results
+  // are not stored.
+  const int esz = (int)sizeof(T);
+  const int toff = (g * I + (iok ? i : 0)) * esz;
+  int yoff[NN];
+#pragma unroll
+  for (int n = 0; n < NN; ++n) yoff[n] = (g * O + (o0 + 16 * n + l15 < O ? o0 + 16 * n + l15 : 0)) * esz;
+  T tn[KU], yn[KU][NN];
+  auto load = [&](int64_t u) {
+    const int64_t left = B - u * kU;
+    const int rows = (int)(left < kU ? left : kU);
+    const __amdgpu_buffer_rsrc_t rt = buffer_rsrc(t + u * kU * I, rows * I * esz);
+    const __amdgpu_buffer_rsrc_t ry = buffer_rsrc(dy + u * kU * O, rows * O * esz);
+#pragma unroll
+    for (int k = 0; k < KU; ++k) {
+      tn[k] = buffer_load<T>(rt, toff, 4 * k * I * esz);
+#pragma unroll
+      for (int n = 0; n < NN; ++n) yn[k][n] = buffer_load<T>(ry, yoff[n], 4 * k * O * esz);
+    }
+  };
+  if (ub < ue) load(ub);
+  for (int64_t u = ub; u < ue; ++u) {
+    Rec<T, GEN> r[KU];
+    T yc[KU][NN];
+#pragma unroll
+    for (int k = 0; k < KU; ++k) {
+      r[k].init(tn[k], rs, D);
+#pragma unroll
+      for (int n = 0; n < NN; ++n) yc[k][n] = yn[k][n];
+    }
+    if ((u + 1) * kU > B) {  // a basis value of a row past B may not be finite
+#pragma unroll
+      for (int k = 0; k < KU; ++k)
+        if (u * kU + 4 * k + g >= B) r[k].clear();
+    }
+    load(u + 1 < ue ? u + 1 : u);
+    // to the chunk's first degree, the rows side by side
+    if (d0 & 1) {
+#pragma unroll
+      for (int k = 0; k < KU; ++k) r[k].step(rs, D, 1);
+    }
+    for (int n = 1 + (d0 & 1); n <= d0; n += 2) {
+#pragma unroll
+      for (int k = 0; k < KU; ++k) r[k].step2(rs, D, n);
+    }
+#pragma unroll
+    for (int k = 0; k < KU; ++k) {
+#pragma unroll
+      for (int d = 0; d < DM; ++d) {
+#pragma unroll
+        for (int n = 0; n < NN; ++n) acc[d][n] = Mx<T>::mma(r[k].pc, yc[k][n], acc[d][n]);
+        if (d + 1 < DM) r[k].step(rs, D, d0 + d + 1);
+      }
+    }
+  }
+  constexpr int kAcc = DM * NN * 4;
+  for (int h = f.wk / 2; h >= 1; h /= 2) {
+    T* red = lds + f.rec_elems + (size_t)((wk % h) * WT + wt) * (64 * kAcc) + lane;
+    if (wk >= h && wk < 2 * h) {
+#pragma unroll
+      for (int q = 0; q < kAcc; ++q) red[q * 64] = acc[q / 4 / NN][q / 4 % NN][q % 4];
+    }
+    __syncthreads();
+    if (wk < h) {
+#pragma unroll
+      for (int q = 0; q < kAcc; ++q) acc[q / 4 / NN][q / 4 % NN][q % 4] += red[q * 64];
+    }
+    __syncthreads();
+  }
+  if (wk != 0 || !live) return;
+#pragma unroll
+  for (int n = 0; n < NN; ++n)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int io = i0 + Mx<T>::row(v, g), o = o0 + 16 * n + l15;
+      if (io >= I || o >= O) continue;
+      T* dst = dC + ((size_t)io * O + o) * D + d0;
+#pragma unroll
+      for (int d = 0; d < DM; ++d)
+        if (d0 + d < D) DcWrite<T>::put(dst + d, acc[d][n][v], om);
+    }
+}
+
+template <typename T, int DM, int NN>
+__global__ void __launch_bounds__(512)
+k_gen_dc(const T* __restrict__ t, const T* __restrict__ dy, T* __restrict__ dC, int64_t B, int I,
+         int O, int D, GenDc f, DcOut om, const T* __restrict__ rec) {
+  T* lds = dyn_lds<T>();
+  const bool gen = stage_rec<T>(lds, rec, D);
+  __syncthreads();
+  if (gen) gen_dc_body<T, DM, NN, true>(t, dy, dC, B, I, O, D, f, om, lds, lds);
+  else gen_dc_body<T, DM, NN, false>(t, dy, dC, B, I, O, D, f, om, lds, lds);
+}
+
+// dst = float(src) (or dst += float(src)), src fp32 or bf16: the coefficient
+// copy of this path.
+__global__ void __launch_bounds__(256)
+k_to_f32(const void* __restrict__ src, int src_bf16, float* __restrict__ dst, int64_t n,
+         int accumulate) {
+  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < n;
+       q += (int64_t)gridDim.x * blockDim.x) {
+    const float v = src_bf16 ? __uint_as_float((uint32_t)static_cast<const uint16_t*>(src)[q] << 16)
+                             : static_cast<const float*>(src)[q];
+    dst[q] = accumulate ? dst[q] + v : v;
+  }
+}
+
+static unsigned vgrid(int64_t n) {
+  int64_t g = (n + 255) / 256;
+  if (g > 65536) g = 65536;
+  return (unsigned)(g < 1 ? 1 : g);
+}
+
+void launch_to_f32(const void* src, bool src_bf16, float* dst, int64_t n, hipStream_t s,
+                   bool accumulate) {
+  if (n > 0)
+    hipLaunchKernelGGL(k_to_f32, dim3(vgrid(n)), dim3(256), 0, s, src, src_bf16 ? 1 : 0, dst, n,
+                       accumulate ? 1 : 0);
+}
+
+// ---- launch shapes ----------------------------------------------------------------
+// Waves that give every SIMD two: below it, tiles shrink and the reduction is
+// split until the launch has as many (or nothing is left to split).  Four per
+// SIMD measured slower: the smaller tiles stage more of C for each product
+// (2048 x 256 -> 256 in fp64: forward 73 -> 84 us, backward 103 -> 117; 4096 x
+// 256 -> 128, degree 24: forward 108 -> 134).
+constexpr int64_t kWantWaves = 2 * 4 * kNumCUs;
+constexpr int kMaxLds = 160 * 1024;
+
+// Degrees per chunk: the fewest chunks of at most `cap` degrees, evenly sized.
+static int even_chunk(int D, int cap) {
+  const int n = (D + cap - 1) / cap;
+  return (D + n - 1) / n;
+}
+
+template <typename T, int NM, int NN>
+static bool gen_fwd_launch(const T* t, const T* C, T* y, int64_t B, int I, int O, int D,
+                           const T* rec, hipStream_t s, bool must) {
+  static std::atomic<uint32_t> lds_done{0};
+  GenFwd f;
+  f.dc = even_chunk(D, kFwdDC<T>);
+  f.nch = (D + f.dc - 1) / f.dc;
+  f.dp = f.dc | 1;
+  f.s = fwd_stride<NN>(f.dp);
+  f.rec_elems = rec_lds_elems(rec != nullptr, D);
+  const int64_t mt = (B + 16 * NM - 1) / (16 * NM), nt = (O + 16 * NN - 1) / (16 * NN);
+  auto bytes = [&](int wk) {
+    const int64_t st = 2LL * wk * 4 * f.s, red = wk > 1 ? (int64_t)(kWaves / wk) * 64 * NM * NN * 4 : 0;
+    return (f.rec_elems + (st > red ? st : red)) * (int64_t)sizeof(T);
+  };
+  const int wk_max = NN == 4 ? 4 : 8;  // WM = 8 / wk >= NN / 2: a thread stages two runs at most
+  int wk = 1;
+  while (wk < wk_max && mt * nt * wk < kWantWaves && 2 * wk <= (I + 3) / 4 && bytes(2 * wk) <= kMaxLds) wk *= 2;
+  if (!must && mt * nt * wk < kWantWaves) return false;
+  f.wk = wk;
+  const int WM = kWaves / wk;
+  f.mblocks = (int)((mt + WM - 1) / WM);
+  f.nblocks = (int)nt;
+  ensure_lds_limit(reinterpret_cast<const void*>(&k_gen_fwd<T, NM, NN>), kMaxLds, lds_done);
+  hipLaunchKernelGGL((k_gen_fwd<T, NM, NN>), dim3((unsigned)f.mblocks * f.nblocks), dim3(512),
+                     (size_t)bytes(wk), s, t, C, y, B, I, O, D, f, rec);
+  return true;
+}
+
+template <typename T>
+void launch_forward_general(const T* x, const T* C, T* y, T* t, int64_t B, int I, int O, int deg,
+                            hipStream_t s, const T* rec, int imap, float ima, float imb) {
+  if (B == 0) return;
+  hipLaunchKernelGGL(k_tanh_v<T>, dim3(vgrid(B * I)), dim3(256), 0, s, x, t, B * I, imap, ima, imb);
+  const int D = deg + 1;
+  // the largest wave tile whose launch still fills the chip
+  if (gen_fwd_launch<T, 2, 4>(t, C, y, B, I, O, D, rec, s, false)) return;
+  if (gen_fwd_launch<T, 2, 2>(t, C, y, B, I, O, D, rec, s, false)) return;
+  gen_fwd_launch<T, 1, 1>(t, C, y, B, I, O, D, rec, s, true);
+}
+
+template <typename T, int DM>
+static void gen_dx(const T* t, const T* C, const T* dy, T* dx, int64_t B, int I, int O, int D,
+                   const T* rec, int imap, float ima, hipStream_t s) {
+  static std::atomic<uint32_t> lds_done{0};
+  GenDx f;
+  f.nch = (D + DM - 1) / DM;
+  f.rec_elems = rec_lds_elems(rec != nullptr, D);
+  f.imap = imap;
+  f.ima = ima;
+  const int64_t mt = (B + 15) / 16, it = (I + 15) / 16;
+  // two reduction groups at most: a group's 4 waves stage one run per thread
+  f.wk = mt * it < kWantWaves && O > 16 ? 2 : 1;
+  const int WM = kWaves / f.wk;
+  f.mblocks = (int)((mt + WM - 1) / WM);
+  const size_t bytes = (f.rec_elems + 2 * (size_t)f.wk * GenDxLds<DM>::kStage) * sizeof(T);
+  ensure_lds_limit(reinterpret_cast<const void*>(&k_gen_dx<T, DM>), kMaxLds, lds_done);
+  hipLaunchKernelGGL((k_gen_dx<T, DM>), dim3((unsigned)(f.mblocks * it)), dim3(512), bytes, s, t, C,
+                     dy, dx, B, I, O, D, f, rec);
+}
+
+template <typename T, int DM, int NN>
+static bool gen_dc_launch(const T* t, const T* dy, T* dC, DcOut om, int64_t B, int I, int O, int D,
+                          const T* rec, hipStream_t s, bool must) {
+  static std::atomic<uint32_t> lds_done{0};
+  GenDc f;
+  f.nch = (D + DM - 1) / DM;
+  f.rec_elems = rec_lds_elems(rec != nullptr, D);
+  f.iblocks = (I + 15) / 16;
+  f.otiles = (O + 16 * NN - 1) / (16 * NN);
+  const int64_t tiles = (int64_t)f.iblocks * f.otiles * f.nch;
+  const int64_t nu = (B + kDcUnit<T> - 1) / kDcUnit<T>;
+  auto bytes = [&](int wk) {
+    const int64_t red = wk > 1 ? 4LL * 64 * DM * NN * 4 : 0;
+    return (f.rec_elems + red) * (int64_t)sizeof(T);
+  };
+  int wk = 1;
+  while (wk < kWaves && tiles * wk < kWantWaves && 2 * wk <= nu && bytes(2 * wk) <= kMaxLds) wk *= 2;
+  if (!must && tiles * wk < kWantWaves) return false;
+  f.wk = wk;
+  f.units = (nu + wk - 1) / wk;
+  const int WT = kWaves / wk;
+  ensure_lds_limit(reinterpret_cast<const void*>(&k_gen_dc<T, DM, NN>), kMaxLds, lds_done);
+  hipLaunchKernelGGL((k_gen_dc<T, DM, NN>), dim3((unsigned)((tiles + WT - 1) / WT)), dim3(512),
+                     (size_t)bytes(wk), s, t, dy, dC, B, I, O, D, f, om, rec);
+  return true;
+}
+template <typename T, int DM>
+static void gen_dc(const T* t, const T* dy, T* dC, DcOut om, int64_t B, int I, int O, int D,
+                   const T* rec, hipStream_t s) {
+  // accumulators: DM x NN x 4 values a lane, at most 144 registers
+  constexpr int kBig = DM * 4 * 4 * (int)sizeof(T) / 4 <= 150 ? 4 : 2;
+  if (gen_dc_launch<T, DM, kBig>(t, dy, dC, om, B, I, O, D, rec, s, false)) return;
+  gen_dc_launch<T, DM, 1>(t, dy, dC, om, B, I, O, D, rec, s, true);
+}
+
+// Calls f with the degrees per chunk of a layer of D degrees as a constant:
+// the fewest chunks that the accumulators allow (9 degrees in fp64, 17 in
+// fp32), evenly sized, so that few of a chunk's degrees are padding.
+template <typename F> static void with_chunk_f64(int D, F f) {
+  switch (even_chunk(D, 9)) {
+    case 1: case 2: case 3: f(std::integral_constant<int, 3>()); break;
+    case 4: case 5: f(std::integral_constant<int, 5>()); break;
+    case 6: f(std::integral_constant<int, 6>()); break;
+    case 7: f(std::integral_constant<int, 7>()); break;
+    case 8: f(std::integral_constant<int, 8>()); break;
+    default: f(std::integral_constant<int, 9>()); break;
+  }
+}
+template <typename F> static void with_chunk_f32(int D, F f) {  // D >= 18
+  const int c = even_chunk(D, 17);
+  if (c <= 9) f(std::integral_constant<int, 9>());
+  else if (c <= 11) f(std::integral_constant<int, 11>());
+  else if (c <= 13) f(std::integral_constant<int, 13>());
+  else if (c <= 15) f(std::integral_constant<int, 15>());
+  else f(std::integral_constant<int, 17>());
+}
+
+template <typename T>
+void launch_backward_general(const T* t, const T* C, const T* dy, T* dx, T* dC, DcOut om, int64_t B,
+                             int I, int O, int deg, hipStream_t s, const T* rec, int imap,
+                             float ima) {
+  const int D = deg + 1;
+  auto go = [&](auto dm) {
+    constexpr int DM = decltype(dm)::value;
+    if (dx && B > 0) gen_dx<T, DM>(t, C, dy, dx, B, I, O, D, rec, imap, ima, s);
+    if (dC) gen_dc<T, DM>(t, dy, dC, om, B, I, O, D, rec, s);
+  };
+  if constexpr (sizeof(T) == 8) with_chunk_f64(D, go);
+  else with_chunk_f32(D, go);
+}
+
+template void launch_forward_general<float>(const float*, const float*, float*, float*, int64_t, int,
+                                         int, int, hipStream_t, const float*, int, float, float);
+template void launch_forward_general<double>(const double*, const double*, double*, double*, int64_t,
+                                          int, int, int, hipStream_t, const double*, int, float,
+                                          float);
+template void launch_backward_general<float>(const float*, const float*, const float*, float*, float*,
+                                          DcOut, int64_t, int, int, int, hipStream_t, const float*,
+                                          int, float);
+template void launch_backward_general<double>(const double*, const double*, const double*, double*,
+                                           double*, DcOut, int64_t, int, int, int, hipStream_t,
+                                           const double*, int, float);
+
+}  // namespace ckan
+

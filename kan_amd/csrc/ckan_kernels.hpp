@@ -2,6 +2,8 @@
 // byte layout of the packed-coefficient buffer and the workspaces.
 #pragma once
 
+#include <atomic>
+
 #include "ckan_common.hpp"
 
 namespace ckan {
@@ -9,6 +11,17 @@ namespace ckan {
 inline size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 // 16-byte aligned: the float4 load paths of x, dy and C require it.
 inline bool is_al16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
+
+// Raises a kernel's dynamic-LDS limit before its first launch on each device
+// (the attribute is per device).  `done` holds one bit per device.
+inline void ensure_lds_limit(const void* fn, int bytes, std::atomic<uint32_t>& done) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 32) dev = 0;
+  const uint32_t bit = 1u << dev;
+  if (done.load(std::memory_order_acquire) & bit) return;
+  (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  done.fetch_or(bit, std::memory_order_acq_rel);
+}
 
 // Sets the thread-local message returned by ckan_last_error().
 void set_last_error(const char* msg);
@@ -94,7 +107,7 @@ void family_to_chebyshev(const double* a, const double* b, const double* c, int 
 // om.base == dc); dcheb may be dc.
 void launch_coeff_from_cheb(const float* dcheb, float* dc, const Plan& p, const DcOut& om,
                             const BasisXform& xf, hipStream_t s);
-// out[q, n] = P_n(t[q]) (n <= deg <= kValuMaxDegree) and its backward; the
+// out[q, n] = P_n(t[q]) (n <= deg <= kGeneralMaxDegree) and its backward; the
 // recurrence coefficients are formed on the device (recur_coef).
 void launch_basis_family(const float* t, int64_t n, int deg, int family, double alpha,
                          double beta, float* out, hipStream_t s);
@@ -129,24 +142,24 @@ void launch_cheb_deriv_rows(const float* in, float* out, int64_t rows, int degre
 void launch_jacobian(const float* x, const float* c1t, float* jac, int64_t B, int I, int O,
                      int dout, int imap, float ima, float imb, hipStream_t s);
 
-// ---- vector-ALU path (ckan_valu.hip): any degree, T = float or double ------
+// ---- general path (ckan_general.hip): any degree, T = float or double ----------
 // Serves fp64 layers and fp32 layers above kMfmaMaxDegree, with C in its own
 // [I, O, D] layout; t = input map of x, [B, I].  rec: the recurrence block
 // (a[D], b[D], c[D], scale, kind) in the element type (fp32: the packed
 // buffer's; fp64: written by launch_write_recur_f64); nullptr (and kind 0)
 // selects the Chebyshev kernels' specialised recurrence.
 constexpr int kMfmaMaxDegree = 16;   // the packed MFMA kernels' limit
-constexpr int kValuMaxDegree = 1024;  // the vector-ALU path's limit
+constexpr int kGeneralMaxDegree = 1024;  // the general path's limit
 // Input derivatives: degree + order at most this (the series' coefficients
 // grow like n^(2 order), past fp32's useful range well before 1024).
 constexpr int kDerivMaxDegree = 256;
 template <typename T>
-void launch_forward_valu(const T* x, const T* C, T* y, T* t, int64_t B, int I, int O, int deg,
+void launch_forward_general(const T* x, const T* C, T* y, T* t, int64_t B, int I, int O, int deg,
                          hipStream_t s, const T* rec = nullptr, int imap = 0, float ima = 0.0f,
                          float imb = 0.0f);
 // dC written by mode om.mode (for T = double: store or accumulate only).
 template <typename T>
-void launch_backward_valu(const T* t, const T* C, const T* dy, T* dx, T* dC, DcOut om, int64_t B,
+void launch_backward_general(const T* t, const T* C, const T* dy, T* dx, T* dC, DcOut om, int64_t B,
                           int I, int O, int deg, hipStream_t s, const T* rec = nullptr,
                           int imap = 0, float ima = 0.0f);
 // The recurrence block (a[D], b[D], c[D], scale, kind) of a ckan_basis_family.
@@ -281,9 +294,9 @@ int pack_forward_ex(const struct ckan_desc* desc, const void* coeffs, void* pack
                     const float* x, float* out, float* t_cache, void* ws, size_t ws_bytes,
                     void* stream, bool t_ready, bool out_tanh,
                     const struct ckan_basis_spec* spec = nullptr);
-// Whether the layer runs on the vector-ALU path (degree > kMfmaMaxDegree),
+// Whether the layer runs on the general path (degree > kMfmaMaxDegree),
 // whose backward differentiates in the layer's own basis.
-bool layer_on_valu(const struct ckan_desc* desc);
+bool layer_is_general(const struct ckan_desc* desc);
 // Validates a basis spec for a layer of degree `degree`; on the MFMA path
 // (degree <= kMfmaMaxDegree) also forms its change of basis into *xf (when
 // xf is given).  Sets the last error on failure.
