@@ -94,15 +94,31 @@ struct TanhJob {
 };
 constexpr int kPackTanhU = 8;  // tanh float4 per thread in flight at once
 
+// The plane operands a split fp32 pack writes beside Cf and Cb (which it
+// rewrites from the same registers): [NBf][KB] and [NIB*P][KBx] fragments of
+// three planes.  The pack is HBM-bound; at 1024 -> 1024, degree 8 (with the
+// tanh of 8192 rows) the planes take it from 28.6 to 40.5 us and the dy
+// re-layout from 20 to 31 us, against 1.2 ms that they take off the GEMMs.
+struct PackPlanes {
+  uint16_t* cf3;
+  uint16_t* cb3;
+};
+static PackPlanes pack_planes(void* packed, const Plan& p) {
+  char* base = reinterpret_cast<char*>(packed);
+  return {reinterpret_cast<uint16_t*>(base + packed_cf3_offset(p)),
+          reinterpret_cast<uint16_t*>(base + packed_cb3_offset(p))};
+}
+
 // One pack block: input block ib, output block ob; `lin` numbers the block
 // for its tanh share.
 template <int P, bool BF, typename CT, bool XF>
 __device__ __forceinline__ void pack_tile(const CT* __restrict__ C, typename Elem<BF>::type* __restrict__ Cf,
                                           typename Elem<BF>::type* __restrict__ Cb,
-                                          float* __restrict__ bias_part, const Plan& p, int cal,
-                                          const XfArg<XF>& xf, const TanhJob& tj, int ib, int ob,
-                                          int64_t lin) {
+                                          float* __restrict__ bias_part, const PackPlanes& pl,
+                                          const Plan& p, int cal, const XfArg<XF>& xf,
+                                          const TanhJob& tj, int ib, int ob, int64_t lin) {
   using G = FwdGroup<P>;
+  constexpr bool SP = !BF && P >= kSplitMinP;
   constexpr int RPMAX = 32 * (P + 1) + 1;
   __shared__ float tile[32 * RPMAX];
   __shared__ float bsum[8][32];
@@ -237,6 +253,7 @@ __device__ __forceinline__ void pack_tile(const CT* __restrict__ C, typename Ele
         v[j] = (d <= p.deg) ? tile[(i - i0) * RP + ol * D + d] : 0.0f;
       }
       store_frag<BF>(Cf + cf_elem<BF>(p.KB, ob, kb, lane) - (size_t)lane * 8, lane, v);
+      if constexpr (SP) store_frag<kSplit>(pl.cf3 + ((size_t)ob * p.KB + kb) * kFragLen<kSplit>, lane, v);
     }
   }
 
@@ -252,7 +269,9 @@ __device__ __forceinline__ void pack_tile(const CT* __restrict__ C, typename Ele
       // scaled by the degree d = e + 1, the factor of dT_d/dt = d U_{d-1}(t)
       v[j] = (e + 1 <= p.deg) ? tile[il * RP + ol * D + e + 1] * (float)(e + 1) : 0.0f;
     }
-    store_frag<BF>(Cb + ((size_t)(ib * P + e) * p.KBx + kbx) * kFragElems, lane, v);
+    const size_t q = (size_t)(ib * P + e) * p.KBx + kbx;
+    if (!SP || packed_has_cb(p)) store_frag<BF>(Cb + q * kFragElems, lane, v);
+    if constexpr (SP) store_frag<kSplit>(pl.cb3 + q * kFragLen<kSplit>, lane, v);
   }
 
   for (int64_t c0 = first_done ? tj0 + 256 * kPackTanhU : tj0; c0 < tj1; c0 += 256 * kPackTanhU) {
@@ -270,9 +289,9 @@ __device__ __forceinline__ void pack_tile(const CT* __restrict__ C, typename Ele
 template <int P, bool BF, typename CT, bool XF>
 __global__ void __launch_bounds__(256)
 k_pack(const CT* __restrict__ C, typename Elem<BF>::type* __restrict__ Cf,
-       typename Elem<BF>::type* __restrict__ Cb, float* __restrict__ bias_part, Plan p, int cal,
-       XfArg<XF> xf, TanhJob tj) {
-  pack_tile<P, BF, CT, XF>(C, Cf, Cb, bias_part, p, cal, xf, tj, blockIdx.x, blockIdx.y,
+       typename Elem<BF>::type* __restrict__ Cb, float* __restrict__ bias_part, PackPlanes pl,
+       Plan p, int cal, XfArg<XF> xf, TanhJob tj) {
+  pack_tile<P, BF, CT, XF>(C, Cf, Cb, bias_part, pl, p, cal, xf, tj, blockIdx.x, blockIdx.y,
                            blockIdx.x + (int64_t)gridDim.x * blockIdx.y);
 }
 
@@ -284,6 +303,7 @@ template <bool BF> struct PackJob {
   typename Elem<BF>::type* Cf;
   typename Elem<BF>::type* Cb;
   float* bias;
+  PackPlanes pl;
   Plan p;
   int cal, nx, nblocks;
   TanhJob tj;
@@ -293,10 +313,10 @@ __global__ void __launch_bounds__(256)
 k_pack2(PackJob<BF> a, PackJob<BF> b) {
   const int bid = blockIdx.x;
   if (bid < a.nblocks)
-    pack_tile<P, BF, float, false>(a.C, a.Cf, a.Cb, a.bias, a.p, a.cal, XfArg<false>{}, a.tj,
+    pack_tile<P, BF, float, false>(a.C, a.Cf, a.Cb, a.bias, a.pl, a.p, a.cal, XfArg<false>{}, a.tj,
                                    bid % a.nx, bid / a.nx, bid);
   else
-    pack_tile<P, BF, float, false>(b.C, b.Cf, b.Cb, b.bias, b.p, b.cal, XfArg<false>{}, b.tj,
+    pack_tile<P, BF, float, false>(b.C, b.Cf, b.Cb, b.bias, b.pl, b.p, b.cal, XfArg<false>{}, b.tj,
                                    (bid - a.nblocks) % b.nx, (bid - a.nblocks) / b.nx, bid - a.nblocks);
 }
 
@@ -322,6 +342,7 @@ k_col_reduce(const float* __restrict__ part, int nparts, int pitch, int n, float
 // Re-lays dy [B, O] (fp32) into
 //   dYx: dX A operand  [B32/32][KBx][64][8]  (rows b, reduction o)
 //   dYc: dC B operand  [NBf][KBc][64][8]     (columns o, reduction b)
+// (three planes per fragment in split mode)
 // and writes colsum_part[bb][o] = sum of dy over rows [64 bb, 64 bb + 64).
 // A wave's unit is (32 columns, 64 rows): it reads that tile of dy once, each
 // load instruction covering 8 whole 128-byte row segments, writes it to a
@@ -334,10 +355,10 @@ k_col_reduce(const float* __restrict__ part, int nparts, int pitch, int n, float
 #define CKAN_PREP_BLOCKS 512
 #endif
 constexpr int kPrepBlocks = CKAN_PREP_BLOCKS;  // grid cap: 2 blocks (8 waves) per CU
-template <bool BF>
+template <int M>
 __global__ void __launch_bounds__(256)
-k_prep_dy(const float* __restrict__ dy, typename Elem<BF>::type* __restrict__ dYx,
-           typename Elem<BF>::type* __restrict__ dYc, float* __restrict__ colsum_part,
+k_prep_dy(const float* __restrict__ dy, typename Elem<M>::type* __restrict__ dYx,
+           typename Elem<M>::type* __restrict__ dYc, float* __restrict__ colsum_part,
            Plan p, int need_dx, int need_dc, int nob, int nbb, int64_t dx_rows, int dyal) {
   constexpr int TP = 36;  // row pitch (floats): 16-byte aligned rows
   constexpr int NL = kPrepRows / 8;
@@ -387,7 +408,7 @@ k_prep_dy(const float* __restrict__ dy, typename Elem<BF>::type* __restrict__ dY
             const f32x4_t a = *reinterpret_cast<const f32x4_t*>(src);
             const f32x4_t e = *reinterpret_cast<const f32x4_t*>(src + 4);
             const float vv[8] = {a[0], a[1], a[2], a[3], e[0], e[1], e[2], e[3]};
-            store_frag<BF>(dYx + ((size_t)(b0 / 32) * p.KBx + ob * 2 + kbl) * kFragElems, lane, vv);
+            store_frag<M>(dYx + ((size_t)(b0 / 32) * p.KBx + ob * 2 + kbl) * kFragLen<M>, lane, vv);
           }
         }
       }
@@ -404,7 +425,7 @@ k_prep_dy(const float* __restrict__ dy, typename Elem<BF>::type* __restrict__ dY
         const int64_t b0 = r0 + kbl * 16;
 #pragma unroll
         for (int j = 0; j < 8; ++j) cs += u[kbl][j];
-        if (b0 < p.Bc) store_frag<BF>(dYc + ((size_t)ob * p.KBc + b0 / 16) * kFragElems, lane, u[kbl]);
+        if (b0 < p.Bc) store_frag<M>(dYc + ((size_t)ob * p.KBc + b0 / 16) * kFragLen<M>, lane, u[kbl]);
       }
       // rows of lane halves interleave in blocks of 8; add the halves in a fixed order
       const float other = __shfl_xor(cs, 32);
@@ -603,10 +624,11 @@ static void launch_pack_t(const void* C, bool c_bf16, void* packed, const Plan& 
   dim3 grid(p.NIB, p.O64 / 32);
   if (c_bf16)
     hipLaunchKernelGGL((k_pack<P, BF, uint16_t, XF>), grid, dim3(256), 0, s,
-                       reinterpret_cast<const uint16_t*>(C), Cf, Cb, bias, p, 0, xf, tj);
+                       reinterpret_cast<const uint16_t*>(C), Cf, Cb, bias, pack_planes(packed, p), p, 0, xf, tj);
   else
     hipLaunchKernelGGL((k_pack<P, BF, float, XF>), grid, dim3(256), 0, s,
-                       reinterpret_cast<const float*>(C), Cf, Cb, bias, p, (int)is_al16(C), xf, tj);
+                       reinterpret_cast<const float*>(C), Cf, Cb, bias, pack_planes(packed, p), p,
+                       (int)is_al16(C), xf, tj);
 }
 
 template <bool XF>
@@ -667,6 +689,7 @@ static void launch_pack2_t(const float* Ca, void* pa, const Plan& qa, const Tanh
     j.Cb = j.Cf + packed_cf_elems(q);
     j.bias = reinterpret_cast<float*>(reinterpret_cast<char*>(packed) +
                                       (q.NIB == 1 ? packed_biasf_offset(q) : packed_bias_offset(q)));
+    j.pl = pack_planes(packed, q);
     j.p = q;
     j.cal = (int)is_al16(C);
     j.nx = q.NIB;
@@ -1015,7 +1038,6 @@ k_dc_pack2(DcPackJob<BF> a, DcPackJob<BF> b, LossMean lm) {
 // fragment layout.  Block: 32 rows x 8 inputs, one (row, input) per thread;
 // dy rows and the block's coefficients are staged in LDS with every load in
 // flight at once.
-constexpr int kDxSmallO = 64;  // outputs staged at once (all of them)
 template <int P, bool BF>
 __device__ __forceinline__ void dx_small_body(const float* __restrict__ dy,
                                               const typename Elem<BF>::type* __restrict__ Cb,
@@ -1259,12 +1281,16 @@ void launch_prep_dy(const float* dy, void* dYx, void* dYc, float* colsum_part, c
   const int nbb = (int)ceil_div(row_end, kPrepRows);
   const int64_t blocks = ceil_div((int64_t)nob * nbb, 4);
   dim3 grid((unsigned)(blocks < kPrepBlocks ? blocks : kPrepBlocks));
-  if (p.esz == 2)
-    hipLaunchKernelGGL((k_prep_dy<true>), grid, dim3(256), 0, s, dy,
+  if (p.split)
+    hipLaunchKernelGGL((k_prep_dy<kSplit>), grid, dim3(256), 0, s, dy,
+                       reinterpret_cast<uint16_t*>(dYx), reinterpret_cast<uint16_t*>(dYc),
+                       colsum_part, p, (int)need_dx, (int)need_dc, nob, nbb, dx_rows, (int)is_al16(dy));
+  else if (p.esz == 2)
+    hipLaunchKernelGGL((k_prep_dy<kBf16>), grid, dim3(256), 0, s, dy,
                        reinterpret_cast<uint16_t*>(dYx), reinterpret_cast<uint16_t*>(dYc),
                        colsum_part, p, (int)need_dx, (int)need_dc, nob, nbb, dx_rows, (int)is_al16(dy));
   else
-    hipLaunchKernelGGL((k_prep_dy<false>), grid, dim3(256), 0, s, dy,
+    hipLaunchKernelGGL((k_prep_dy<kFp32>), grid, dim3(256), 0, s, dy,
                        reinterpret_cast<float*>(dYx), reinterpret_cast<float*>(dYc),
                        colsum_part, p, (int)need_dx, (int)need_dc, nob, nbb, dx_rows, (int)is_al16(dy));
 }
@@ -1276,15 +1302,11 @@ float* launch_colsum_reduce(float* colsum_part, const Plan& p, hipStream_t s) {
   return colsum;
 }
 
+// Fp32 layers of degree 1-2: the only ones whose dC is not pipelined.
 void launch_dc_finalize(const float* part, int S, const float* colsum, float* dC,
                         DcOut om, const Plan& p, hipStream_t s) {
   dim3 grid((unsigned)ceil_div(p.I, 16), (unsigned)ceil_div(p.O, 64));
-  switch (p.P) {
-    case 2: hipLaunchKernelGGL((k_dc_finalize<2>), grid, dim3(256), 0, s, part, S, colsum, dC, om, p); break;
-    case 4: hipLaunchKernelGGL((k_dc_finalize<4>), grid, dim3(256), 0, s, part, S, colsum, dC, om, p); break;
-    case 8: hipLaunchKernelGGL((k_dc_finalize<8>), grid, dim3(256), 0, s, part, S, colsum, dC, om, p); break;
-    default: hipLaunchKernelGGL((k_dc_finalize<16>), grid, dim3(256), 0, s, part, S, colsum, dC, om, p); break;
-  }
+  hipLaunchKernelGGL((k_dc_finalize<2>), grid, dim3(256), 0, s, part, S, colsum, dC, om, p);
 }
 
 // dC[q] (stored, added or applied as an SGD step, by om) = sum_z part[z][q],

@@ -54,6 +54,22 @@ template <int P> struct FwdGroup {
 __host__ __device__ inline int fwd_sgi(int P) { return 4 * 2 * (P < 8 ? 8 / P : 1); }
 __host__ __device__ inline int fwd_sgk(int P) { return 4 * (P > 8 ? P / 8 : 1); }
 
+// The operand modes of the MFMA kernels: fp32 instructions, bf16, or fp32 by
+// bf16 instructions ("split").  In split mode an fp32 value x is the exact sum
+// of three bf16 values h + m + l (each the rounding of what the ones before
+// left, 3 x 8 significant bits), an operand fragment is three 1 KiB planes,
+// and a product takes the six plane products above 2^-24 of it: h l, l h, m m,
+// h m, m h, h h, summed in fp32 in that order.  Six bf16 instructions take
+// 192 clk per 32x32x16 block product against 512 for eight fp32 ones, and
+// round the accumulator less often: the errors against 64 bits are below the
+// fp32 instruction's at every length and distribution tried (K = 512 / 8192
+// normal coefficients: 3.2e-7 / 1.4e-6 against 4.1e-7 / 1.6e-6).  Four or
+// three products are not enough (3e-6 at any length).
+enum OperandMode : int { kFp32 = 0, kBf16 = 1, kSplit = 2 };
+// Degrees 1-2 (P = 2) stay on the fp32 instructions: their kernels are bound by
+// the operand traffic, which the planes would raise by half.
+constexpr int kSplitMinP = 4;
+
 inline int64_t round_up(int64_t a, int64_t b) { return (a + b - 1) / b * b; }
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
@@ -77,6 +93,8 @@ struct Plan {
   int64_t Bc, KBc; // rows padded to kDcStageRows; dC reduction k-blocks
   int NBB;         // prep_dy row blocks (colsum partials)
   int esz;         // bytes per packed operand element (2 bf16, 4 fp32)
+  bool split;      // fp32 by three-plane bf16 operands (kSplit below)
+  int bsz;         // bytes per element of the backward operands (2, 4, or 6 split)
   int imap;        // input map: 0 t = tanh(x), 1 t = ima * x + imb
   float ima, imb;
 };
@@ -237,6 +255,8 @@ inline Plan make_plan(int64_t B, int I, int O, int deg, bool bf16) {
   p.KBc = p.Bc / 16;
   p.NBB = (int)ceil_div(B, kPrepRows);
   p.esz = bf16 ? 2 : 4;
+  p.split = !bf16 && p.P >= kSplitMinP;
+  p.bsz = p.split ? 6 : p.esz;
   p.imap = 0;
   p.ima = p.imb = 0.0f;
   return p;
@@ -246,31 +266,80 @@ inline Plan make_plan(int64_t B, int I, int O, int deg, bool bf16) {
 // Device helpers
 // ---------------------------------------------------------------------------
 
-template <bool BF> struct Elem;
-template <> struct Elem<true> { typedef uint16_t type; };
-template <> struct Elem<false> { typedef float type; };
+template <int M> struct Elem;
+template <> struct Elem<kBf16> { typedef uint16_t type; };
+template <> struct Elem<kFp32> { typedef float type; };
+template <> struct Elem<kSplit> { typedef uint16_t type; };
 
 // One lane's share of an MFMA operand fragment for one k-block.
-template <bool BF> struct Frag;
-template <> struct Frag<true> { bf16x8_t v; };
-template <> struct Frag<false> { f32x4_t lo, hi; };
+template <int M> struct Frag;
+template <> struct Frag<kBf16> { bf16x8_t v; };
+template <> struct Frag<kFp32> { f32x4_t lo, hi; };
+template <> struct Frag<kSplit> { bf16x8_t p[3]; };  // h, m, l
 
-__device__ __forceinline__ Frag<true> make_frag_bf(const float* v) {
-  Frag<true> f;
+// Elements (of Elem<M>) of a fragment.
+template <int M> constexpr int kFragLen = M == kSplit ? 3 * kFragElems : kFragElems;
+
+__device__ __forceinline__ Frag<kBf16> make_frag_bf(const float* v) {
+  Frag<kBf16> f;
 #pragma unroll
   for (int j = 0; j < 8; ++j) f.v[j] = (__bf16)v[j];  // v_cvt_pk_bf16_f32, RNE
   return f;
 }
 
-template <bool BF> __device__ __forceinline__ Frag<BF> make_frag(const float* v);
-template <> __device__ __forceinline__ Frag<true> make_frag<true>(const float* v) {
+// The planes of 8 finite values.
+__device__ __forceinline__ Frag<kSplit> make_frag_split(const float* v) {
+  Frag<kSplit> f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const __bf16 h = (__bf16)v[j];
+    const float r = v[j] - (float)h;  // exact
+    const __bf16 m = (__bf16)r;
+    f.p[0][j] = h;
+    f.p[1][j] = m;
+    f.p[2][j] = (__bf16)(r - (float)m);
+  }
+  return f;
+}
+// The planes of values a caller handed in (coefficients, dy), which may be
+// infinite, NaN or next to overflow.  A non-finite value goes to the l plane
+// alone: its only product is with the other operand's h plane, so it keeps the
+// sign and the infinity that the fp32 product has (in the h plane it would
+// also meet the m and l planes, whose signs differ).  A finite value whose
+// rounding to bf16 overflows takes the largest finite bf16 instead.
+__device__ __forceinline__ Frag<kSplit> make_frag_split_any(const float* v) {
+  float s[8];
+  bool odd = false;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) odd |= (__float_as_uint(v[j]) & 0x7fffffffu) >= 0x7f7f8000u;
+  if (!odd) return make_frag_split(v);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) s[j] = __builtin_isfinite(v[j]) ? v[j] : 0.0f;
+  Frag<kSplit> f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float h = __uint_as_float(__float_as_uint(s[j]) & 0xffff0000u);  // toward zero
+    const float r = s[j] - h;
+    const __bf16 m = (__bf16)r;
+    f.p[0][j] = (__bf16)h;
+    f.p[1][j] = m;
+    f.p[2][j] = __builtin_isfinite(v[j]) ? (__bf16)(r - (float)m) : (__bf16)v[j];
+  }
+  return f;
+}
+
+template <int M> __device__ __forceinline__ Frag<M> make_frag(const float* v);
+template <> __device__ __forceinline__ Frag<kBf16> make_frag<kBf16>(const float* v) {
   return make_frag_bf(v);
 }
-template <> __device__ __forceinline__ Frag<false> make_frag<false>(const float* v) {
-  Frag<false> f;
+template <> __device__ __forceinline__ Frag<kFp32> make_frag<kFp32>(const float* v) {
+  Frag<kFp32> f;
   f.lo = f32x4_t{v[0], v[1], v[2], v[3]};
   f.hi = f32x4_t{v[4], v[5], v[6], v[7]};
   return f;
+}
+template <> __device__ __forceinline__ Frag<kSplit> make_frag<kSplit>(const float* v) {
+  return make_frag_split(v);
 }
 
 // The bf16 forward coefficients (Cf) are stored by 8-output streams: for a
@@ -292,7 +361,13 @@ template <bool BF> __host__ __device__ inline size_t cf_elem(int KB, int nb, int
 }
 
 // Load this lane's 8 values of a fragment stored at `base` (fragment start).
-template <bool BF> __device__ __forceinline__ Frag<BF> load_frag(const typename Elem<BF>::type* base, int lane);
+template <int M> __device__ __forceinline__ Frag<M> load_frag(const typename Elem<M>::type* base, int lane);
+template <> __device__ __forceinline__ Frag<kSplit> load_frag<kSplit>(const uint16_t* base, int lane) {
+  Frag<kSplit> f;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) f.p[k] = *reinterpret_cast<const bf16x8_t*>(base + k * kFragElems + lane * 8);
+  return f;
+}
 template <> __device__ __forceinline__ Frag<true> load_frag<true>(const uint16_t* base, int lane) {
   Frag<true> f;
   f.v = *reinterpret_cast<const bf16x8_t*>(base + lane * 8);
@@ -311,7 +386,7 @@ template <> __device__ __forceinline__ Frag<false> load_frag<false>(const float*
 // they leave the caches to the data that is reused (config 5 at B = 1:
 // 14.1 -> 13.2 us cold).  Outputs nothing in the same step reads again (y,
 // dx, dC) are stored non-temporally for the same reason.
-template <bool BF> __device__ __forceinline__ Frag<BF> load_frag_nt(const typename Elem<BF>::type* base, int lane);
+template <int M> __device__ __forceinline__ Frag<M> load_frag_nt(const typename Elem<M>::type* base, int lane);
 template <> __device__ __forceinline__ Frag<true> load_frag_nt<true>(const uint16_t* base, int lane) {
   Frag<true> f;
   f.v = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(base + lane * 8));
@@ -325,7 +400,7 @@ template <> __device__ __forceinline__ Frag<false> load_frag_nt<false>(const flo
   return f;
 }
 
-template <bool BF> __device__ __forceinline__ Frag<BF> zero_frag();
+template <int M> __device__ __forceinline__ Frag<M> zero_frag();
 template <> __device__ __forceinline__ Frag<true> zero_frag<true>() {
   Frag<true> f;
 #pragma unroll
@@ -340,7 +415,12 @@ template <> __device__ __forceinline__ Frag<false> zero_frag<false>() {
 }
 
 // Store 8 values as this lane's share of a fragment at `base`.
-template <bool BF> __device__ __forceinline__ void store_frag(typename Elem<BF>::type* base, int lane, const float* v);
+template <int M> __device__ __forceinline__ void store_frag(typename Elem<M>::type* base, int lane, const float* v);
+template <> __device__ __forceinline__ void store_frag<kSplit>(uint16_t* base, int lane, const float* v) {
+  const Frag<kSplit> f = make_frag_split_any(v);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) *reinterpret_cast<bf16x8_t*>(base + k * kFragElems + lane * 8) = f.p[k];
+}
 template <> __device__ __forceinline__ void store_frag<true>(uint16_t* base, int lane, const float* v) {
   Frag<true> f = make_frag_bf(v);
   *reinterpret_cast<bf16x8_t*>(base + lane * 8) = f.v;
@@ -364,6 +444,48 @@ __device__ __forceinline__ void mma(f32x16_t& acc, const Frag<false>& a, const F
   acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.hi[1], b.hi[1], acc, 0, 0, 0);
   acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.hi[2], b.hi[2], acc, 0, 0, 0);
   acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.hi[3], b.hi[3], acc, 0, 0, 0);
+}
+
+// The six plane products, smallest first.
+constexpr int kSplitProducts = 6;
+template <int Q> __device__ __forceinline__ void mma_split(f32x16_t& acc, const Frag<kSplit>& a, const Frag<kSplit>& b) {
+  constexpr int ia[kSplitProducts] = {0, 2, 1, 0, 1, 0}, ib[kSplitProducts] = {2, 0, 1, 1, 0, 0};
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[ia[Q]], b.p[ib[Q]], acc, 0, 0, 0);
+}
+__device__ __forceinline__ void mma(f32x16_t& acc, const Frag<kSplit>& a, const Frag<kSplit>& b) {
+  mma_split<0>(acc, a, b);
+  mma_split<1>(acc, a, b);
+  mma_split<2>(acc, a, b);
+  mma_split<3>(acc, a, b);
+  mma_split<4>(acc, a, b);
+  mma_split<5>(acc, a, b);
+}
+// The same for two accumulators, their instructions alternating so that
+// none waits for the one before it.
+__device__ __forceinline__ void mma2(f32x16_t& c0, const Frag<kSplit>& a0, const Frag<kSplit>& b0,
+                                     f32x16_t& c1, const Frag<kSplit>& a1, const Frag<kSplit>& b1) {
+  mma_split<0>(c0, a0, b0); mma_split<0>(c1, a1, b1);
+  mma_split<1>(c0, a0, b0); mma_split<1>(c1, a1, b1);
+  mma_split<2>(c0, a0, b0); mma_split<2>(c1, a1, b1);
+  mma_split<3>(c0, a0, b0); mma_split<3>(c1, a1, b1);
+  mma_split<4>(c0, a0, b0); mma_split<4>(c1, a1, b1);
+  mma_split<5>(c0, a0, b0); mma_split<5>(c1, a1, b1);
+}
+// mma2 with the five small products summed apart (e0, e1).
+__device__ __forceinline__ void mma_apart(f32x16_t& c0, f32x16_t& e0, const Frag<kSplit>& a0,
+                                          const Frag<kSplit>& b0, f32x16_t& c1, f32x16_t& e1,
+                                          const Frag<kSplit>& a1, const Frag<kSplit>& b1) {
+  mma_split<0>(e0, a0, b0); mma_split<0>(e1, a1, b1);
+  mma_split<5>(c0, a0, b0); mma_split<5>(c1, a1, b1);
+  mma_split<1>(e0, a0, b0); mma_split<1>(e1, a1, b1);
+  mma_split<2>(e0, a0, b0); mma_split<2>(e1, a1, b1);
+  mma_split<3>(e0, a0, b0); mma_split<3>(e1, a1, b1);
+  mma_split<4>(e0, a0, b0); mma_split<4>(e1, a1, b1);
+}
+template <int M> __device__ __forceinline__ void mma2(f32x16_t& c0, const Frag<M>& a0, const Frag<M>& b0,
+                                                       f32x16_t& c1, const Frag<M>& a1, const Frag<M>& b1) {
+  mma(c0, a0, b0);
+  mma(c1, a1, b1);
 }
 
 // ---- pipeline primitives ----------------------------------------------------

@@ -609,6 +609,225 @@ k_fwd_pipe(const float* __restrict__ tc, const typename Elem<BF>::type* __restri
 }
 
 // ---------------------------------------------------------------------------
+// Forward, large batch, split fp32 (kSplit): block tile 256 rows x 32 NN
+// outputs, 8 waves (2 per SIMD) of one row fragment each, so a wave's basis
+// fragments are its own (no value is generated twice in a block) and serve NN
+// output fragments, six products each: 24 MFMAs (768 clk) per generated
+// fragment at NN = 4, beside ~110 vector instructions for the recurrence and
+// the planes, which the SIMD's other wave overlaps.  A stage is 4 k-blocks
+// (12 KiB of coefficient planes per output fragment, and the super-group's
+// tanh tile): 6144 clk of products per SIMD, so two ring slots hide the copies,
+// issued by every wave at the start of a stage for the next one.
+// At 8192 x 1024 -> 1024, degree 8: 983 us on the fp32 instructions (96 % of
+// their peak) -> 580-600 us, 1.4 PFLOP/s of bf16 products, what hipBLASLt's
+// bf16 GEMM reaches on 8192^3 on the same card (1.44): the MFMA pipe is busy 77 %
+// of the cycles at 1.7 GHz, where the card's power holds it.  Generating each
+// stage's first fragment before its barrier (tanh tiles one stage further
+// ahead) changed the clock, not the time.  Error against 64 bits there: 1.0e-6
+// on the fp32 instructions (two chains), 5.3e-7 here (1.3e-6 with all six
+// products in one accumulator).
+// ---------------------------------------------------------------------------
+template <int P, int NN>
+struct FwdSplit {
+  typedef FwdGroup<P> G;
+  static constexpr int BM = 256, THREADS = 512;
+  static constexpr int FB = kFragLen<kSplit> * 2;
+  static constexpr int KS = 4;                    // k-blocks per stage
+  static constexpr int HS = G::SGK / KS;          // stages per super-group
+  static constexpr int B_BYTES = NN * KS * FB;
+  static constexpr int T_BYTES = BM * G::SGI * 4;
+  static constexpr int STAGE_BYTES = B_BYTES + T_BYTES;
+  static constexpr int B_OPS = B_BYTES / (1024 * 8), T_OPS = T_BYTES / (1024 * 8);  // copies per wave
+  static constexpr int BIAS_BYTES = NN * 32 * 4;
+  static constexpr int LDS_BYTES = 2 * STAGE_BYTES + BIAS_BYTES;
+  static_assert(LDS_BYTES <= 160 * 1024 && B_BYTES % 8192 == 0 && T_BYTES % 8192 == 0, "stage copies");
+};
+
+// Arguments as k_fwd_pipe's.
+template <int P, bool OT, int NN>
+__global__ void __launch_bounds__(512)
+k_fwd_split(const float* __restrict__ tc, const uint16_t* __restrict__ Cf3,
+            const float* __restrict__ bias_f, float* __restrict__ y, float* __restrict__ part,
+            Plan p, int sg_per_split, const float* __restrict__ bias_part, int nib,
+            float* __restrict__ bias_out) {
+  typedef FwdSplit<P, NN> K;
+  typedef typename K::G G;
+  constexpr int KS = K::KS, HS = K::HS, FB = K::FB, KBG = G::KBG;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int bx, by;
+  xcd_patch(bx, by);
+  const int64_t m_blk = (int64_t)bx * K::BM;
+  const int nb0 = by * NN;
+  const int nsg = p.I_sg / G::SGI;
+  const int sg0 = blockIdx.z * sg_per_split;
+  const int nst = (min(nsg, sg0 + sg_per_split) - sg0) * HS;
+
+  // copies: a coefficient copy is one plane of one fragment (1 KiB, lane order);
+  // tanh copy c = (q * 8 + wave) * 64 + lane fills stored chunk c of the tile
+  const char* bsrc = reinterpret_cast<const char*>(Cf3) + (size_t)sg0 * G::SGK * FB;
+  size_t boff[K::B_OPS];  // uniform
+#pragma unroll
+  for (int q = 0; q < K::B_OPS; ++q) {
+    const int c = q * 8 + wave;  // plane c % 3 of k-block c / 3 % KS of fragment c / (3 KS)
+    const int nb = min(nb0 + c / (3 * KS), p.NBf - 1);
+    boff[q] = (size_t)nb * p.KB * FB + (size_t)(c % (3 * KS)) * 1024;
+  }
+  const char* tsrc = reinterpret_cast<const char*>(tc) + ((size_t)m_blk * p.I_sg + (size_t)sg0 * G::SGI) * 4;
+  uint32_t toff[K::T_OPS];
+#pragma unroll
+  for (int q = 0; q < K::T_OPS; ++q) {
+    const int c = (q * 8 + wave) * 64 + lane;
+    const int rl = c / (G::SGI / 4), part4 = c - rl * (G::SGI / 4);
+    int64_t r = m_blk + rl;
+    if (r >= p.B) r = p.B - 1;  // rows past B: results not stored
+    toff[q] = (uint32_t)(((size_t)(r - m_blk) * p.I_sg + (part4 ^ fwd_t_xor<G::SGI / 4>(rl)) * 4) * 4);
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
+  const uint32_t l16 = lane * 16;
+  auto issue = [&](int st) __attribute__((always_inline)) {
+    const uint32_t l = lds0 + (st & 1) * K::STAGE_BYTES + wave * 1024;
+#pragma unroll
+    for (int q = 0; q < K::B_OPS; ++q) dma16s_salu(bsrc + boff[q] + (size_t)st * KS * FB, l16, l + q * 8192);
+#pragma unroll
+    for (int q = 0; q < K::T_OPS; ++q)
+      dma16s_salu(tsrc + (size_t)(st / HS) * G::SGI * 4, toff[q], l + K::B_BYTES + q * 8192);
+  };
+
+  // h h products, and the five small ones apart: a chain of K / 16 roundings at
+  // the size of the result instead of six times as many
+  f32x16_t acc[NN], lo[NN];
+#pragma unroll
+  for (int ni = 0; ni < NN; ++ni)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[ni][v] = lo[ni][v] = 0.0f;
+
+  auto compute = [&](int st) __attribute__((always_inline)) {
+    const char* base = smem + (st & 1) * K::STAGE_BYTES;
+    const uint16_t* bl = reinterpret_cast<const uint16_t*>(base);
+    const float* tl = reinterpret_cast<const float*>(base + K::B_BYTES);
+    const int hs = HS == 1 ? 0 : st % HS;
+    float tv[G::LANE_T];
+    {
+      const int rl = wave * 32 + (lane & 31);
+      const f32x4_t* src = reinterpret_cast<const f32x4_t*>(tl + rl * G::SGI);
+      const int sx = fwd_t_xor<G::SGI / 4>(rl);
+#pragma unroll
+      for (int q = 0; q < G::LANE_T / 4; ++q) {
+        const f32x4_t w = src[(g * (G::LANE_T / 4) + q) ^ sx];
+        tv[4 * q + 0] = w[0]; tv[4 * q + 1] = w[1];
+        tv[4 * q + 2] = w[2]; tv[4 * q + 3] = w[3];
+      }
+    }
+    // k-block kb of the stage: group s (of the stage's KS / KBG), half h of its degrees
+    constexpr int NS = KS / KBG;
+    static_assert(HS == 1 || (HS == 2 && G::IPG == 2), "stages per super-group");
+    Frag<kSplit> af[2][KBG], bq[2][2];
+    auto gen = [&](int s, Frag<kSplit> (&dst)[KBG]) __attribute__((always_inline)) {
+      float vals[8 * KBG];
+#pragma unroll
+      for (int u = 0; u < G::IPG / 2; ++u) {
+        float t;
+        if constexpr (HS == 1) t = tv[s * (G::IPG / 2) + u];
+        else t = hs ? tv[NS + s] : tv[s];  // two stages a super-group, one input per group
+        cheb_T<P>(t, vals + u * P);
+      }
+#pragma unroll
+      for (int h = 0; h < KBG; ++h) dst[h] = make_frag_split(vals + 8 * h);
+    };
+    auto load_b = [&](int kb, int np, Frag<kSplit> (&dst)[2]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        dst[j] = load_frag<kSplit>(bl + (size_t)((np * 2 + j) * KS + kb) * kFragLen<kSplit>, lane);
+    };
+    constexpr int NP = NN / 2;  // output fragments go in pairs
+    load_b(0, 0, bq[0]);
+    gen(0, af[0]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int kb = 0; kb < KS; ++kb) {
+      const int s = kb / KBG, h = kb % KBG;
+#pragma unroll
+      for (int np = 0; np < NP; ++np) {
+        const int cur = (kb * NP + np) & 1;
+        // the next pair's planes, and the next group's basis, beside this pair's MFMAs
+        if (np + 1 < NP) load_b(kb, np + 1, bq[cur ^ 1]);
+        else if (kb + 1 < KS) load_b(kb + 1, 0, bq[cur ^ 1]);
+        if (np == 0 && h == 0 && s + 1 < NS) gen(s + 1, af[(s + 1) & 1]);
+        mma_apart(acc[2 * np], lo[2 * np], af[s & 1][h], bq[cur][0], acc[2 * np + 1], lo[2 * np + 1],
+                  af[s & 1][h], bq[cur][1]);
+      }
+#pragma unroll
+      for (int q = 0; q < NN * kSplitProducts; ++q) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
+        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);  // up to five VALU
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // up to one LDS read
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  pin_sgpr(y);  // used after the loop
+  pin_sgpr(part);
+  pin_sgpr(bias_f);
+  pin_sgpr(bias_part);
+  pin_sgpr(bias_out);
+  pin_sgpr(nib);
+  issue(0);
+  for (int st = 0; st < nst; ++st) {
+    // stage st landed; every wave has read stage st - 1, so its slot is free
+    wait_vmcnt<0>();
+    wait_lgkmcnt<0>();
+    block_barrier();
+    if (st + 1 < nst) issue(st + 1);
+    compute(st);
+  }
+
+  // bias from the partials, in k_col_reduce's order (as in k_fwd_pipe)
+  const bool split = gridDim.z > 1;
+  float* bias_l = reinterpret_cast<float*>(smem + 2 * K::STAGE_BYTES);
+  if (nib > 0) {
+    const int bo = nb0 * 32 + (tid >> 2);
+    const bool mine = (tid >> 2) < NN * 32;
+    float bsum = 0.0f;
+    if (mine && bo < p.O32)
+      for (int k = tid & 3; k < nib; k += 4) bsum += bias_part[(size_t)k * p.O32 + bo];
+    const int q0 = lane & ~3;
+    const float s0 = __shfl(bsum, q0), s1 = __shfl(bsum, q0 + 1);
+    const float s2 = __shfl(bsum, q0 + 2), s3 = __shfl(bsum, q0 + 3);
+    const float tot = ((s0 + s1) + s2) + s3;
+    if ((tid & 3) == 0 && mine) {
+      bias_l[tid >> 2] = tot;
+      if (bias_out && bx == 0 && blockIdx.z == 0 && bo < p.O32) bias_out[bo] = tot;
+    }
+    __syncthreads();
+  }
+  const bool full_rows = m_blk + K::BM <= (split ? p.B32 : p.B);
+  const int64_t pitch = split ? p.O32 : p.O, nrow = split ? p.B32 : p.B;
+  float* out = split ? part + (size_t)blockIdx.z * p.B32 * p.O32 : y;
+#pragma unroll
+  for (int ni = 0; ni < NN; ++ni) {
+    const int nb = nb0 + ni;
+    const int o = nb * 32 + (lane & 31);
+    if (split ? nb >= p.NBf : o >= p.O) continue;
+    const float add = split ? 0.0f : (nib > 0 ? bias_l[ni * 32 + (lane & 31)] : bias_f[o]);
+    const int64_t r0 = m_blk + wave * 32 + 4 * g;
+    float* op = out + r0 * pitch + o;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int rv = 8 * (v >> 2) + (v & 3);
+      if (!full_rows && r0 + rv >= nrow) continue;
+      const float yv = (acc[ni][v] + lo[ni][v]) + add;
+      float* a = op + rv * pitch;
+      if (split) *a = yv;
+      else if constexpr (OT) *a = tanhf(yv);  // read again soon, by the next layer
+      else __builtin_nontemporal_store(yv, a);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Forward, small batch (B <= 64): coefficient streaming.  The work is the
 // HBM stream of Cf; the MFMAs run at a few percent of their peak.  Each wave
 // takes one 32-output column block and SPW super-groups (16 k-blocks) of the
@@ -1187,161 +1406,11 @@ k_fwd_cols(const float* __restrict__ x, float* __restrict__ tc, const uint16_t* 
 }
 
 // ---------------------------------------------------------------------------
-// dX, pipelined.  A block's tile is 256 rows (4 waves x NM fragments) x one
-// input block (32 inputs x P degrees).  Both operands (dy fragments for the
-// wave's rows, coefficient fragments for the input block) are copied
-// global -> LDS by global_load_lds_dwordx4 into a ring of NBUF stages of KI
-// k-blocks (16 outputs each), NBUF-1 stages ahead; each wave reads the next
-// k-block's fragments into registers while its MFMAs run on the current one.
-// The epilogue sums over degrees with d U_{d-1}(t) and the tanh chain factor
-// in registers.
-// ---------------------------------------------------------------------------
-template <int P, bool BF>
-struct DxPipe {
-  typedef typename Elem<BF>::type E;
-  static constexpr int NM = BwdTile<P>::NM, WGM = 4, KI = 2;  // KI even (loop unroll)
-  static constexpr int FB = kFragElems * (int)sizeof(E);  // bytes per fragment
-  static constexpr int A_BYTES = WGM * NM * KI * FB;
-  static constexpr int B_BYTES = P * KI * FB;
-  static constexpr int STAGE_BYTES = A_BYTES + B_BYTES;
-  static constexpr int NBUF_FIT = (160 * 1024) / STAGE_BYTES;
-  static constexpr int NBUF = NBUF_FIT > 5 ? 5 : NBUF_FIT;
-  static constexpr int OPS = STAGE_BYTES / 4096;  // dma16 per thread per stage
-  static constexpr int A_OPS = A_BYTES / 4096;
-  static constexpr bool kOk = NBUF >= 3 && STAGE_BYTES % 4096 == 0 && A_BYTES % 4096 == 0 &&
-                              OPS * (NBUF - 2) < 64;
-};
-
-template <int P, bool BF>
-__global__ void __launch_bounds__(256)
-k_dx_pipe(const typename Elem<BF>::type* __restrict__ dYx,
-          const typename Elem<BF>::type* __restrict__ Cb, const float* __restrict__ tc,
-          float* __restrict__ dx, Plan p, int n_rb) {
-  typedef DxPipe<P, BF> K;
-  typedef typename K::E E;
-  constexpr int NM = K::NM, WGM = K::WGM, KI = K::KI, FB = K::FB, NBUF = K::NBUF;
-  constexpr int RUN = KI * FB / 16;  // 16-byte chunks per contiguous fragment run
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int g = lane >> 5;
-  const int nst = p.KBx / KI;
-  const int rb = blockIdx.x % n_rb, ib = blockIdx.x / n_rb;
-
-  // per-op source offsets (bytes); dYx rows are padded to whole tiles
-  const char* abase = reinterpret_cast<const char*>(dYx) + (size_t)rb * WGM * NM * p.KBx * FB;
-  const char* bbase = reinterpret_cast<const char*>(Cb) + (size_t)ib * P * p.KBx * FB;
-  uint32_t off[K::OPS];
-#pragma unroll
-  for (int q = 0; q < K::OPS; ++q) {
-    const int c = (q * 4 + wave) * 64 + lane;
-    if (q < K::A_OPS) {
-      const int run = c / RUN, w = c - run * RUN;  // run = wave' * NM + mi
-      off[q] = (uint32_t)(run * p.KBx * FB + w * 16);
-    } else {
-      const int cc = c - K::A_OPS * 256;
-      const int e = cc / RUN, w = cc - e * RUN;
-      off[q] = (uint32_t)(e * p.KBx * FB + w * 16);
-    }
-  }
-  auto issue = [&](int st) __attribute__((always_inline)) {
-    if (st >= nst) return;
-    const size_t sb = (size_t)st * KI * FB;
-    char* dst = smem + (st % NBUF) * K::STAGE_BYTES + wave * 1024;
-#pragma unroll
-    for (int q = 0; q < K::OPS; ++q)
-      dma16((q < K::A_OPS ? abase : bbase) + sb + off[q], dst + q * 4096);
-  };
-
-  struct Regs {
-    Frag<BF> a[NM];
-    Frag<BF> b[P];
-  };
-  auto lds_read = [&](int kb, Regs& R) __attribute__((always_inline)) {
-    const int kk = kb % KI;
-    const char* base = smem + ((kb / KI) % NBUF) * K::STAGE_BYTES;
-#pragma unroll
-    for (int mi = 0; mi < NM; ++mi)
-      R.a[mi] = load_frag<BF>(reinterpret_cast<const E*>(base + ((wave * NM + mi) * KI + kk) * FB), lane);
-#pragma unroll
-    for (int e = 0; e < P; ++e)
-      R.b[e] = load_frag<BF>(reinterpret_cast<const E*>(base + K::A_BYTES + (e * KI + kk) * FB), lane);
-  };
-
-  f32x16_t acc[NM][P];
-#pragma unroll
-  for (int mi = 0; mi < NM; ++mi)
-#pragma unroll
-    for (int e = 0; e < P; ++e)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[mi][e][v] = 0.0f;
-
-#pragma unroll
-  for (int q = 0; q < NBUF - 1; ++q) issue(q);
-  if (NBUF - 2 <= nst - 1) wait_vmcnt<K::OPS * (NBUF - 2)>();
-  else wait_vmcnt<0>();
-  block_barrier();
-  // the transition into stage st refills with st + NBUF - 1; stage 0 has no
-  // transition, so its refill (stage NBUF - 1) is issued here
-  issue(NBUF - 1);
-  Regs R0, R1;
-  lds_read(0, R0);
-
-  const int nkb = nst * KI;
-  auto step = [&](int kb, const Regs& Rc, Regs& Rn) __attribute__((always_inline)) {
-    const int nxt = kb + 1;
-    if (nxt < nkb) {
-      if (nxt % KI == 0) {
-        const int st = nxt / KI;
-        wait_lgkmcnt<0>();  // this wave's reads of the slot being refilled are done
-        if (st + NBUF - 2 <= nst - 1) wait_vmcnt<K::OPS * (NBUF - 2)>();
-        else wait_vmcnt<0>();
-        block_barrier();
-        issue(st + NBUF - 1);
-      }
-      lds_read(nxt, Rn);
-    }
-#pragma unroll
-    for (int mi = 0; mi < NM; ++mi)
-#pragma unroll
-      for (int e = 0; e < P; ++e) mma(acc[mi][e], Rc.a[mi], Rc.b[e]);
-  };
-  for (int kb = 0; kb < nkb; kb += 2) {
-    step(kb, R0, R1);
-    step(kb + 1, R1, R0);
-  }
-
-  const int i = ib * 32 + (lane & 31);
-  const bool icol = i < p.I;
-#pragma unroll
-  for (int mi = 0; mi < NM; ++mi) {
-    const int64_t r0 = ((int64_t)rb * WGM * NM + wave * NM + mi) * 32 + 4 * g;
-    float tv[16];
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int64_t r = r0 + 8 * (v >> 2) + (v & 3);
-      tv[v] = (icol && r < p.B) ? tc[r * p.I_sg + i] : 0.0f;
-    }
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int64_t r = r0 + 8 * (v >> 2) + (v & 3);
-      const float t2 = tv[v] + tv[v];
-      float up = 0.0f, u = 1.0f, sum = 0.0f;  // U_{-1}, U_0
-#pragma unroll
-      for (int e = 0; e < P; ++e) {
-        sum = fmaf(acc[mi][e][v], u, sum);
-        const float un = fmaf(t2, u, -up);
-        up = u;
-        u = un;
-      }
-      if (icol && r < p.B) __builtin_nontemporal_store(sum * input_slope(tv[v], p), dx + r * p.I + i);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
 // dX for degrees up to 8 (and fp32 at degree 16, with NM = 1: 128-row
-// blocks; bf16 at degree 16 takes k_dx16 below).  One block = 2*RG waves
+// blocks; bf16 at degree 16 takes k_dx16 below).  Split fp32 (M = kSplit) holds
+// two or three stages of one k-block, 48 products a wave each; at 8192 x
+// 1024 -> 1024, degree 8: 992 us on the fp32 instructions -> 535-555 us (MFMA
+// busy 80 % at 1.76 GHz, where the card's power holds it).  One block = 2*RG waves
 // (dh, rg): wave rg takes NM = 2 fragments of 32 rows, wave dh half of the P
 // degrees, for one input block (32 inputs); acc = NM x P/2 fragments, two
 // waves per SIMD.  RG = 4
@@ -1353,33 +1422,34 @@ k_dx_pipe(const typename Elem<BF>::type* __restrict__ dYx,
 // pair exchanges halves through LDS, and each wave stores one fragment row of
 // dx = (1 - t^2) sum_d d C U_{d-1}(t) dy.
 // ---------------------------------------------------------------------------
-template <int P, bool BF>
+template <int P, int M>
 struct DxDh {
-  typedef typename Elem<BF>::type E;
+  typedef typename Elem<M>::type E;
   static constexpr int RG = 4;  // row groups: 2 * RG waves
   static constexpr int NM = P == 16 ? 1 : 2, PH = P / 2, THR = 2 * RG * 64;
-  static constexpr int FB = kFragElems * (int)sizeof(E);
-  static constexpr int KI = BF ? 2 : 1;
+  static constexpr int FB = kFragLen<M> * (int)sizeof(E);
+  // k-blocks per stage: 3072 clk of products per SIMD in split mode, 1024 in bf16
+  static constexpr int KI = M == kSplit && P > 4 ? 1 : 2;
   static constexpr int A_BYTES = RG * NM * KI * FB;
   static constexpr int B_BYTES = P * KI * FB;
   static constexpr int STAGE_BYTES = A_BYTES + B_BYTES;
-  static constexpr int NBUF = 3;
+  static constexpr int NBUF = 3 * STAGE_BYTES <= 160 * 1024 ? 3 : 2;
   static constexpr int LDS_BYTES = NBUF * STAGE_BYTES;
-  static constexpr int OPS = STAGE_BYTES / (THR * 16);  // dma16 per thread per stage
-  static constexpr int A_OPS = A_BYTES / (THR * 16);
+  // dma16 per thread of a 256-thread half, were it to copy the whole stage
+  static constexpr int HOPS = STAGE_BYTES / 4096, HA_OPS = A_BYTES / 4096;
   static constexpr bool kOk = P >= 2 && LDS_BYTES <= 160 * 1024 &&
-                              A_BYTES % (THR * 16) == 0 && B_BYTES % (THR * 16) == 0 &&
+                              A_BYTES % 4096 == 0 && B_BYTES % 4096 == 0 &&
                               2 * RG * 16 * 64 * 4 <= LDS_BYTES;
 };
 
-template <int P, bool BF>
+template <int P, int M>
 __global__ void __launch_bounds__(512)
-k_dx_dh(const typename Elem<BF>::type* __restrict__ dYx,
-         const typename Elem<BF>::type* __restrict__ Cb, const float* __restrict__ tc,
+k_dx_dh(const typename Elem<M>::type* __restrict__ dYx,
+         const typename Elem<M>::type* __restrict__ Cb, const float* __restrict__ tc,
          float* __restrict__ dx, Plan p, int n_rb) {
-  typedef DxDh<P, BF> K;
+  typedef DxDh<P, M> K;
   typedef typename K::E E;
-  constexpr int NM = K::NM, PH = K::PH, KI = K::KI, FB = K::FB, NBUF = K::NBUF, OPS = K::OPS;
+  constexpr int NM = K::NM, PH = K::PH, KI = K::KI, FB = K::FB, NBUF = K::NBUF;
   constexpr int RUN = KI * FB / 16;  // 16-byte chunks per fragment run of a stage
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
@@ -1397,7 +1467,7 @@ k_dx_dh(const typename Elem<BF>::type* __restrict__ dYx,
   // whole row blocks.
   constexpr int RG = K::RG, THR = K::THR;
   static_assert(THR == 512, "launch bounds");
-  constexpr int HOPS = 2 * OPS, HA_OPS = 2 * K::A_OPS;
+  constexpr int HOPS = K::HOPS, HA_OPS = K::HA_OPS;
   constexpr int H0 = HOPS / 2, H1 = HOPS - H0;  // copies per thread of waves 0-3 / 4-7
   const char* abase = reinterpret_cast<const char*>(dYx) + (size_t)rb * RG * NM * p.KBx * FB;
   const char* bbase = reinterpret_cast<const char*>(Cb) + (size_t)ib * P * p.KBx * FB;
@@ -1467,28 +1537,61 @@ k_dx_dh(const typename Elem<BF>::type* __restrict__ dYx,
     else wait_vmcnt<H0 * (NBUF - 2)>();
     block_barrier();
     const char* base = smem + (st % NBUF) * K::STAGE_BYTES;
-    // all reads first, in k-block order; the MFMAs of k-block kk wait only for
-    // its own reads (LDS returns in order)
-    Frag<BF> fa[KI][NM], fb[KI][PH];
+    auto frag_a = [&](int kk, int mi) __attribute__((always_inline)) {
+      return load_frag<M>(reinterpret_cast<const E*>(base + ((rg * NM + mi) * KI + kk) * FB), lane);
+    };
+    auto frag_b = [&](int kk, int e) __attribute__((always_inline)) {
+      return load_frag<M>(reinterpret_cast<const E*>(base + K::A_BYTES + ((dh * PH + e) * KI + kk) * FB), lane);
+    };
+    if constexpr (M == kSplit) {
+      // one degree's (NM = 1: two degrees') planes ahead of the products
+      constexpr int EB = NM == 1 ? 2 : 1;
 #pragma unroll
-    for (int kk = 0; kk < KI; ++kk) {
+      for (int kk = 0; kk < KI; ++kk) {
+        Frag<M> fa[NM], fb[2][EB];
 #pragma unroll
-      for (int mi = 0; mi < NM; ++mi)
-        fa[kk][mi] = load_frag<BF>(reinterpret_cast<const E*>(base + ((rg * NM + mi) * KI + kk) * FB), lane);
+        for (int mi = 0; mi < NM; ++mi) fa[mi] = frag_a(kk, mi);
 #pragma unroll
-      for (int e = 0; e < PH; ++e)
-        fb[kk][e] = load_frag<BF>(reinterpret_cast<const E*>(base + K::A_BYTES + ((dh * PH + e) * KI + kk) * FB), lane);
+        for (int j = 0; j < EB; ++j) fb[0][j] = frag_b(kk, j);
+        __builtin_amdgcn_sched_barrier(0);
+        if (kk == 0 && hw) issue(st + NBUF - 1);
+#pragma unroll
+        for (int e = 0; e < PH; e += EB) {
+          const int cur = (e / EB) & 1;
+          if (e + EB < PH) {
+#pragma unroll
+            for (int j = 0; j < EB; ++j) fb[cur ^ 1][j] = frag_b(kk, e + EB + j);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (NM == 2) mma2(acc[0][e], fa[0], fb[cur][0], acc[1][e], fa[1], fb[cur][0]);
+          else mma2(acc[0][e], fa[0], fb[cur][0], acc[0][e + 1], fa[0], fb[cur][EB - 1]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    } else {
+      // all reads first, in k-block order; the MFMAs of k-block kk wait only for
+      // its own reads (LDS returns in order)
+      Frag<M> fa[KI][NM], fb[KI][PH];
+#pragma unroll
+      for (int kk = 0; kk < KI; ++kk) {
+#pragma unroll
+        for (int mi = 0; mi < NM; ++mi)
+          fa[kk][mi] = frag_a(kk, mi);
+#pragma unroll
+        for (int e = 0; e < PH; ++e)
+          fb[kk][e] = frag_b(kk, e);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (hw) issue(st + NBUF - 1);
       __builtin_amdgcn_sched_barrier(0);
-    }
-    if (hw) issue(st + NBUF - 1);
-    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int kk = 0; kk < KI; ++kk) {
+      for (int kk = 0; kk < KI; ++kk) {
 #pragma unroll
-      for (int mi = 0; mi < NM; ++mi)
+        for (int mi = 0; mi < NM; ++mi)
 #pragma unroll
-        for (int e = 0; e < PH; ++e) mma(acc[mi][e], fa[kk][mi], fb[kk][e]);
-      __builtin_amdgcn_sched_barrier(0);
+          for (int e = 0; e < PH; ++e) mma(acc[mi][e], fa[kk][mi], fb[kk][e]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
     if (!hw) issue(st + NBUF - 1);
   }
@@ -2070,124 +2173,6 @@ k_dx16(const uint16_t* __restrict__ dYx, const uint16_t* __restrict__ Cb,
 }
 
 // ---------------------------------------------------------------------------
-// dX: one block = 4 waves along rows x one input block (32 inputs x P degrees).
-// B fragments (coefficients, all P degrees of the input block) are shared
-// through LDS; A fragments (dy) are per-wave global loads, prefetched a stage
-// ahead.  Epilogue: per (row, input), sum over degrees with d U_{d-1}(t) and
-// the tanh chain factor, all in registers.
-// ---------------------------------------------------------------------------
-template <int P, bool BF, int NM, int KI>
-__global__ void __launch_bounds__(256)
-k_dx(const typename Elem<BF>::type* __restrict__ dYx, const typename Elem<BF>::type* __restrict__ Cb,
-     const float* __restrict__ tc, float* __restrict__ dx, Plan p) {
-  typedef typename Elem<BF>::type E;
-  constexpr int WGM = 4;
-  constexpr int STAGE = P * KI * kFragElems;
-  constexpr int CE = 16 / (int)sizeof(E);
-  constexpr int NCHUNK = STAGE / CE;
-  constexpr int CPT = NCHUNK / 256;
-  constexpr int CPE = KI * kFragElems / CE;  // chunks per degree
-  static_assert(NCHUNK % 256 == 0, "stage must split evenly over 256 threads");
-  __shared__ __attribute__((aligned(16))) E lds[2 * STAGE];
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int g = lane >> 5;
-  const int ib = blockIdx.y;
-  const int64_t mf0 = (int64_t)blockIdx.x * WGM * NM + wave * NM;  // first 32-row fragment
-  const int64_t nmf = p.B32 / 32;
-  const int nst = p.KBx / KI;
-
-  u32x4_t pre[CPT];
-  auto gload = [&](int st) __attribute__((always_inline)) {
-#pragma unroll
-    for (int q = 0; q < CPT; ++q) {
-      const int c = tid + q * 256;
-      const int e = c / CPE, off = c - e * CPE;
-      pre[q] = *reinterpret_cast<const u32x4_t*>(
-          Cb + ((size_t)(ib * P + e) * p.KBx + (size_t)st * KI) * kFragElems + (size_t)off * CE);
-    }
-  };
-  auto lstore = [&](int buf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int q = 0; q < CPT; ++q)
-      *reinterpret_cast<u32x4_t*>(lds + buf * STAGE + (tid + q * 256) * CE) = pre[q];
-  };
-  Frag<BF> apre[NM][KI];
-  auto aload = [&](int st) __attribute__((always_inline)) {
-#pragma unroll
-    for (int mi = 0; mi < NM; ++mi)
-#pragma unroll
-      for (int k = 0; k < KI; ++k) {
-        const int64_t mf = mf0 + mi;
-        apre[mi][k] = (mf < nmf)
-            ? load_frag<BF>(dYx + ((size_t)mf * p.KBx + (size_t)st * KI + k) * kFragElems, lane)
-            : zero_frag<BF>();
-      }
-  };
-
-  f32x16_t acc[NM][P];
-#pragma unroll
-  for (int mi = 0; mi < NM; ++mi)
-#pragma unroll
-    for (int e = 0; e < P; ++e)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[mi][e][v] = 0.0f;
-
-  gload(0);
-  lstore(0);
-  aload(0);
-  __syncthreads();
-
-  for (int st = 0; st < nst; ++st) {
-    const int buf = st & 1;
-    const bool more = st + 1 < nst;
-    Frag<BF> a[NM][KI];
-#pragma unroll
-    for (int mi = 0; mi < NM; ++mi)
-#pragma unroll
-      for (int k = 0; k < KI; ++k) a[mi][k] = apre[mi][k];
-    if (more) {
-      gload(st + 1);
-      aload(st + 1);
-    }
-    const E* sb = lds + buf * STAGE;
-#pragma unroll
-    for (int k = 0; k < KI; ++k) {
-#pragma unroll
-      for (int e = 0; e < P; ++e) {
-        const Frag<BF> bfr = load_frag<BF>(sb + (e * KI + k) * kFragElems, lane);
-#pragma unroll
-        for (int mi = 0; mi < NM; ++mi) mma(acc[mi][e], a[mi][k], bfr);
-      }
-    }
-    if (more) lstore(buf ^ 1);
-    __syncthreads();
-  }
-
-  const int i = ib * 32 + (lane & 31);
-#pragma unroll
-  for (int mi = 0; mi < NM; ++mi) {
-    const int64_t r0 = (mf0 + mi) * 32;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int64_t r = r0 + acc_row(v, g);
-      const bool ok = r < p.B && i < p.I;
-      const float tv = ok ? tc[r * p.I_sg + i] : 0.0f;
-      const float t2 = tv + tv;
-      float up = 0.0f, u = 1.0f, s = 0.0f;  // U_{-1}, U_0
-#pragma unroll
-      for (int e = 0; e < P; ++e) {
-        s = fmaf(acc[mi][e][v], u, s);
-        const float un = fmaf(t2, u, -up);
-        up = u;
-        u = un;
-      }
-      if (ok) __builtin_nontemporal_store(s * input_slope(tv, p), dx + r * p.I + i);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
 // dC: one block = 4 waves along outputs x one input block (32 inputs x P
 // degrees) x one batch split.  The basis operand (rows = inputs, one fragment
 // per degree) is generated by the block into LDS once per stage of KI
@@ -2325,41 +2310,52 @@ k_dc(const typename Elem<BF>::type* __restrict__ dYc, const float* __restrict__ 
 // One block = 8 waves in H groups ("halves") that take alternate stages of KI
 // k-blocks (16 batch rows each) of the reduction; in a group, wave (dq, og)
 // accumulates PH = min(P, 4) degrees (group dq) x NN output fragments (group
-// og) for the block's 32 inputs, always 8 accumulator fragments.  H = 2 (a
+// og) for the block's 32 inputs, 8 accumulator fragments (4 with NN_ = 1,
+// the split tile for outputs that the wide one would pad).  H = 2 (a
 // K split inside the block), or H = 1 for degree 16 with at least 4 output
 // fragments: 4 output fragments per block keep basis generation at 3 VALU
 // per MFMA.
 // Both streamed operands arrive by LDS DMA, with no vector-register loads in
 // the loop: tanh tiles three pairs of stages ahead, dy fragments two pairs
-// ahead.  The basis operand (P fragments per k-block) is generated from the
+// ahead (split fp32: two and one).  Split fp32 at 8192 x 1024 -> 1024, degree
+// 8: 1046 us on the fp32 instructions -> 610-640 us (MFMA busy 66 % at 1.86
+// GHz; reading dy's planes first changed neither).  Degrees 9-16 and the odd
+// widths ran an unpipelined kernel or padded tiles before: 3000 x 500 -> 300,
+// degree 5: 142 -> 77 us.  The basis operand (P fragments per k-block) is generated from the
 // tanh tile into LDS one pair ahead, interleaved with the MFMAs.  The halves'
 // tiles are summed through LDS, then each output group is staged as
 // [input][output][degree] (d = 0 from the reduced dy column sums) so that the
 // block writes contiguous runs of dC, or of its split-K slice.
 // ---------------------------------------------------------------------------
-template <int P, bool BF, int H_>
+template <int P, int M, int H_, int NN_ = 0>
 struct DcPipe {
-  typedef typename Elem<BF>::type E;
+  typedef typename Elem<M>::type E;
+  static constexpr int PP = P, MM = M, NNA = NN_;
   static constexpr int H = H_;              // stage groups (K split inside the block)
   static constexpr int WG = 8 / H;          // waves per group
   static constexpr int PH = P < 4 ? P : 4;  // degrees per wave
   static constexpr int DQ = P / PH;         // degree groups in a group
   static constexpr int OG = WG / DQ;        // output groups in a group
-  static constexpr int NN = 8 / PH;         // output fragments per wave
+  static constexpr int NN = NN_ ? NN_ : 8 / PH;  // output fragments per wave
   static constexpr int NO = OG * NN;        // output fragments per block
-  static constexpr int NF = PH * NN;        // accumulator fragments per wave (8)
-  static constexpr int KI = (BF && P != 2 && (P != 16 || H == 1)) ? 2 : 1;
-  static constexpr int FB = kFragElems * (int)sizeof(E);
+  static constexpr int NF = PH * NN;        // accumulator fragments per wave (8; 4 with NN_ = 1)
+  static constexpr int KI = (M == kBf16 && P != 2 && (P != 16 || H == 1)) ? 2 : 1;
+  static constexpr int FE = kFragLen<M>;    // elements of a fragment
+  static constexpr int FB = FE * (int)sizeof(E);
+  // Ring slots of dy and tanh tiles.  Split operands fill the LDS with two;
+  // each step's copies are then issued at its start (a step has three times
+  // the products to hide them) instead of after its MFMAs.
+  static constexpr int RING = M == kSplit ? 2 : 3;
   static constexpr int BAS_STAGE = P * KI * FB;
   static constexpr int DY_STAGE = NO * KI * FB;
   static constexpr int DY_CHUNKS = H * DY_STAGE / 16;             // real chunks per step
   static constexpr int DY_OPS = (DY_CHUNKS + 511) / 512;          // dma16 per thread per step
-  static constexpr int DY_SLOT = DY_OPS * 8192;                   // bytes per step slot
+  static constexpr int DY_SLOT = M == kSplit ? (DY_CHUNKS + 255) / 256 * 4096 : DY_OPS * 8192;  // bytes per step slot
   static constexpr int T_STAGE = KI * 16 * 32 * 4;                // tanh rows x 32 inputs
   static constexpr int T_CHUNKS = H * T_STAGE / 16;
-  static constexpr int T_SLOT = 8192;                             // one dma16 per thread
+  static constexpr int T_SLOT = M == kSplit ? 4096 : 8192;        // whole dma16 rounds of 256 or 512 threads
   static constexpr int BAS_BYTES = 2 * H * BAS_STAGE;             // two steps of H stages
-  static constexpr int MAIN_BYTES = BAS_BYTES + 3 * DY_SLOT + 3 * T_SLOT;
+  static constexpr int MAIN_BYTES = BAS_BYTES + RING * (DY_SLOT + T_SLOT);
   static constexpr int XCH_BYTES = H == 2 ? 8 * (NF / 2) * 16 * 64 * 4 : 0;
   static constexpr int STG_BYTES = 32 * NN * 32 * (P + 1) * 4;  // one output group
   static constexpr int BIG_BYTES = MAIN_BYTES > XCH_BYTES
@@ -2377,18 +2373,18 @@ template <bool XF> struct DcXf { BasisXform x; };
 template <> struct DcXf<false> {};
 // LDS for M's rows n <= P, after the pipelined dC's own
 template <int P> constexpr int kDcXfBytes = (P + 1) * kMaxD * (int)sizeof(float);
-template <int P, bool BF, int H>
-constexpr bool dc_xf_fits() { return DcPipe<P, BF, H>::kOk && DcPipe<P, BF, H>::LDS_BYTES + kDcXfBytes<P> <= 160 * 1024; }
+template <int P, int M, int H, int NN = 0>
+constexpr bool dc_xf_fits() { return DcPipe<P, M, H, NN>::kOk && DcPipe<P, M, H, NN>::LDS_BYTES + kDcXfBytes<P> <= 160 * 1024; }
 
-template <int P, bool BF, int H_, bool XF = false>
+template <int P, int M, int H_, bool XF = false, int NN_ = 0>
 __global__ void __launch_bounds__(512)
-k_dc_pipe(const typename Elem<BF>::type* __restrict__ dYc, const float* __restrict__ tc,
+k_dc_pipe(const typename Elem<M>::type* __restrict__ dYc, const float* __restrict__ tc,
           const float* __restrict__ colsum_part, float* __restrict__ out, Plan p, int st_per_split,
           DcOut om, DcXf<XF> xf) {
-  typedef DcPipe<P, BF, H_> K;
+  typedef DcPipe<P, M, H_, NN_> K;
   typedef typename K::E E;
   constexpr int PH = K::PH, DQ = K::DQ, OG = K::OG, NN = K::NN, NO = K::NO, NF = K::NF;
-  constexpr int KI = K::KI, FB = K::FB, H = K::H, WG = K::WG;
+  constexpr int KI = K::KI, FB = K::FB, FE = K::FE, H = K::H, WG = K::WG, RING = K::RING;
   constexpr int RPT = K::RPT, DY_OPS = K::DY_OPS;
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
@@ -2410,7 +2406,7 @@ k_dc_pipe(const typename Elem<BF>::type* __restrict__ dYc, const float* __restri
   const int npair = (st1 - st0) / H;  // steps of H stages (split stage counts are even)
   char* bas = smem;
   char* dyr = smem + K::BAS_BYTES;
-  char* tlr = dyr + 3 * K::DY_SLOT;
+  char* tlr = dyr + RING * K::DY_SLOT;
 
   // DMA: waves 0-3 issue every copy of a step (the H stages of one pair step),
   // DH_OPS dy and TH_OPS tanh copies per thread, after their MFMAs of the
@@ -2425,16 +2421,22 @@ k_dc_pipe(const typename Elem<BF>::type* __restrict__ dYc, const float* __restri
   // dy: chunk c < DY_CHUNKS of a step is [stage hs][fragment f][k-block kk][16 B];
   // chunks past that repeat real ones into the unused end of the slot
   const char* dyb = reinterpret_cast<const char*>(dYc) + (size_t)obk * NO * p.KBc * FB;
+  // split: a wave's 64 chunks are one plane of one fragment (192 chunks), so
+  // the fragment's offset is a scalar and only the chunk's is per lane
   uint32_t doff[DH_OPS];
+  size_t dsb[DH_OPS];
+  const int w4 = __builtin_amdgcn_readfirstlane(wave & 3);
 #pragma unroll
   for (int q = 0; q < DH_OPS; ++q) {
-    const int c = (q * 256 + t256) % K::DY_CHUNKS;
+    const int c = M == kSplit ? (q * 256 + w4 * 64) % K::DY_CHUNKS : (q * 256 + t256) % K::DY_CHUNKS;
     const int hs = c / (NO * KI * CPF), r1 = c - hs * (NO * KI * CPF);
     const int f = r1 / (KI * CPF), r2 = r1 - f * (KI * CPF);
     const int kk = r2 / CPF, piece = r2 - kk * CPF;
     const int mf = min(obk * NO + f, p.NBf - 1);
-    doff[q] = (uint32_t)(((size_t)(mf - obk * NO) * p.KBc + kk) * FB + (size_t)piece * 16 +
-                         (size_t)hs * KI * FB);
+    const size_t off = ((size_t)(mf - obk * NO) * p.KBc + kk) * FB + (size_t)piece * 16 +
+                       (size_t)hs * KI * FB;
+    dsb[q] = M == kSplit ? off : 0;
+    doff[q] = M == kSplit ? lane * 16 : (uint32_t)off;
   }
   // tanh tile of a stage: rows of 32 fp32 inputs.  Row rho is stored at row
   // t_row(rho) with its 16-byte chunks XOR-ed by t_xor(rho) / 4, so that the
@@ -2467,14 +2469,18 @@ k_dc_pipe(const typename Elem<BF>::type* __restrict__ dYc, const float* __restri
     int st = st0 + H * j;
     if (st + H > st1) st = st0;  // past the end: any in-range source, never read
     const char* sb = dyb + (size_t)st * KI * FB;
-    const uint32_t l = dyl0 + (j % 3) * K::DY_SLOT;
+    const uint32_t l = dyl0 + (j % RING) * K::DY_SLOT;
 #pragma unroll
-    for (int q = 0; q < DH_OPS; ++q) dma16s_salu(sb, doff[q], l + q * 4096);
+    for (int q = 0; q < DH_OPS; ++q) {
+      // the split bases may be held in vector registers: the guarded copy
+      if constexpr (M == kSplit) dma16s(sb + dsb[q], doff[q], l + q * 4096);
+      else dma16s_salu(sb, doff[q], l + q * 4096);
+    }
   };
   auto dma_t = [&](int j) __attribute__((always_inline)) {
     int st = st0 + H * j;
     if (st + H > st1) st = st0;
-    const uint32_t l = tll0 + (j % 3) * K::T_SLOT;
+    const uint32_t l = tll0 + (j % RING) * K::T_SLOT;
 #pragma unroll
     for (int q = 0; q < TH_OPS; ++q) {
       const int64_t row0 = (int64_t)(st + tst[q]) * SROWS;
@@ -2500,7 +2506,7 @@ k_dc_pipe(const typename Elem<BF>::type* __restrict__ dYc, const float* __restri
   // the generation's tanh reads, issued apart so that they can go ahead of
   // the step's fragment reads (LDS returns in order)
   auto gen_read = [&](int j, float (&tv)[RPT]) __attribute__((always_inline)) {
-    const float* tl = reinterpret_cast<const float*>(tlr + (j % 3) * K::T_SLOT + half * K::T_STAGE);
+    const float* tl = reinterpret_cast<const float*>(tlr + (j % RING) * K::T_SLOT + half * K::T_STAGE);
 #pragma unroll
     for (int r = 0; r < RPT; ++r) tv[r] = tl[t_row(trow0 + r) * 32 + ((gl & 31) ^ t_xor(trow0 + r))];
   };
@@ -2520,7 +2526,24 @@ k_dc_pipe(const typename Elem<BF>::type* __restrict__ dYc, const float* __restri
         }
       }
       char* d = dst + e * KI * FB;
-      if constexpr (BF) {
+      if constexpr (M == kSplit) {
+        // the planes of this thread's RPT rows
+        __bf16 w[3][RPT];
+#pragma unroll
+        for (int r = 0; r < RPT; ++r) {
+          const __bf16 h = (__bf16)b[r];
+          const float rm = b[r] - (float)h;
+          const __bf16 m = (__bf16)rm;
+          w[0][r] = h;
+          w[1][r] = m;
+          w[2][r] = (__bf16)(rm - (float)m);
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          if constexpr (RPT == 2) *reinterpret_cast<bf16x2_t*>(d + k * kFragElems * 2) = bf16x2_t{w[k][0], w[k][1]};
+          else *reinterpret_cast<__bf16*>(d + k * kFragElems * 2) = w[k][0];
+        }
+      } else if constexpr (M == kBf16) {
         if constexpr (RPT == 4) {
           bf16x4_t w;
 #pragma unroll
@@ -2549,35 +2572,51 @@ k_dc_pipe(const typename Elem<BF>::type* __restrict__ dYc, const float* __restri
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[e][ni][v] = 0.0f;
 
+  // the narrow split tile has registers for the small plane products' own sums
+  static_assert(NN > 1 || M == kSplit, "one output fragment per wave only in split mode");
+  f32x16_t lo[NN == 1 ? PH : 1];
+#pragma unroll
+  for (int e = 0; e < (NN == 1 ? PH : 1); ++e)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) lo[e][v] = 0.0f;
+
   // One pair step of this wave: the fragments of all KI k-blocks of its stage
   // are read from LDS up front, and the basis generation for the next pair
   // (VALU + LDS traffic) is interleaved with the MFMAs.
   auto step = [&](int j) __attribute__((always_inline)) {
     const E* ab = reinterpret_cast<const E*>(bas + ((j & 1) * H + half) * K::BAS_STAGE) +
-                  (size_t)(dh * PH) * KI * kFragElems;
-    const E* bb = reinterpret_cast<const E*>(dyr + (j % 3) * K::DY_SLOT + half * K::DY_STAGE) +
-                  (size_t)(og * NN) * KI * kFragElems;
+                  (size_t)(dh * PH) * KI * FE;
+    const E* bb = reinterpret_cast<const E*>(dyr + (j % RING) * K::DY_SLOT + half * K::DY_STAGE) +
+                  (size_t)(og * NN) * KI * FE;
     float tv[RPT];
     gen_read(j + 1, tv);
     __builtin_amdgcn_sched_barrier(0);
-    Frag<BF> fa[KI][PH], fb[KI][NN];
+    Frag<M> fa[KI][PH], fb[KI][NN];
 #pragma unroll
     for (int kk = 0; kk < KI; ++kk) {
 #pragma unroll
-      for (int e = 0; e < PH; ++e) fa[kk][e] = load_frag<BF>(ab + (e * KI + kk) * kFragElems, lane);
+      for (int e = 0; e < PH; ++e) fa[kk][e] = load_frag<M>(ab + (e * KI + kk) * FE, lane);
 #pragma unroll
-      for (int ni = 0; ni < NN; ++ni) fb[kk][ni] = load_frag<BF>(bb + (ni * KI + kk) * kFragElems, lane);
+      for (int ni = 0; ni < NN; ++ni) fb[kk][ni] = load_frag<M>(bb + (ni * KI + kk) * FE, lane);
       __builtin_amdgcn_sched_barrier(0);  // k-block order of the reads (LDS returns in order)
     }
     gen_write(j + 1, tv);
 #pragma unroll
     for (int kk = 0; kk < KI; ++kk)
 #pragma unroll
-      for (int e = 0; e < PH; ++e)
+      for (int e = 0; e < PH; e += NN == 1 ? 2 : 1) {
+        if constexpr (NN == 1) {
+          mma_apart(acc[e][0], lo[e], fa[kk][e], fb[kk][0], acc[e + 1][0], lo[e + 1], fa[kk][e + 1],
+                    fb[kk][0]);
+        } else {
 #pragma unroll
-        for (int ni = 0; ni < NN; ++ni) mma(acc[e][ni], fa[kk][e], fb[kk][ni]);
+          for (int ni = 0; ni < NN; ni += 2)
+            mma2(acc[e][ni], fa[kk][e], fb[kk][ni], acc[e][ni + 1], fa[kk][e], fb[kk][ni + 1]);
+        }
+      }
+    constexpr int PR = M == kSplit ? kSplitProducts : 1;
 #pragma unroll
-    for (int q = 0; q < KI * PH * NN; ++q) {
+    for (int q = 0; q < KI * PH * NN * PR; ++q) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
       __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // up to four VALU
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // up to one LDS read
@@ -2594,33 +2633,66 @@ k_dc_pipe(const typename Elem<BF>::type* __restrict__ dYc, const float* __restri
   const bool copier = wave < 4;
   pin_sgpr(colsum_part);  // used after the loop
   pin_sgpr(out);
-  if (copier) {
-    dma_t(0);
-    dma_t(1);
-    dma_dy(0);
-    dma_t(2);
-    dma_dy(1);
-    wait_vmcnt<2 * HOPS>();  // t(0) landed
-  }
-  block_barrier();
-  {
-    float tv0[RPT];
-    gen_read(0, tv0);
-    gen_write(0, tv0);
-  }
-  for (int j = 0; j < npair; ++j) {
-    // dy(j) and t(j+1) have landed once only the copies of the last issue
-    // (t(j+2), dy(j+1)) may be in flight
-    if (copier) wait_vmcnt<HOPS>();
-    wait_lgkmcnt<0>();  // this thread's basis writes for pair j are done
-    block_barrier();
-    step(j);  // also generates pair j+1 (unused after the last pair)
+  if constexpr (RING == 2) {
+    // two slots: step j's start frees the slots that step j - 1 read (dy(j - 1),
+    // t(j)), so t(j + 2) and dy(j + 1) are issued there and waited for at its end
     if (copier) {
-      dma_t(j + 3);
-      dma_dy(j + 2);
+      dma_t(0);
+      dma_t(1);
+      dma_dy(0);
+      wait_vmcnt<HOPS>();  // t(0) landed
+    }
+    block_barrier();
+    {
+      float tv0[RPT];
+      gen_read(0, tv0);
+      gen_write(0, tv0);
+    }
+    for (int j = 0; j < npair; ++j) {
+      if (copier) wait_vmcnt<0>();
+      wait_lgkmcnt<0>();  // this thread's basis writes for pair j are done
+      block_barrier();
+      if (copier) {
+        dma_t(j + 2);
+        dma_dy(j + 1);
+      }
+      step(j);  // also generates pair j+1 (unused after the last pair)
+    }
+  } else {
+    if (copier) {
+      dma_t(0);
+      dma_t(1);
+      dma_dy(0);
+      dma_t(2);
+      dma_dy(1);
+      wait_vmcnt<2 * HOPS>();  // t(0) landed
+    }
+    block_barrier();
+    {
+      float tv0[RPT];
+      gen_read(0, tv0);
+      gen_write(0, tv0);
+    }
+    for (int j = 0; j < npair; ++j) {
+      // dy(j) and t(j+1) have landed once only the copies of the last issue
+      // (t(j+2), dy(j+1)) may be in flight
+      if (copier) wait_vmcnt<HOPS>();
+      wait_lgkmcnt<0>();  // this thread's basis writes for pair j are done
+      block_barrier();
+      step(j);  // also generates pair j+1 (unused after the last pair)
+      if (copier) {
+        dma_t(j + 3);
+        dma_dy(j + 2);
+      }
     }
   }
   wait_vmcnt<0>();  // the prefetches past the end land before the LDS is reused
+  if constexpr (NN == 1) {
+#pragma unroll
+    for (int e = 0; e < PH; ++e)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[e][0][v] += lo[e][v];
+  }
 
   // d = 0 column, sum_b dy[b, o]: thread (rgp, oi) adds every RS-th of the
   // NBB per-64-row partials of output oi (fixed order); the RS results are
@@ -2922,7 +2994,33 @@ static void fwd_dispatch(const float* x, float* t, const void* packed, float* y,
                              p, c.sg_per_split, bpart, nib_k, bias_out, nullptr);
         break;
       default:
-        if constexpr (FwdPipe<P, BF>::kOk) {
+        if constexpr (!BF && P >= kSplitMinP) {
+          if (!fwd_pipe_offsets_fit(p)) {  // per-lane copy offsets are 32-bit
+            hipLaunchKernelGGL((k_fwd<P, BF, 2, 4, 4, 1>), grid, dim3(256), 0, s, t, Cf, bias, y,
+                               part, p, c.sg_per_split, bpart, nib_k, bias_out, nullptr);
+            break;
+          }
+          const uint16_t* cf3 = reinterpret_cast<const uint16_t*>(pk + packed_cf3_offset(p));
+          auto launch = [&](auto OTc, auto NNc, std::atomic<uint32_t>& flag) {
+            constexpr bool OTv = decltype(OTc)::value;
+            constexpr int NNv = decltype(NNc)::value;
+            typedef FwdSplit<P, NNv> KV;
+            ensure_lds_limit(reinterpret_cast<const void*>(&k_fwd_split<P, OTv, NNv>), KV::LDS_BYTES, flag);
+            hipLaunchKernelGGL((k_fwd_split<P, OTv, NNv>), grid, dim3(KV::THREADS),
+                               (size_t)KV::LDS_BYTES, s, t, cf3, bias, y, part, p, c.sg_per_split,
+                               bpart, nib_k, nib_k > 0 ? bias_out : nullptr);
+          };
+          typedef std::integral_constant<bool, true> OT1;
+          typedef std::integral_constant<bool, false> OT0;
+          static std::atomic<uint32_t> lds_split[4];
+          if (c.bnf == 2) {
+            if (out_tanh) launch(OT1{}, std::integral_constant<int, 2>{}, lds_split[0]);
+            else launch(OT0{}, std::integral_constant<int, 2>{}, lds_split[1]);
+          } else {
+            if (out_tanh) launch(OT1{}, std::integral_constant<int, 4>{}, lds_split[2]);
+            else launch(OT0{}, std::integral_constant<int, 4>{}, lds_split[3]);
+          }
+        } else if constexpr (FwdPipe<P, BF>::kOk) {
           if (!fwd_pipe_offsets_fit(p)) {  // per-lane copy offsets are 32-bit
             hipLaunchKernelGGL((k_fwd<P, BF, 2, 4, 4, 1>), grid, dim3(256), 0, s, t, Cf, bias, y,
                                part, p, c.sg_per_split, bpart, nib_k, bias_out, nullptr);
@@ -2969,7 +3067,7 @@ static void fwd_dispatch(const float* x, float* t, const void* packed, float* y,
 // stores y itself; a split forward's reduce stores every y.
 template <int P, bool BF> static bool out_tanh_ok(const Plan& p, const FwdChoice& c) {
   if (c.tile != kFwdCols && (c.splits > 1 || fwd_streaming(c))) return true;
-  if constexpr (FwdPipe<P, BF>::kOk)
+  if constexpr ((!BF && P >= kSplitMinP) || FwdPipe<P, BF>::kOk)
     return c.tile == kFwdBig && c.splits == 1 && fwd_pipe_offsets_fit(p);
   else
     return false;
@@ -3016,9 +3114,6 @@ void launch_fwd_gemm(const float* x, float* t, const void* packed, float* y, voi
 #undef CKAN_FW
 }
 
-// dX stage depth: 4 k-blocks for bf16; fp32 halves it to bound LDS.
-template <bool BF> struct DxKI { static constexpr int v = BF ? 4 : 2; };
-
 // k_dx16's limits: 32-bit per-lane offsets into the tanh cache and a tile
 // count that fits an int
 static bool dx16_ok(const Plan& p) {
@@ -3039,7 +3134,6 @@ template <int P, bool BF>
 static void dx_dispatch(const void* dYx, const void* packed, const float* t, float* dx,
                         const Plan& p, hipStream_t s) {
   typedef typename Elem<BF>::type E;
-  constexpr int NM = BwdTile<P>::NM;
   const E* Cb = reinterpret_cast<const E*>(packed) + packed_cf_elems(p);
   if constexpr (P == 16 && BF) {
     if (dx16_ok(p)) {
@@ -3066,29 +3160,18 @@ static void dx_dispatch(const void* dYx, const void* packed, const float* t, flo
       return;
     }
   }
-  if constexpr (DxDh<P, BF>::kOk) {
-    typedef DxDh<P, BF> K;
-    const int n_rb = (int)ceil_div(p.B32 / 32, K::RG * K::NM);
-    static std::atomic<uint32_t> lds_set{0};
-    ensure_lds_limit(reinterpret_cast<const void*>(&k_dx_dh<P, BF>), K::LDS_BYTES, lds_set);
-    hipLaunchKernelGGL((k_dx_dh<P, BF>), dim3(n_rb * p.NIB), dim3(K::THR), K::LDS_BYTES, s,
-                       reinterpret_cast<const E*>(dYx), Cb, t, dx, p, n_rb);
-    return;
-  }
-  if constexpr (DxPipe<P, BF>::kOk) {
-    typedef DxPipe<P, BF> K;
-    const int n_rb = (int)ceil_div(p.B32 / 32, K::WGM * NM);
-    const int blocks = n_rb * p.NIB;
-    const size_t lds = (size_t)K::NBUF * K::STAGE_BYTES;
-    static std::atomic<uint32_t> lds_set{0};
-    ensure_lds_limit(reinterpret_cast<const void*>(&k_dx_pipe<P, BF>), (int)lds, lds_set);
-    hipLaunchKernelGGL((k_dx_pipe<P, BF>), dim3(blocks), dim3(256), lds, s,
-                       reinterpret_cast<const E*>(dYx), Cb, t, dx, p, n_rb);
-    return;
-  }
-  dim3 grid((unsigned)ceil_div(p.B32 / 32, 4 * NM), p.NIB);
-  hipLaunchKernelGGL((k_dx<P, BF, NM, DxKI<BF>::v>), grid, dim3(256), 0, s,
-                     reinterpret_cast<const E*>(dYx), Cb, t, dx, p);
+  // the operand mode of the GEMMs: fp32 layers split above degree 2
+  constexpr int M = BF ? kBf16 : P >= kSplitMinP ? kSplit : kFp32;
+  typedef DxDh<P, M> K;
+  static_assert(K::kOk, "the dX kernel of every other shape");
+  typedef typename K::E ME;
+  const ME* cb = M == kSplit ? reinterpret_cast<const ME*>(reinterpret_cast<const char*>(packed) + packed_cb3_offset(p))
+                             : reinterpret_cast<const ME*>(Cb);
+  const int n_rb = (int)ceil_div(p.B32 / 32, K::RG * K::NM);
+  static std::atomic<uint32_t> lds_set{0};
+  ensure_lds_limit(reinterpret_cast<const void*>(&k_dx_dh<P, M>), K::LDS_BYTES, lds_set);
+  hipLaunchKernelGGL((k_dx_dh<P, M>), dim3(n_rb * p.NIB), dim3(K::THR), K::LDS_BYTES, s,
+                     reinterpret_cast<const ME*>(dYx), cb, t, dx, p, n_rb);
 }
 
 void launch_dx_gemm(const void* dYx, const void* packed, const float* t, float* dx,
@@ -3102,40 +3185,53 @@ void launch_dx_gemm(const void* dYx, const void* packed, const float* t, float* 
   }
 }
 
-// dC stage depth in k-blocks: 4 for bf16, 2 for fp32 (LDS bound).
+// dC stage depth in k-blocks of the unpipelined kernel: 4 for bf16, 2 for fp32
+// (LDS bound).
 template <bool BF> struct DcKI { static constexpr int v = BF ? 4 : 2; };
 
-// Stage groups of the pipelined dC kernel for this shape (see DcPipe).
-static int dc_h(const Plan& p) { return (p.P == 16 && p.NBf >= 4) ? 1 : 2; }
+// Stage groups of the pipelined dC kernel for this shape (see DcPipe): split
+// fp32 at degree 16 has LDS for one group only.
+static int dc_h(const Plan& p) { return (p.P == 16 && (p.split || p.NBf >= 4)) ? 1 : 2; }
 
-template <int P, bool BF> static bool dc_ok_t(int h) {
-  return h == 1 ? DcPipe<P, BF, 1>::kOk : DcPipe<P, BF, 2>::kOk;
+// Output fragments per wave: split layers take the tile (1 or 2 fragments per
+// wave) whose blocks cover fewer padded fragments, the wide one when equal
+// (half the basis generation per product).  Elsewhere the kernel's own.
+template <int P> static bool dc_narrow_t(const Plan& p) {
+  constexpr int H = P == 16 ? 1 : 2;
+  constexpr int W = DcPipe<P, kSplit, H>::NO, N = DcPipe<P, kSplit, H, 1>::NO;
+  return ceil_div(p.NBf, N) * N < ceil_div(p.NBf, W) * W;
+}
+static bool dc_narrow(const Plan& p) {
+  if (!p.split) return false;
+  return p.P == 4 ? dc_narrow_t<4>(p) : p.P == 8 ? dc_narrow_t<8>(p) : dc_narrow_t<16>(p);
+}
+
+// Calls f with the pipelined dC configuration of this shape as a type.
+template <typename F> static auto with_dc(const Plan& p, F f) {
+  const bool h1 = dc_h(p) == 1;
+  if (p.split) {
+    const bool n = dc_narrow(p);
+    switch (p.P) {
+      case 4: return n ? f(DcPipe<4, kSplit, 2, 1>()) : f(DcPipe<4, kSplit, 2>());
+      case 8: return n ? f(DcPipe<8, kSplit, 2, 1>()) : f(DcPipe<8, kSplit, 2>());
+      default: return n ? f(DcPipe<16, kSplit, 1, 1>()) : f(DcPipe<16, kSplit, 1>());
+    }
+  }
+  if (p.esz != 2) return f(DcPipe<2, kFp32, 2>());
+  switch (p.P) {
+    case 2: return f(DcPipe<2, kBf16, 2>());
+    case 4: return f(DcPipe<4, kBf16, 2>());
+    case 8: return f(DcPipe<8, kBf16, 2>());
+    default: return h1 ? f(DcPipe<16, kBf16, 1>()) : f(DcPipe<16, kBf16, 2>());
+  }
 }
 static bool dc_pipe_ok(const Plan& p) {
-  const bool bf = p.esz == 2;
-  const int h = dc_h(p);
-  switch (p.P) {
-    case 2: return bf ? dc_ok_t<2, true>(h) : dc_ok_t<2, false>(h);
-    case 4: return bf ? dc_ok_t<4, true>(h) : dc_ok_t<4, false>(h);
-    case 8: return bf ? dc_ok_t<8, true>(h) : dc_ok_t<8, false>(h);
-    default: return bf ? dc_ok_t<16, true>(h) : dc_ok_t<16, false>(h);
-  }
+  return with_dc(p, [](auto k) { return decltype(k)::kOk; });
 }
-
 // output fragments per dC block and k-blocks per stage of the pipelined kernel
-template <int P, bool BF> static void dc_shape_t(int h, int& no, int& ki) {
-  no = h == 1 ? DcPipe<P, BF, 1>::NO : DcPipe<P, BF, 2>::NO;
-  ki = h == 1 ? DcPipe<P, BF, 1>::KI : DcPipe<P, BF, 2>::KI;
-}
 static void dc_pipe_shape(const Plan& p, int& no, int& ki) {
-  const bool bf = p.esz == 2;
-  const int h = dc_h(p);
-  switch (p.P) {
-    case 2: bf ? dc_shape_t<2, true>(h, no, ki) : dc_shape_t<2, false>(h, no, ki); break;
-    case 4: bf ? dc_shape_t<4, true>(h, no, ki) : dc_shape_t<4, false>(h, no, ki); break;
-    case 8: bf ? dc_shape_t<8, true>(h, no, ki) : dc_shape_t<8, false>(h, no, ki); break;
-    default: bf ? dc_shape_t<16, true>(h, no, ki) : dc_shape_t<16, false>(h, no, ki); break;
-  }
+  no = with_dc(p, [](auto k) { return (int)decltype(k)::NO; });
+  ki = with_dc(p, [](auto k) { return (int)decltype(k)::KI; });
 }
 
 BwdLayout bwd_layout(const Plan& p, bool need_dx_arg, bool need_dc_arg) {
@@ -3146,9 +3242,9 @@ BwdLayout bwd_layout(const Plan& p, bool need_dx_arg, bool need_dc_arg) {
   const bool need_dc = need_dc_arg && !L.dc_small, need_dx = need_dx_arg && !L.dx_small;
   size_t off = 0;
   L.dyx_off = off;
-  if (need_dx) off += align256((size_t)dx_row_frags(p) * p.KBx * kFragElems * p.esz);
+  if (need_dx) off += align256((size_t)dx_row_frags(p) * p.KBx * kFragElems * p.bsz);
   L.dyc_off = off;
-  if (need_dc) off += align256((size_t)p.NBf * p.KBc * kFragElems * p.esz);
+  if (need_dc) off += align256((size_t)p.NBf * p.KBc * kFragElems * p.bsz);
   L.colsum_off = off;  // NBB partial rows + the reduced row
   if (need_dc) off += align256((size_t)(p.NBB + 1) * p.O32 * sizeof(float));
   L.part_off = off;
@@ -3190,83 +3286,60 @@ BwdLayout bwd_layout(const Plan& p, bool need_dx_arg, bool need_dc_arg) {
   return L;
 }
 
-template <int P, bool BF, int H>
-static bool dc_pipe_launch(const void* dYc, const float* t, const float* colsum, float* part,
+template <typename K>
+static void dc_pipe_launch(const void* dYc, const float* t, const float* colsum, float* part,
                            float* dC, DcOut om, const Plan& p, const BwdLayout& L,
                            hipStream_t s, const BasisXform* xf) {
-  typedef typename Elem<BF>::type E;
-  if constexpr (DcPipe<P, BF, H>::kOk) {
-    typedef DcPipe<P, BF, H> K;
-    const bool split = L.dc_splits > 1;
-    dim3 grid(p.NIB, (unsigned)ceil_div(p.NBf, K::NO), L.dc_splits);
-    if constexpr (dc_xf_fits<P, BF, H>()) {
-      if (xf && !split) {  // the unsplit launch writes the whole gradient: it maps it
-        static std::atomic<uint32_t> lds_xf{0};
-        const int lds = K::LDS_BYTES + kDcXfBytes<P>;
-        ensure_lds_limit(reinterpret_cast<const void*>(&k_dc_pipe<P, BF, H, true>), lds, lds_xf);
-        hipLaunchKernelGGL((k_dc_pipe<P, BF, H, true>), grid, dim3(512), (size_t)lds, s,
-                           reinterpret_cast<const E*>(dYc), t, colsum, dC, p, L.dc_st_per_split,
-                           om, DcXf<true>{*xf});
-        return true;
-      }
+  constexpr int P = K::PP, M = K::MM, H = K::H, NN = K::NNA;
+  typedef typename K::E E;
+  const bool split = L.dc_splits > 1;
+  dim3 grid(p.NIB, (unsigned)ceil_div(p.NBf, K::NO), L.dc_splits);
+  if constexpr (dc_xf_fits<P, M, H, NN>()) {
+    if (xf && !split) {  // the unsplit launch writes the whole gradient: it maps it
+      static std::atomic<uint32_t> lds_xf{0};
+      const int lds = K::LDS_BYTES + kDcXfBytes<P>;
+      ensure_lds_limit(reinterpret_cast<const void*>(&k_dc_pipe<P, M, H, true, NN>), lds, lds_xf);
+      hipLaunchKernelGGL((k_dc_pipe<P, M, H, true, NN>), grid, dim3(512), (size_t)lds, s,
+                         reinterpret_cast<const E*>(dYc), t, colsum, dC, p, L.dc_st_per_split,
+                         om, DcXf<true>{*xf});
+      return;
     }
-    static std::atomic<uint32_t> lds_set{0};
-    ensure_lds_limit(reinterpret_cast<const void*>(&k_dc_pipe<P, BF, H>), K::LDS_BYTES, lds_set);
-    hipLaunchKernelGGL((k_dc_pipe<P, BF, H>), grid, dim3(512), K::LDS_BYTES, s,
-                       reinterpret_cast<const E*>(dYc), t, colsum, split ? part : dC, p,
-                       L.dc_st_per_split, split ? DcOut{kDcStore} : om, DcXf<false>{});
-    return true;
   }
-  return false;
-}
-
-template <int P, bool BF>
-static void dc_dispatch(const void* dYc, const float* t, const float* colsum, float* part,
-                        float* dC, DcOut om, const Plan& p, const BwdLayout& L,
-                        hipStream_t s, const BasisXform* xf) {
-  typedef typename Elem<BF>::type E;
-  if (L.dc_pipe) {
-    bool done = false;
-    if constexpr (P == 16) {  // dc_h(p) is 1 only for degree 16
-      if (dc_h(p) == 1) done = dc_pipe_launch<P, BF, 1>(dYc, t, colsum, part, dC, om, p, L, s, xf);
-    }
-    if (!done) done = dc_pipe_launch<P, BF, 2>(dYc, t, colsum, part, dC, om, p, L, s, xf);
-    if (done) return;
-  }
-  constexpr int NM = BwdTile<P>::NM;
-  dim3 grid((unsigned)ceil_div(p.NBf, 4 * NM), p.NIB, L.dc_splits);
-  hipLaunchKernelGGL((k_dc<P, BF, NM, DcKI<BF>::v>), grid, dim3(256), 0, s,
-                     reinterpret_cast<const E*>(dYc), t, part, p, L.dc_st_per_split);
+  static std::atomic<uint32_t> lds_set{0};
+  ensure_lds_limit(reinterpret_cast<const void*>(&k_dc_pipe<P, M, H, false, NN>), K::LDS_BYTES, lds_set);
+  hipLaunchKernelGGL((k_dc_pipe<P, M, H, false, NN>), grid, dim3(512), K::LDS_BYTES, s,
+                     reinterpret_cast<const E*>(dYc), t, colsum, split ? part : dC, p,
+                     L.dc_st_per_split, split ? DcOut{kDcStore} : om, DcXf<false>{});
 }
 
 bool dc_gemm_maps_basis(const Plan& p, const BwdLayout& L) {
   if (!L.dc_pipe || L.dc_splits > 1) return false;
-  const bool bf = p.esz == 2;
-  // the instantiation dc_dispatch launches, and whether it has LDS left for M
-  switch (p.P) {
-    case 2: return bf ? dc_xf_fits<2, true, 2>() : dc_xf_fits<2, false, 2>();
-    case 4: return bf ? dc_xf_fits<4, true, 2>() : dc_xf_fits<4, false, 2>();
-    case 8: return bf ? dc_xf_fits<8, true, 2>() : dc_xf_fits<8, false, 2>();
-    default: {  // H = 1 where dc_h says so and that kernel fits, else H = 2
-      const bool h1 = dc_h(p) == 1 && (bf ? DcPipe<16, true, 1>::kOk : DcPipe<16, false, 1>::kOk);
-      if (h1) return bf ? dc_xf_fits<16, true, 1>() : dc_xf_fits<16, false, 1>();
-      return bf ? dc_xf_fits<16, true, 2>() : dc_xf_fits<16, false, 2>();
-    }
-  }
+  // whether the instantiation launched has LDS left for M
+  return with_dc(p, [](auto k) {
+    typedef decltype(k) K;
+    return dc_xf_fits<K::PP, K::MM, K::H, K::NNA>();
+  });
 }
 
 void launch_dc_gemm(const void* dYc, const float* t, const float* colsum, float* part, float* dC,
                     DcOut om, const Plan& p, const BwdLayout& L, hipStream_t s,
                     const BasisXform* xf) {
-  const bool bf = p.esz == 2;
-#define CKAN_DC(PP, BB) dc_dispatch<PP, BB>(dYc, t, colsum, part, dC, om, p, L, s, xf)
-  switch (p.P) {
-    case 2: bf ? CKAN_DC(2, true) : CKAN_DC(2, false); break;
-    case 4: bf ? CKAN_DC(4, true) : CKAN_DC(4, false); break;
-    case 8: bf ? CKAN_DC(8, true) : CKAN_DC(8, false); break;
-    default: bf ? CKAN_DC(16, true) : CKAN_DC(16, false); break;
-  }
-#undef CKAN_DC
+  with_dc(p, [&](auto k) {
+    typedef decltype(k) K;
+    if constexpr (K::kOk) {
+      dc_pipe_launch<K>(dYc, t, colsum, part, dC, om, p, L, s, xf);
+    } else {
+      constexpr int P = K::PP;
+      constexpr bool BF = K::MM == kBf16;
+      static_assert(K::MM != kSplit, "a split layer has no other dC kernel");
+      constexpr int NM = BwdTile<P>::NM;
+      dim3 grid((unsigned)ceil_div(p.NBf, 4 * NM), p.NIB, L.dc_splits);
+      hipLaunchKernelGGL((k_dc<P, BF, NM, DcKI<BF>::v>), grid, dim3(256), 0, s,
+                         reinterpret_cast<const typename Elem<BF>::type*>(dYc), t, part, p,
+                         L.dc_st_per_split);
+    }
+    return 0;
+  });
 }
 
 bool fwd_tail_ce_ok(const Plan& pa, const FwdChoice& ca, int Ob, int Db) {

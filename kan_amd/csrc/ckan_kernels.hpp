@@ -26,14 +26,26 @@ inline void ensure_lds_limit(const void* fn, int bytes, std::atomic<uint32_t>& d
 // Sets the thread-local message returned by ckan_last_error().
 void set_last_error(const char* msg);
 
-// ---- packed coefficients: [Cf][Cb][bias partials][bias] -------------------
+// ---- packed coefficients: [Cf][Cb][Cf3][Cb3][bias partials][bias] -----------
 // Cf: forward B operand, C[i, o, d] for d >= 1 by (input, degree) k-blocks.
 // Cb: dX B operand, d * C[i, o, d] (the factor of dT_d/dt = d U_{d-1}) by
-// (input block, degree) and output k-blocks.
+// (input block, degree) and output k-blocks.  Both in the compute precision.
+// Split fp32 layers add the same operands in planes: Cf3 for the large-batch
+// forward (the small-batch ones stream Cf, a third fewer bytes), Cb3 for the
+// dX GEMM; there Cb itself is kept only for layers narrow enough for the
+// small dx (kDxSmallO outputs).
+constexpr int kDxSmallO = 64;  // outputs the small dx stages at once (all of them)
 inline size_t packed_cf_elems(const Plan& p) { return (size_t)p.NBf * p.KB * kFragElems; }
 inline size_t packed_cb_elems(const Plan& p) { return (size_t)p.NIB * p.P * p.KBx * kFragElems; }
+__host__ __device__ inline bool packed_has_cb(const Plan& p) { return !p.split || p.O <= kDxSmallO; }
+inline size_t packed_cf3_offset(const Plan& p) {
+  return align256((packed_cf_elems(p) + (packed_has_cb(p) ? packed_cb_elems(p) : 0)) * p.esz);
+}
+inline size_t packed_cb3_offset(const Plan& p) {
+  return packed_cf3_offset(p) + (p.split ? packed_cf_elems(p) * 6 : 0);
+}
 inline size_t packed_bias_offset(const Plan& p) {
-  return align256((packed_cf_elems(p) + packed_cb_elems(p)) * p.esz);
+  return align256(packed_cb3_offset(p) + (p.split ? packed_cb_elems(p) * 6 : 0));
 }
 // final per-output bias sum_i C[i, o, 0], reduced from the partials
 inline size_t packed_biasf_offset(const Plan& p) {

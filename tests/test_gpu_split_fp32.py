@@ -1,0 +1,93 @@
+"""GPU parity of the fp32 layers' three-plane bf16 GEMMs (degrees 3-16) at the
+sizes where their tilings change: row, input, output and degree remainders,
+the 64- and 128-column forward tiles with the reduction whole and split, both
+dC tile widths, split batches, and the input gradient's row blocks.
+
+Tolerance against the oracle in fp64: 4e-6 norm-wise.  The plane products
+dropped are below 2^-24 of each product and the planes are exact, so what
+remains is fp32 accumulation (at most 16384 terms here, at 2^-24 per rounding
+and the square root of their number: 1.5e-6 at 8192 terms) and the basis
+recurrence's rounding."""
+import pytest
+import torch
+
+from oracle import chebykan_oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+TOL = 4e-6
+
+
+def _rel(a, b):
+    a, b = a.detach().double().cpu(), b.detach().double().cpu()
+    return (a - b).norm().item() / b.norm().item()
+
+
+def _inputs(B, I, O, deg, seed=0):
+    g = torch.Generator().manual_seed(B + 3 * I + 5 * O + 7 * deg + seed)
+    x = torch.randn(B, I, generator=g) * 1.5
+    c = torch.randn(I, O, deg + 1, generator=g) / (I * (deg + 1))
+    dy = torch.randn(B, O, generator=g)
+    return x, c, dy
+
+
+def _run(x, c, dy):
+    from kan_amd import functional as F
+    xd, cd = x.cuda().requires_grad_(True), c.cuda().requires_grad_(True)
+    y = F.chebykan(xd, cd, "fp32")
+    y.backward(dy.cuda())
+    torch.cuda.synchronize()
+    return y.detach(), xd.grad, cd.grad
+
+
+@pytest.mark.parametrize("B,I,O,deg", [
+    (513, 40, 40, 3), (600, 33, 64, 4), (770, 100, 65, 4), (1025, 65, 130, 4),   # P = 4
+    (513, 40, 40, 5), (600, 33, 64, 8), (770, 100, 65, 7), (1025, 65, 130, 8),   # P = 8
+    (513, 40, 40, 9), (600, 33, 64, 16), (770, 100, 65, 12), (1025, 65, 130, 16),  # P = 16
+    (4097, 96, 300, 5),     # dC's narrow tile, batch split
+    (3000, 500, 257, 4),    # dC's wide and narrow tiles with remainders
+    (16400, 40, 33, 8),     # many row tiles, one output pair
+    (640, 1024, 128, 16),   # the forward reduction split over blocks
+    (130, 70, 500, 10), (300, 300, 96, 6),  # small batches: the fp32 forward, split gradients
+])
+def test_split_fp32_tilings(B, I, O, deg):
+    print(f"split fp32 B={B} I={I} O={O} deg={deg}", flush=True)
+    x, c, dy = _inputs(B, I, O, deg)
+    ref = orc.layer_forward_backward(x.double(), c.double(), dy.double())
+    for got, want in zip(_run(x, c, dy), ref):
+        assert _rel(got, want) <= TOL
+
+
+@pytest.mark.parametrize("deg", [4, 8, 16])
+def test_non_finite_and_extreme_values_stay_where_they_were(deg):
+    """An infinite coefficient or upstream gradient reaches exactly the results
+    that the fp32 products reach, with their sign; values next to overflow and
+    far below 1 keep their precision."""
+    B, I, O = 600, 40, 70
+    x, c, dy = _inputs(B, I, O, deg, 1)
+    x = x.abs() * 0.3 + 0.05
+    big = torch.finfo(torch.float32).max
+    c[3, 5, 1], c[7, 9, 1], c[11, 20, 0] = float("inf"), float("-inf"), float("nan")
+    c[:, 30] = 0
+    c[2, 30, 1] = big            # t < 1: finite results
+    c[:, 31] *= 1e-30
+    dy[10, 4], dy[20, 6] = float("inf"), float("-inf")
+    t = torch.tanh(x)
+    y, dx, dc = (v.cpu() for v in _run(x, c, dy))
+    basis = orc.basis_recurrence(t, deg)
+    # one non-finite term per affected sum: its sign decides
+    y_ref = torch.einsum("bid,iod->bo", basis.double(), c.double())
+    for o in (5, 9, 20):
+        assert torch.equal(torch.isnan(y[:, o]), torch.isnan(y_ref[:, o]))
+        ok = ~torch.isnan(y_ref[:, o])
+        assert torch.equal(y[ok, o], y_ref[ok, o].float())
+    rest = [o for o in range(O) if o not in (5, 9, 20)]
+    assert torch.isfinite(y[:, rest]).all()
+    for o in (30, 31):
+        assert _rel(y[:, o], y_ref[:, o]) <= TOL
+    for b, o, sign in ((10, 4, 1.0), (20, 6, -1.0)):
+        want = sign * basis[b] * float("inf")  # [I, D]: +-inf, nan where the basis is 0
+        got = dc[:, o]
+        sel = (basis[b].abs() > 0)
+        assert torch.equal(got[sel], want[sel])
+    assert torch.isfinite(dc[:, [o for o in range(O) if o not in (4, 6)]]).all()
