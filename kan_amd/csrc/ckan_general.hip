@@ -35,9 +35,9 @@
 // sizes, how far the reduction can be split to fill it.  Against the
 // vector-ALU register tiles that these kernels replaced (which put 64-128
 // blocks on the chip at these sizes), forward / dx / dC:
-//   2048 x 256 -> 256, degree 8, fp64:  483 / 112 / 532 -> 70 / 58 / 51 us
-//   4096 x 256 -> 128, degree 24, fp32: 1013 / 191 / 1534 -> 106 / 82 / 85 us
-// (41 / 49 / 56 TFLOP/s of products in fp64; 63 / 82 / 79 in fp32).
+//   2048 x 256 -> 256, degree 8, fp64:  483 / 112 / 532 -> 67 / 58 / 51 us
+//   4096 x 256 -> 128, degree 24, fp32: 1013 / 191 / 1534 -> 90 / 78 / 86 us
+// (36-47 TFLOP/s of products in fp64; 74-87 in fp32).
 #include "ckan_kernels.hpp"
 
 #include <math.h>
@@ -187,9 +187,14 @@ __device__ __forceinline__ void load_run(const T* src, const T* cend, int n, boo
 }
 
 // ---- forward ------------------------------------------------------------------
-// Wave tile 16 NM rows x 16 NN outputs.  A step is 4 inputs x one chunk of at
-// most kFwdDC degrees: its C tile goes through registers into one of two LDS
-// buffers while the other one's step runs.  LDS image: element (ii, o, d) at
+// Wave tile 16 NM rows x 16 NN outputs.  A step is 4 inputs x every degree
+// (WHOLE), or one chunk of at most kFwdDC degrees where LDS or registers do not
+// hold them: its C tile goes through registers into one of two LDS buffers
+// while the other one's step runs.  A WHOLE tile is 4 contiguous pieces of C,
+// read 16 bytes a lane in order; runs of a chunk are read by one thread each,
+// whose strided loads touch every line of the tile once per 16 bytes of run
+// and lose the L1 to each other (4096 x 256 -> 128, degree 24, fp32: 106 -> 90 us;
+// 2048 x 256 -> 256, degree 8, fp64: 70 -> 67).  LDS image: element (ii, o, d) at
 // ii * S + o * DP + d with DP odd and S = 16 DP (mod 64), so that the 64 lanes
 // of a read (16 outputs x 4 inputs at one degree) take distinct banks.
 template <typename T> constexpr int kFwdDC = sizeof(T) == 8 ? 9 : 17;
@@ -200,11 +205,12 @@ struct GenFwd {
   int rec_elems;
   int mblocks, nblocks;
 };
+constexpr int kFwdVecs = 9;  // 16-byte pieces of a WHOLE tile that a thread stages
 template <int NN> __host__ __device__ constexpr int fwd_stride(int dp) {
   return 16 * NN * dp + (16 * dp * (NN == 4 ? 1 : NN == 2 ? 3 : 0)) % 64;
 }
 
-template <typename T, int NM, int NN, bool GEN>
+template <typename T, int NM, int NN, bool WHOLE, bool GEN>
 __device__ __forceinline__ void gen_fwd_body(const T* __restrict__ t, const T* __restrict__ C,
                                              T* __restrict__ y, int64_t B, int I, int O, int D,
                                              const GenFwd f, T* lds, const T* rs) {
@@ -233,31 +239,89 @@ __device__ __forceinline__ void gen_fwd_body(const T* __restrict__ t, const T* _
     trow[m] = t + (b < B ? b : 0) * I;
   }
 
-  // C's tile is 64 NN runs of dn degrees, (input q / 16 NN, output q % 16 NN);
-  // thread q of the group's first NN waves stages run q (two runs where a
-  // group has NN / 2 waves)
-  constexpr int kRuns = NN > 1 ? 2 : 1;
-  T pre[kRuns][kFwdDC<T>], tn[NM];
   const T* cend = C + (size_t)I * O * D;
-  auto load_tile = [&](int i0, int d0, int dn) {
+  constexpr int V = Run<T>::V;
+  typedef typename Run<T>::vec vec;
+  // WHOLE: thread q stages pieces q, q + nth, ...: piece -> (input ii, element e
+  // of its 16 NN D); an even D leaves one element of LDS after each output
+  const int per_in = 16 * NN * D / V, nth = 64 * WM, total = 4 * per_in;
+  int goff[WHOLE ? kFwdVecs : 1], loff[WHOLE ? kFwdVecs : 1], dv[WHOLE ? kFwdVecs : 1];
+  vec pv[WHOLE ? kFwdVecs : 1];
+  if constexpr (WHOLE) {
 #pragma unroll
-    for (int r = 0; r < kRuns; ++r) {
-      if (r * WM + wm < NN) {
-        const int q = (r * WM + wm) * 64 + lane, i = i0 + q / (16 * NN), o = o0 + q % (16 * NN);
-        const bool ok = i < I && o < O;
-        load_run<T, kFwdDC<T>>(ok ? C + ((size_t)i * O + o) * D + d0 : C, cend, dn, ok, pre[r]);
+    for (int k = 0; k < kFwdVecs; ++k) {
+      const int q = k * nth + wm * 64 + lane, qc = q < total ? q : 0;
+      const int ii = qc / per_in, e = (qc - ii * per_in) * V, od = e / D;
+      goff[k] = ii * O * D + e;
+      loff[k] = ii * f.s + e + (D & 1 ? 0 : od);
+      dv[k] = e - od * D;
+    }
+  }
+  // chunked: C's tile is 64 NN runs of dn degrees, (input q / 16 NN, output
+  // q % 16 NN); thread q of the group's first NN waves stages run q (two runs
+  // where a group has NN / 2 waves)
+  constexpr int kRuns = NN > 1 ? 2 : 1;
+  T pre[WHOLE ? 1 : kRuns][WHOLE ? 1 : kFwdDC<T>], tn[NM];
+  auto load_tile = [&](int i0, int d0, int dn) {
+    if constexpr (WHOLE) {
+      const T* base = C + ((size_t)i0 * O + o0) * D;
+      if (i0 + 4 <= I && base + 3 * (size_t)O * D + 16 * NN * D <= cend) {
+#pragma unroll
+        for (int k = 0; k < kFwdVecs; ++k)
+          if (k * nth < total) pv[k] = *reinterpret_cast<const vec*>(base + goff[k]);
+      } else {
+        // the layer's last inputs or outputs, element by element: zeros past the
+        // inputs; past the outputs, whatever C holds there (results not stored)
+        const int64_t left = cend - base;
+        const int last = (int)(left > (1 << 30) ? (1 << 30) : left) - 1, ni = I - i0;
+#pragma unroll
+        for (int k = 0; k < kFwdVecs; ++k) {
+          if (k * nth < total) {
+            int e0 = goff[k];
+            asm volatile("" : "+v"(e0));  // addresses formed here, not kept across the loop
+            const bool ok = ni > 0 && (k * nth + wm * 64 + lane) < ni * per_in;
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+              const T x = ok ? base[e0 + v < last ? e0 + v : last] : T(0);
+              pv[k][v] = x;
+            }
+          }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < kRuns; ++r) {
+        if (r * WM + wm < NN) {
+          const int q = (r * WM + wm) * 64 + lane, i = i0 + q / (16 * NN), o = o0 + q % (16 * NN);
+          const bool ok = i < I && o < O;
+          load_run<T, kFwdDC<T>>(ok ? C + ((size_t)i * O + o) * D + d0 : C, cend, dn, ok, pre[r]);
+        }
       }
     }
   };
   auto store_tile = [&](T* dst, int dn) {
+    if constexpr (WHOLE) {
 #pragma unroll
-    for (int r = 0; r < kRuns; ++r) {
-      if (r * WM + wm < NN) {
-        const int q = (r * WM + wm) * 64 + lane;
-        T* run = dst + (q / (16 * NN)) * f.s + (q % (16 * NN)) * f.dp;
+      for (int k = 0; k < kFwdVecs; ++k) {
+        if (k * nth < total && k * nth + wm * 64 + lane < total) {
+          if (D & 1) {
+            *reinterpret_cast<vec*>(dst + loff[k]) = pv[k];
+          } else {
 #pragma unroll
-        for (int d = 0; d < kFwdDC<T>; ++d)
-          if (d < dn) run[d] = pre[r][d];
+            for (int v = 0; v < V; ++v) dst[loff[k] + v + (dv[k] + v >= D)] = pv[k][v];
+          }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < kRuns; ++r) {
+        if (r * WM + wm < NN) {
+          const int q = (r * WM + wm) * 64 + lane;
+          T* run = dst + (q / (16 * NN)) * f.s + (q % (16 * NN)) * f.dp;
+#pragma unroll
+          for (int d = 0; d < kFwdDC<T>; ++d)
+            if (d < dn) run[d] = pre[r][d];
+        }
       }
     }
   };
@@ -349,15 +413,15 @@ template <typename T> __device__ __forceinline__ T* dyn_lds() {
   return reinterpret_cast<T*>(gen_lds);
 }
 
-template <typename T, int NM, int NN>
+template <typename T, int NM, int NN, bool WHOLE>
 __global__ void __launch_bounds__(512)
 k_gen_fwd(const T* __restrict__ t, const T* __restrict__ C, T* __restrict__ y, int64_t B, int I,
           int O, int D, GenFwd f, const T* __restrict__ rec) {
   T* lds = dyn_lds<T>();
   const bool gen = stage_rec<T>(lds, rec, D);
   __syncthreads();
-  if (gen) gen_fwd_body<T, NM, NN, true>(t, C, y, B, I, O, D, f, lds, lds);
-  else gen_fwd_body<T, NM, NN, false>(t, C, y, B, I, O, D, f, lds, lds);
+  if (gen) gen_fwd_body<T, NM, NN, WHOLE, true>(t, C, y, B, I, O, D, f, lds, lds);
+  else gen_fwd_body<T, NM, NN, WHOLE, false>(t, C, y, B, I, O, D, f, lds, lds);
 }
 
 // ---- dx -------------------------------------------------------------------------
@@ -365,10 +429,12 @@ k_gen_fwd(const T* __restrict__ t, const T* __restrict__ C, T* __restrict__ y, i
 // degree; a chunk's G is folded into dx by the lane that holds it before the
 // next chunk starts.  A step is 16 outputs: lane group g takes outputs 4 g ..
 // 4 g + 3 of it, so a lane reads 4 consecutive dy values.  C's tile [16
-// inputs][16 outputs][DM] goes through registers into one of two LDS buffers,
-// one (input, output) run of degrees per thread; element (i, o = 4 g + s, d)
-// at i * S + g * Q + s * DM + d with S odd and Q = 16 S (mod 64): the 64 lanes
-// of a read take distinct banks.  A second row fragment per wave would halve
+// inputs][16 outputs][degrees] goes through registers into one of two LDS
+// buffers; element (i, o = 4 g + s, d) at i * S + g * Q + s * ds + d with S odd
+// and Q = 16 S (mod 64): the 64 lanes of a read take distinct banks.  WHOLE
+// (every degree in one chunk, ds = D <= DM): 16 contiguous pieces of C, read 16
+// bytes a lane in order; else one (input, output) run of degrees per thread,
+// ds = DM.  A second row fragment per wave would halve
 // the LDS reads, which are far from the bound (4 per SIMD round of one matrix
 // instruction each), and spills.
 template <int DM> struct GenDxLds {
@@ -383,7 +449,7 @@ struct GenDx {
   float ima;
 };
 
-template <typename T, int DM, bool GEN>
+template <typename T, int DM, bool WHOLE, bool GEN>
 __device__ __forceinline__ void gen_dx_body(const T* __restrict__ t, const T* __restrict__ C,
                                             const T* __restrict__ dy, T* __restrict__ dx, int64_t B,
                                             int I, int O, int D, const GenDx f, T* lds,
@@ -400,25 +466,59 @@ __device__ __forceinline__ void gen_dx_body(const T* __restrict__ t, const T* __
   const int half = f.wk * L::kStage;
 
   const T* yrow = dy + (b0 + l15 < B ? b0 + l15 : 0) * O + 4 * g;  // rows past B are not stored
-  // waves 0-3 of a group stage its C tile: thread q the run of degrees of
-  // (input q / 16, output q % 16)
+  // waves 0-3 of a group stage its C tile: pieces q, q + 256, ... (WHOLE), or
+  // thread q the run of degrees of (input q / 16, output q % 16)
   const bool stager = wm < 4;
   const int q = (wm & 3) * 64 + lane;
+  const T* cend = C + (size_t)I * O * D;
+  constexpr int V = Run<T>::V, NV = (DM + V - 1) / V;
+  typedef typename Run<T>::vec vec;
+  const int per_in = 16 * D / V, total = 16 * per_in;  // D / V pieces a thread
+  int goff[WHOLE ? NV : 1], loff[WHOLE ? NV : 1];
+  vec pv[WHOLE ? NV : 1];
+  if constexpr (WHOLE) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const int qc = k * 256 + q < total ? k * 256 + q : 0;
+      const int ii = qc / per_in, e = (qc - ii * per_in) * V, gg = e / (4 * D);
+      goff[k] = ii * O * D + e;
+      loff[k] = ii * L::S + gg * L::Q + (e - gg * 4 * D);
+    }
+  }
   const bool iok = i0 + (q >> 4) < I;
   const T* crun = C + (size_t)(iok ? i0 + (q >> 4) : 0) * O * D;
-  const T* cend = C + (size_t)I * O * D;
   T* cdst = buf + (q >> 4) * L::S + ((q >> 2) & 3) * L::Q + (q & 3) * DM;
 
   T s[4];  // this lane's (b, i) pairs: rows b0 + row(v, g), input i0 + l15
 #pragma unroll
   for (int v = 0; v < 4; ++v) s[v] = T(0);
 
-  T pre[DM], an[4];
+  T pre[WHOLE ? 1 : DM], an[4];
   auto load_step = [&](int ob, int d0, int dn) {
-    if (stager) {
+    if (stager && WHOLE) {
+      const T* base = C + ((size_t)i0 * O + ob) * D;
+      if (i0 + 16 <= I && ob + 16 <= O) {
+#pragma unroll
+        for (int k = 0; k < NV; ++k)
+          if (k * 256 < total) pv[k] = *reinterpret_cast<const vec*>(base + goff[k]);
+      } else {  // zeros past the layer's inputs and outputs
+        const int lim = (O - ob) * D, ni = I - i0;
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+          if (k * 256 < total) {
+            int e0 = goff[k], qk = k * 256 + q;
+            asm volatile("" : "+v"(e0), "+v"(qk));  // addresses formed here, not kept across the loop
+            const int e = (qk % per_in) * V;
+            const bool ok = qk < total && qk < ni * per_in;
+#pragma unroll
+            for (int v = 0; v < V; ++v) pv[k][v] = ok && e + v < lim ? base[e0 + v] : T(0);
+          }
+        }
+      }
+    } else if (stager) {
       const int o = ob + (q & 15);
       const bool ok = iok && o < O;
-      load_run<T, DM>(ok ? crun + (size_t)o * D + d0 : C, cend, dn, ok, pre);
+      if constexpr (!WHOLE) load_run<T, DM>(ok ? crun + (size_t)o * D + d0 : C, cend, dn, ok, pre);
     }
     if (ob + 16 <= O) {
       constexpr int V = Run<T>::V;
@@ -434,9 +534,17 @@ __device__ __forceinline__ void gen_dx_body(const T* __restrict__ t, const T* __
     }
   };
   auto store_step = [&](int b) {
-    if (stager) {
+    if (stager && WHOLE) {
 #pragma unroll
-      for (int k = 0; k < DM; ++k) cdst[b * half + k] = pre[k];
+      for (int k = 0; k < NV; ++k) {
+        if (k * 256 < total && k * 256 + q < total) {
+#pragma unroll
+          for (int v = 0; v < V; ++v) buf[b * half + loff[k] + v] = pv[k][v];
+        }
+      }
+    } else if (stager) {
+#pragma unroll
+      for (int k = 0; k < DM; ++k) cdst[b * half + k] = pre[WHOLE ? 0 : k];
     }
   };
 
@@ -461,14 +569,18 @@ __device__ __forceinline__ void gen_dx_body(const T* __restrict__ t, const T* __
       }
       const T* bp = buf + cur * half + l15 * L::S + g * L::Q;
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
+      for (int k = 0; k < 4; ++k) {
+        const T* bk = bp + k * (WHOLE ? D : DM);  // (degrees past D: values no one uses)
 #pragma unroll
-        for (int d = 0; d < DM; ++d) acc[d] = Mx<T>::mma(a[k], bp[k * DM + d], acc[d]);
+        for (int d = 0; d < DM; ++d) acc[d] = Mx<T>::mma(a[k], bk[d], acc[d]);
+      }
       if (more) store_step(cur ^ 1);
       cur ^= 1;
       __syncthreads();
     }
-    // s += sum_d G_d P_d'(t) over the chunk (this reduction group's share of G)
+    // s += sum_d G_d P_d'(t) over the chunk (this reduction group's share of G);
+    // a WHOLE chunk in two sums, as two chunks would be
+    const int dh = WHOLE && sizeof(T) == 4 ? (D + 1) / 2 : 0;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int64_t b = b0 + Mx<T>::row(v, g);
@@ -493,6 +605,10 @@ __device__ __forceinline__ void gen_dx_body(const T* __restrict__ t, const T* __
         for (int n = 1; n <= d0; ++n) step(n);
 #pragma unroll
         for (int d = 0; d < DM; ++d) {
+          if (d > 0 && d == dh) {
+            s[v] += sum * rs[3 * D];
+            sum = T(0);
+          }
           if (d < dn) {
             sum = fma(acc[d][v], qc, sum);
             step(d0 + d + 1);
@@ -511,6 +627,10 @@ __device__ __forceinline__ void gen_dx_body(const T* __restrict__ t, const T* __
         T deg = (T)d0;  // counted in T (exact)
 #pragma unroll
         for (int d = 0; d < DM; ++d) {
+          if (d > 0 && d == dh) {
+            s[v] += sum;
+            sum = T(0);
+          }
           if (d < dn && (d > 0 || d0 > 0)) {
             sum = fma(acc[d][v] * deg, u, sum);
             const T un = fma(t2, u, -up);
@@ -548,15 +668,15 @@ __device__ __forceinline__ void gen_dx_body(const T* __restrict__ t, const T* __
   }
 }
 
-template <typename T, int DM>
+template <typename T, int DM, bool WHOLE>
 __global__ void __launch_bounds__(512)
 k_gen_dx(const T* __restrict__ t, const T* __restrict__ C, const T* __restrict__ dy,
          T* __restrict__ dx, int64_t B, int I, int O, int D, GenDx f, const T* __restrict__ rec) {
   T* lds = dyn_lds<T>();
   const bool gen = stage_rec<T>(lds, rec, D);
   __syncthreads();
-  if (gen) gen_dx_body<T, DM, true>(t, C, dy, dx, B, I, O, D, f, lds, lds);
-  else gen_dx_body<T, DM, false>(t, C, dy, dx, B, I, O, D, f, lds, lds);
+  if (gen) gen_dx_body<T, DM, WHOLE, true>(t, C, dy, dx, B, I, O, D, f, lds, lds);
+  else gen_dx_body<T, DM, WHOLE, false>(t, C, dy, dx, B, I, O, D, f, lds, lds);
 }
 
 // ---- dC ---------------------------------------------------------------------------
@@ -752,12 +872,12 @@ static int even_chunk(int D, int cap) {
   return (D + n - 1) / n;
 }
 
-template <typename T, int NM, int NN>
+template <typename T, int NM, int NN, bool WHOLE>
 static bool gen_fwd_launch(const T* t, const T* C, T* y, int64_t B, int I, int O, int D,
                            const T* rec, hipStream_t s, bool must) {
   static std::atomic<uint32_t> lds_done{0};
   GenFwd f;
-  f.dc = even_chunk(D, kFwdDC<T>);
+  f.dc = WHOLE ? D : even_chunk(D, kFwdDC<T>);
   f.nch = (D + f.dc - 1) / f.dc;
   f.dp = f.dc | 1;
   f.s = fwd_stride<NN>(f.dp);
@@ -767,16 +887,21 @@ static bool gen_fwd_launch(const T* t, const T* C, T* y, int64_t B, int I, int O
     const int64_t st = 2LL * wk * 4 * f.s, red = wk > 1 ? (int64_t)(kWaves / wk) * 64 * NM * NN * 4 : 0;
     return (f.rec_elems + (st > red ? st : red)) * (int64_t)sizeof(T);
   };
-  const int wk_max = NN == 4 ? 4 : 8;  // WM = 8 / wk >= NN / 2: a thread stages two runs at most
+  // what a thread stages, and the 32-bit offsets of a WHOLE tile
+  auto fits = [&](int wk) {
+    const int WM = kWaves / wk;
+    return bytes(wk) <= kMaxLds &&
+           (WHOLE ? NN * D <= kFwdVecs * Run<T>::V * WM && (int64_t)O * D < (1 << 28) : WM >= NN / 2);
+  };
   int wk = 1;
-  while (wk < wk_max && mt * nt * wk < kWantWaves && 2 * wk <= (I + 3) / 4 && bytes(2 * wk) <= kMaxLds) wk *= 2;
-  if (!must && mt * nt * wk < kWantWaves) return false;
+  while (wk < 8 && mt * nt * wk < kWantWaves && 2 * wk <= (I + 3) / 4 && fits(2 * wk)) wk *= 2;
+  if (!fits(wk) || (!must && mt * nt * wk < kWantWaves)) return false;
   f.wk = wk;
   const int WM = kWaves / wk;
   f.mblocks = (int)((mt + WM - 1) / WM);
   f.nblocks = (int)nt;
-  ensure_lds_limit(reinterpret_cast<const void*>(&k_gen_fwd<T, NM, NN>), kMaxLds, lds_done);
-  hipLaunchKernelGGL((k_gen_fwd<T, NM, NN>), dim3((unsigned)f.mblocks * f.nblocks), dim3(512),
+  ensure_lds_limit(reinterpret_cast<const void*>(&k_gen_fwd<T, NM, NN, WHOLE>), kMaxLds, lds_done);
+  hipLaunchKernelGGL((k_gen_fwd<T, NM, NN, WHOLE>), dim3((unsigned)f.mblocks * f.nblocks), dim3(512),
                      (size_t)bytes(wk), s, t, C, y, B, I, O, D, f, rec);
   return true;
 }
@@ -787,13 +912,16 @@ void launch_forward_general(const T* x, const T* C, T* y, T* t, int64_t B, int I
   if (B == 0) return;
   hipLaunchKernelGGL(k_tanh_v<T>, dim3(vgrid(B * I)), dim3(256), 0, s, x, t, B * I, imap, ima, imb);
   const int D = deg + 1;
-  // the largest wave tile whose launch still fills the chip
-  if (gen_fwd_launch<T, 2, 4>(t, C, y, B, I, O, D, rec, s, false)) return;
-  if (gen_fwd_launch<T, 2, 2>(t, C, y, B, I, O, D, rec, s, false)) return;
-  gen_fwd_launch<T, 1, 1>(t, C, y, B, I, O, D, rec, s, true);
+  // the largest wave tile whose launch still fills the chip, WHOLE where it fits
+  if (gen_fwd_launch<T, 2, 4, true>(t, C, y, B, I, O, D, rec, s, false)) return;
+  if (gen_fwd_launch<T, 2, 2, true>(t, C, y, B, I, O, D, rec, s, false)) return;
+  if (gen_fwd_launch<T, 2, 4, false>(t, C, y, B, I, O, D, rec, s, false)) return;
+  if (gen_fwd_launch<T, 2, 2, false>(t, C, y, B, I, O, D, rec, s, false)) return;
+  if (gen_fwd_launch<T, 1, 1, true>(t, C, y, B, I, O, D, rec, s, true)) return;
+  gen_fwd_launch<T, 1, 1, false>(t, C, y, B, I, O, D, rec, s, true);
 }
 
-template <typename T, int DM>
+template <typename T, int DM, bool WHOLE>
 static void gen_dx(const T* t, const T* C, const T* dy, T* dx, int64_t B, int I, int O, int D,
                    const T* rec, int imap, float ima, hipStream_t s) {
   static std::atomic<uint32_t> lds_done{0};
@@ -808,8 +936,8 @@ static void gen_dx(const T* t, const T* C, const T* dy, T* dx, int64_t B, int I,
   const int WM = kWaves / f.wk;
   f.mblocks = (int)((mt + WM - 1) / WM);
   const size_t bytes = (f.rec_elems + 2 * (size_t)f.wk * GenDxLds<DM>::kStage) * sizeof(T);
-  ensure_lds_limit(reinterpret_cast<const void*>(&k_gen_dx<T, DM>), kMaxLds, lds_done);
-  hipLaunchKernelGGL((k_gen_dx<T, DM>), dim3((unsigned)(f.mblocks * it)), dim3(512), bytes, s, t, C,
+  ensure_lds_limit(reinterpret_cast<const void*>(&k_gen_dx<T, DM, WHOLE>), kMaxLds, lds_done);
+  hipLaunchKernelGGL((k_gen_dx<T, DM, WHOLE>), dim3((unsigned)(f.mblocks * it)), dim3(512), bytes, s, t, C,
                      dy, dx, B, I, O, D, f, rec);
 }
 
@@ -848,40 +976,43 @@ static void gen_dc(const T* t, const T* dy, T* dC, DcOut om, int64_t B, int I, i
   gen_dc_launch<T, DM, 1>(t, dy, dC, om, B, I, O, D, rec, s, true);
 }
 
-// Calls f with the degrees per chunk of a layer of D degrees as a constant:
-// the fewest chunks that the accumulators allow (9 degrees in fp64, 17 in
-// fp32), evenly sized, so that few of a chunk's degrees are padding.
-template <typename F> static void with_chunk_f64(int D, F f) {
-  switch (even_chunk(D, 9)) {
-    case 1: case 2: case 3: f(std::integral_constant<int, 3>()); break;
-    case 4: case 5: f(std::integral_constant<int, 5>()); break;
-    case 6: f(std::integral_constant<int, 6>()); break;
-    case 7: f(std::integral_constant<int, 7>()); break;
-    case 8: f(std::integral_constant<int, 8>()); break;
-    default: f(std::integral_constant<int, 9>()); break;
+// Calls f with the accumulators' degree capacity as a constant: the first of
+// the list that holds n (its last one does).
+template <int A, int... R, typename F> static void with_degrees(int n, F f) {
+  if constexpr (sizeof...(R) > 0) {
+    if (n > A) return with_degrees<R...>(n, f);
   }
+  f(std::integral_constant<int, A>());
 }
-template <typename F> static void with_chunk_f32(int D, F f) {  // D >= 18
-  const int c = even_chunk(D, 17);
-  if (c <= 9) f(std::integral_constant<int, 9>());
-  else if (c <= 11) f(std::integral_constant<int, 11>());
-  else if (c <= 13) f(std::integral_constant<int, 13>());
-  else if (c <= 15) f(std::integral_constant<int, 15>());
-  else f(std::integral_constant<int, 17>());
-}
+
+// Degrees of dx in one chunk: what fits the registers beside the staging.
+template <typename T> constexpr int kDxDegrees = sizeof(T) == 8 ? 9 : 27;
 
 template <typename T>
 void launch_backward_general(const T* t, const T* C, const T* dy, T* dx, T* dC, DcOut om, int64_t B,
                              int I, int O, int deg, hipStream_t s, const T* rec, int imap,
                              float ima) {
   const int D = deg + 1;
-  auto go = [&](auto dm) {
-    constexpr int DM = decltype(dm)::value;
-    if (dx && B > 0) gen_dx<T, DM>(t, C, dy, dx, B, I, O, D, rec, imap, ima, s);
-    if (dC) gen_dc<T, DM>(t, dy, dC, om, B, I, O, D, rec, s);
-  };
-  if constexpr (sizeof(T) == 8) with_chunk_f64(D, go);
-  else with_chunk_f32(D, go);
+  constexpr bool F64 = sizeof(T) == 8;
+  if (dx && B > 0) {
+    // one chunk, staged whole (32-bit offsets), or the fewest chunks of equal size
+    const bool whole = D <= kDxDegrees<T> && (int64_t)O * D < (1 << 26);
+    auto go = [&](auto dm) { gen_dx<T, decltype(dm)::value, true>(t, C, dy, dx, B, I, O, D, rec, imap, ima, s); };
+    auto chunks = [&](auto dm) { gen_dx<T, decltype(dm)::value, false>(t, C, dy, dx, B, I, O, D, rec, imap, ima, s); };
+    const int c = even_chunk(D, kDxDegrees<T>);
+    if constexpr (F64) {
+      if (whole) with_degrees<2, 3, 4, 5, 6, 7, 8, 9>(D, go);
+      else with_degrees<3, 5, 6, 7, 8, 9>(c, chunks);
+    } else {  // D >= 18
+      if (whole) with_degrees<19, 21, 23, 25, 27>(D, go);
+      else with_degrees<15, 17, 21, 25, 27>(c, chunks);
+    }
+  }
+  if (dC) {
+    auto go = [&](auto dm) { gen_dc<T, decltype(dm)::value>(t, dy, dC, om, B, I, O, D, rec, s); };
+    if constexpr (F64) with_degrees<3, 5, 6, 7, 8, 9>(even_chunk(D, 9), go);
+    else with_degrees<9, 11, 13, 15, 17>(even_chunk(D, 17), go);
+  }
 }
 
 template void launch_forward_general<float>(const float*, const float*, float*, float*, int64_t, int,

@@ -59,6 +59,7 @@ def _check(dtype, B, I, O, deg, family=None):
     (2050, 257, 20, 7),    # dx unsplit; odd widths
     (70, 250, 500, 8),     # dC on 32-output tiles
     (130, 100, 130, 2),    # dC on 64-output tiles
+    (200, 30, 33, 4), (200, 33, 30, 3), (90, 20, 250, 17),  # even and odd degree counts of the staging
     (48, 40, 30, 9), (50, 20, 24, 10), (31, 17, 40, 12), (33, 24, 20, 14), (40, 18, 35, 27),  # chunks
 ])
 @pytest.mark.parametrize("family", [None, "jacobi"])
@@ -69,6 +70,7 @@ def test_fp64_tilings(B, I, O, deg, family):
 @pytest.mark.parametrize("B,I,O,deg", [
     (4100, 20, 250, 17), (2049, 33, 100, 24), (65, 50, 18, 20), (1, 3, 1, 17), (17, 5, 33, 33),
     (2050, 257, 20, 18), (70, 250, 500, 24), (70, 260, 500, 17),
+    (300, 40, 33, 25), (2049, 17, 33, 26),  # dx in one chunk: row, input and output remainders
     (40, 18, 35, 28), (33, 24, 20, 30), (50, 20, 24, 40), (31, 17, 40, 100),
 ])
 @pytest.mark.parametrize("family", [None, "jacobi"])
