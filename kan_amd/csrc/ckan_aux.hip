@@ -2,6 +2,8 @@
 // coefficient packing, the dy re-layout, the dC finalisation, the optimizers
 // and the materialised basis.  All are HBM-bound elementwise or re-layout
 // passes; each moves its bytes once with coalesced accesses.
+#include <type_traits>
+
 #include "ckan_kernels.hpp"
 
 namespace ckan {
@@ -109,19 +111,36 @@ static PackPlanes pack_planes(void* packed, const Plan& p) {
           reinterpret_cast<uint16_t*>(base + packed_cb3_offset(p))};
 }
 
-// One pack block: input block ib, output block ob; `lin` numbers the block
-// for its tanh share.
-template <int P, bool BF, typename CT, bool XF>
-__device__ __forceinline__ void pack_tile(const CT* __restrict__ C, typename Elem<BF>::type* __restrict__ Cf,
+// Outputs per pack block: 32 (whole fragments, the longest runs of C), or 8
+// (one 16-byte piece of a Cb lane, 8 lanes of a Cf fragment) where 32 would
+// leave CUs without a block, so that the pack is the latency of a block's loads
+// and re-layouts, and at P = 16, where 32 outputs take 70 KB of LDS and two
+// blocks a CU.  Measured, 32 against 8 outputs (us): 736 -> 42, degree 7, fp32
+// 14 / 7; 64 -> 128 and 128 -> 13, degree 14, in one launch 18 / 8; 1184 -> 211,
+// degree 15 (Hermite, the change of basis and tanh included) 51 / 28; 1792 ->
+// 544, degree 13 (the same) 77 / 58; 1020 -> 640, degree 9 37 / 30; but 1024 ->
+// 1024, degree 8 28 / 37 and 600 -> 500, degree 4 18 / 20.
+inline int pack_ow(const Plan& p) {
+  return p.P == 16 || (int64_t)p.NIB * (p.O64 / 32) < kNumCUs ? 8 : 32;
+}
+inline int64_t pack_blocks(const Plan& p) { return (int64_t)p.NIB * (p.O64 / pack_ow(p)); }
+// LDS of one block: the tile and the bias groups.
+template <int P, int OW> struct PackLds {
+  float tile[32 * (OW * (P + 1) + 1)];
+  float bsum[8][OW];
+};
+
+// One pack block: input block ib, outputs OW ow .. OW ow + OW - 1; `lin`
+// numbers the block for its tanh share.
+template <int P, bool BF, typename CT, bool XF, int OW>
+__device__ __forceinline__ void pack_tile(PackLds<P, OW>& lds, const CT* __restrict__ C, typename Elem<BF>::type* __restrict__ Cf,
                                           typename Elem<BF>::type* __restrict__ Cb,
                                           float* __restrict__ bias_part, const PackPlanes& pl,
                                           const Plan& p, int cal, const XfArg<XF>& xf,
-                                          const TanhJob& tj, int ib, int ob, int64_t lin) {
+                                          const TanhJob& tj, int ib, int ow, int64_t lin) {
   using G = FwdGroup<P>;
   constexpr bool SP = !BF && P >= kSplitMinP;
-  constexpr int RPMAX = 32 * (P + 1) + 1;
-  __shared__ float tile[32 * RPMAX];
-  __shared__ float bsum[8][32];
+  float* tile = lds.tile;
   const int tid = threadIdx.x;
   // tanh share: the first chunk's loads go out with the tile's, so both streams
   // are in flight together; the tanh itself runs after the re-layout
@@ -145,22 +164,22 @@ __device__ __forceinline__ void pack_tile(const CT* __restrict__ C, typename Ele
     }
   };
   bool first_done = false;  // the first chunk is done while the tile loads (float4 path)
-  const int i0 = ib * 32, o0 = ob * 32;
+  const int i0 = ib * 32, o0 = ow * OW, ob = o0 >> 5, olo = o0 & 31;
   const int D = p.D;
-  const int RP = 32 * D + 1;
-  const int ocount = min(32, p.O - o0);  // may be <= 0 for the Cb zero-fill blocks
+  const int RP = OW * D + 1;
+  const int ocount = min(OW, p.O - o0);  // may be <= 0 for the Cb zero-fill blocks
   const int nrow = ocount > 0 ? ocount * D : 0;
   // Each input's run of 32*D values is contiguous in C.  When the run is
   // 16-byte aligned, every thread issues its float4 loads before any use.
-  const bool vec = sizeof(CT) == 4 && cal && ((size_t)p.O * D) % 4 == 0 && ocount == 32;
+  const bool vec = sizeof(CT) == 4 && cal && ((size_t)p.O * D) % 4 == 0 && ocount == OW;
   if (vec) {
-    constexpr int MAXV = (32 * 32 * (P + 1) / 4 + 255) / 256;  // float4 per thread
-    const int nv = 32 * 8 * D;                                   // float4 in the tile
+    constexpr int MAXV = (32 * OW * (P + 1) / 4 + 255) / 256;  // float4 per thread
+    const int nv = 32 * (OW / 4) * D;                                   // float4 in the tile
     f32x4_t buf[MAXV];
 #pragma unroll
     for (int q = 0; q < MAXV; ++q) {
       const int v = tid + q * 256;
-      const int il = v / (8 * D), k4 = v - il * (8 * D);
+      const int il = v / (OW / 4 * D), k4 = v - il * (OW / 4 * D);
       const int i = i0 + il;
       buf[q] = (v < nv && i < p.I)
           ? __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(C) + ((size_t)i * p.O + o0) * D + k4 * 4))
@@ -174,7 +193,7 @@ __device__ __forceinline__ void pack_tile(const CT* __restrict__ C, typename Ele
     for (int q = 0; q < MAXV; ++q) {
       const int v = tid + q * 256;
       if (v < nv) {
-        const int il = v / (8 * D), k4 = v - il * (8 * D);
+        const int il = v / (OW / 4 * D), k4 = v - il * (OW / 4 * D);
         float* dst = tile + il * RP + k4 * 4;
         dst[0] = buf[q][0]; dst[1] = buf[q][1]; dst[2] = buf[q][2]; dst[3] = buf[q][3];
       }
@@ -183,20 +202,20 @@ __device__ __forceinline__ void pack_tile(const CT* __restrict__ C, typename Ele
     // element k of the flattened [32 inputs][32 * D] tile; 16 loads in flight
     // per thread before any is stored (one at a time made small packs
     // latency-bound: 13.7 us for a 64 x 10 x 5 layer)
-    const int nt = 32 * 32 * D;
+    const int nt = 32 * OW * D;
     for (int k0 = 0; k0 < nt; k0 += 256 * 16) {
       float v[16];
 #pragma unroll
       for (int u = 0; u < 16; ++u) {
         const int k = k0 + u * 256 + tid;
-        const int il = k / (32 * D), e = k - il * (32 * D);
+        const int il = k / (OW * D), e = k - il * (OW * D);
         const int i = i0 + il;
         v[u] = (k < nt && i < p.I && e < nrow) ? to_f32<CT>(C[((size_t)i * p.O + o0) * D + e]) : 0.0f;
       }
 #pragma unroll
       for (int u = 0; u < 16; ++u) {
         const int k = k0 + u * 256 + tid;
-        const int il = k / (32 * D), e = k - il * (32 * D);
+        const int il = k / (OW * D), e = k - il * (OW * D);
         if (k < nt) tile[il * RP + e] = v[u];
       }
     }
@@ -204,8 +223,8 @@ __device__ __forceinline__ void pack_tile(const CT* __restrict__ C, typename Ele
   __syncthreads();
 
   if constexpr (XF) {
-    for (int row = tid; row < 32 * 32; row += 256) {
-      float* r = tile + (row >> 5) * RP + (row & 31) * D;
+    for (int row = tid; row < 32 * OW; row += 256) {
+      float* r = tile + (row / OW) * RP + (row % OW) * D;
       float v[P + 1];
 #pragma unroll
       for (int n = 0; n <= P; ++n) v[n] = n < D ? r[n] : 0.0f;
@@ -221,27 +240,28 @@ __device__ __forceinline__ void pack_tile(const CT* __restrict__ C, typename Ele
   }
 
   {  // bias partial: 8 groups of 4 inputs, then a fixed-order sum
-    const int ol = tid & 31, grp = tid >> 5;
-    float s = 0.0f;
+    const int ol = tid % OW, grp = tid / OW;
+    if (grp < 8) {
+      float s = 0.0f;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) s += tile[(grp * 4 + q) * RP + ol * D];
-    bsum[grp][ol] = s;
+      for (int q = 0; q < 4; ++q) s += tile[(grp * 4 + q) * RP + ol * D];
+      lds.bsum[grp][ol] = s;
+    }
   }
   __syncthreads();
-  if (tid < 32 && o0 + tid < p.O32) {
+  if (tid < OW && o0 + tid < p.O32) {
     float s = 0.0f;
 #pragma unroll
-    for (int grp = 0; grp < 8; ++grp) s += bsum[grp][tid];
+    for (int grp = 0; grp < 8; ++grp) s += lds.bsum[grp][tid];
     bias_part[(size_t)ib * p.O32 + o0 + tid] = s;
   }
 
   if (ob < p.NBf) {
     const int kb_base = ib * 2 * P;  // 32 inputs * P values / 16 per k-block
-    for (int item = tid; item < 2 * P * 64; item += 256) {
-      const int kbl = item >> 6, lane = item & 63;
-      const int kb = kb_base + kbl;
+    for (int item = tid; item < 2 * P * 2 * OW; item += 256) {
+      const int kbl = item / (2 * OW), g = item / OW & 1, ol = item % OW;
+      const int kb = kb_base + kbl, lane = 32 * g + olo + ol;
       if (kb >= p.KB) continue;
-      const int ol = lane & 31, g = lane >> 5;
       const int r = kb / G::SGK, q = kb - r * G::SGK;
       const int s = q / G::KBG, h = q - s * G::KBG;
       float v[8];
@@ -257,15 +277,16 @@ __device__ __forceinline__ void pack_tile(const CT* __restrict__ C, typename Ele
     }
   }
 
-  for (int item = tid; item < P * 2 * 64; item += 256) {
-    const int e = item >> 7, rem = item & 127;
-    const int kbl = rem >> 6, lane = rem & 63;
-    const int il = lane & 31, g = lane >> 5;
-    const int kbx = ob * 2 + kbl;
+  // a piece: 8 outputs (o8 of the block's OW / 8) of one input at one degree
+  for (int item = tid; item < P * 32 * (OW / 8); item += 256) {
+    const int e = item / (32 * (OW / 8)), rem = item % (32 * (OW / 8));
+    const int o8 = rem >> 5, il = rem & 31;
+    const int kbx = ((o0 >> 3) + o8) >> 1, g = ((o0 >> 3) + o8) & 1;  // output k-block, half
+    const int lane = 32 * g + il;
     float v[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const int ol = 16 * kbl + 8 * g + j;
+      const int ol = 8 * o8 + j;
       // scaled by the degree d = e + 1, the factor of dT_d/dt = d U_{d-1}(t)
       v[j] = (e + 1 <= p.deg) ? tile[il * RP + ol * D + e + 1] * (float)(e + 1) : 0.0f;
     }
@@ -286,12 +307,13 @@ __device__ __forceinline__ void pack_tile(const CT* __restrict__ C, typename Ele
   }
 }
 
-template <int P, bool BF, typename CT, bool XF>
+template <int P, bool BF, typename CT, bool XF, int OW>
 __global__ void __launch_bounds__(256)
 k_pack(const CT* __restrict__ C, typename Elem<BF>::type* __restrict__ Cf,
        typename Elem<BF>::type* __restrict__ Cb, float* __restrict__ bias_part, PackPlanes pl,
        Plan p, int cal, XfArg<XF> xf, TanhJob tj) {
-  pack_tile<P, BF, CT, XF>(C, Cf, Cb, bias_part, pl, p, cal, xf, tj, blockIdx.x, blockIdx.y,
+  __shared__ PackLds<P, OW> lds;
+  pack_tile<P, BF, CT, XF, OW>(lds, C, Cf, Cb, bias_part, pl, p, cal, xf, tj, blockIdx.x, blockIdx.y,
                            blockIdx.x + (int64_t)gridDim.x * blockIdx.y);
 }
 
@@ -305,19 +327,27 @@ template <bool BF> struct PackJob {
   float* bias;
   PackPlanes pl;
   Plan p;
-  int cal, nx, nblocks;
+  int cal, nx, nblocks, ow;  // ow: outputs per block (pack_ow)
   TanhJob tj;
 };
 template <int P, bool BF>
 __global__ void __launch_bounds__(256)
 k_pack2(PackJob<BF> a, PackJob<BF> b) {
-  const int bid = blockIdx.x;
-  if (bid < a.nblocks)
-    pack_tile<P, BF, float, false>(a.C, a.Cf, a.Cb, a.bias, a.pl, a.p, a.cal, XfArg<false>{}, a.tj,
-                                   bid % a.nx, bid / a.nx, bid);
-  else
-    pack_tile<P, BF, float, false>(b.C, b.Cf, b.Cb, b.bias, b.pl, b.p, b.cal, XfArg<false>{}, b.tj,
-                                   (bid - a.nblocks) % b.nx, (bid - a.nblocks) / b.nx, bid - a.nblocks);
+  extern __shared__ __attribute__((aligned(16))) char pack_lds[];  // PackLds of the wider job
+  const bool first = (int)blockIdx.x < a.nblocks;
+  const int bid = first ? blockIdx.x : blockIdx.x - a.nblocks;
+  auto run = [&](const PackJob<BF>& j, auto owc) __attribute__((always_inline)) {
+    constexpr int OW = decltype(owc)::value;
+    pack_tile<P, BF, float, false, OW>(*reinterpret_cast<PackLds<P, OW>*>(pack_lds), j.C, j.Cf, j.Cb,
+                                       j.bias, j.pl, j.p, j.cal, XfArg<false>{}, j.tj, bid % j.nx,
+                                       bid / j.nx, bid);
+  };
+  auto tile = [&](const PackJob<BF>& j) __attribute__((always_inline)) {
+    if (P == 16 || j.ow == 8) run(j, std::integral_constant<int, 8>{});
+    else run(j, std::integral_constant<int, P == 16 ? 8 : 32>{});
+  };
+  if (first) tile(a);
+  else tile(b);
 }
 
 // out[o] = sum_k part[k][o] for k < nparts (row pitch `pitch`): 4 interleaved
@@ -621,14 +651,20 @@ static void launch_pack_t(const void* C, bool c_bf16, void* packed, const Plan& 
   // with one input block its bias partial is the bias itself
   float* bias = reinterpret_cast<float*>(reinterpret_cast<char*>(packed) +
                                          (p.NIB == 1 ? packed_biasf_offset(p) : packed_bias_offset(p)));
-  dim3 grid(p.NIB, p.O64 / 32);
-  if (c_bf16)
-    hipLaunchKernelGGL((k_pack<P, BF, uint16_t, XF>), grid, dim3(256), 0, s,
-                       reinterpret_cast<const uint16_t*>(C), Cf, Cb, bias, pack_planes(packed, p), p, 0, xf, tj);
-  else
-    hipLaunchKernelGGL((k_pack<P, BF, float, XF>), grid, dim3(256), 0, s,
-                       reinterpret_cast<const float*>(C), Cf, Cb, bias, pack_planes(packed, p), p,
-                       (int)is_al16(C), xf, tj);
+  auto go = [&](auto owc) {
+    constexpr int OW = decltype(owc)::value;
+    dim3 grid(p.NIB, p.O64 / OW);
+    if (c_bf16)
+      hipLaunchKernelGGL((k_pack<P, BF, uint16_t, XF, OW>), grid, dim3(256), 0, s,
+                         reinterpret_cast<const uint16_t*>(C), Cf, Cb, bias, pack_planes(packed, p),
+                         p, 0, xf, tj);
+    else
+      hipLaunchKernelGGL((k_pack<P, BF, float, XF, OW>), grid, dim3(256), 0, s,
+                         reinterpret_cast<const float*>(C), Cf, Cb, bias, pack_planes(packed, p), p,
+                         (int)is_al16(C), xf, tj);
+  };
+  if (P == 16 || pack_ow(p) == 8) go(std::integral_constant<int, 8>{});
+  else go(std::integral_constant<int, P == 16 ? 8 : 32>{});
 }
 
 template <bool XF>
@@ -649,7 +685,7 @@ bool pack_tanh_fusable(const Plan& p, const float* x) {
   // and the pack has blocks enough for one pass of tanh each: a pack with few
   // blocks (narrow outputs) would run the tanh stream serially (config 4's
   // 512 -> 64 layer: 639 us fused against ~45 us in two launches)
-  const int64_t blocks = (int64_t)p.NIB * (p.O64 / 32);
+  const int64_t blocks = pack_blocks(p);
   return x && p.I == p.I_sg && p.I % 4 == 0 && is_al16(x) &&
          blocks * 256 * kPackTanhU >= p.B * (int64_t)p.I / 4;
 }
@@ -662,8 +698,7 @@ void launch_pack(const void* C, bool c_bf16, void* packed, const Plan& p, hipStr
     tj.x = reinterpret_cast<const f32x4_t*>(x);
     tj.t = reinterpret_cast<f32x4_t*>(t);
     tj.n4 = p.B * p.I / 4;
-    const int64_t blocks = (int64_t)p.NIB * (p.O64 / 32);
-    tj.per = round_up(ceil_div(tj.n4, blocks), 256);
+    tj.per = round_up(ceil_div(tj.n4, pack_blocks(p)), 256);
   }
   if (xf) {
     XfArg<true> a;
@@ -693,17 +728,20 @@ static void launch_pack2_t(const float* Ca, void* pa, const Plan& qa, const Tanh
     j.p = q;
     j.cal = (int)is_al16(C);
     j.nx = q.NIB;
-    j.nblocks = q.NIB * (q.O64 / 32);
+    j.ow = pack_ow(q);
+    j.nblocks = (int)pack_blocks(q);
     j.tj = tj;
     return j;
   };
   const PackJob<BF> a = job(Ca, pa, qa, tja);
   const PackJob<BF> b = job(Cb_, pb, qb, TanhJob{nullptr, nullptr, 0, 0, qb.imap, qb.ima, qb.imb});
-  hipLaunchKernelGGL((k_pack2<P, BF>), dim3((unsigned)(a.nblocks + b.nblocks)), dim3(256), 0, s, a, b);
+  // at most 37 KB (P = 8)
+  const size_t lds = a.ow == 8 && b.ow == 8 ? sizeof(PackLds<P, 8>) : sizeof(PackLds<P, P == 16 ? 8 : 32>);
+  hipLaunchKernelGGL((k_pack2<P, BF>), dim3((unsigned)(a.nblocks + b.nblocks)), dim3(256), lds, s, a, b);
 }
 
 bool pack_pair_ok(const Plan& a, const Plan& b) {
-  return a.P == b.P && a.esz == b.esz && (int64_t)a.NIB * (a.O64 / 32) + (int64_t)b.NIB * (b.O64 / 32) < (1 << 30);
+  return a.P == b.P && a.esz == b.esz && pack_blocks(a) + pack_blocks(b) < (1 << 30);
 }
 
 void launch_pack_pair(const float* Ca, void* pa, const Plan& qa, bool reduce_a, const float* xa,
@@ -714,7 +752,7 @@ void launch_pack_pair(const float* Ca, void* pa, const Plan& qa, bool reduce_a, 
     tj.x = reinterpret_cast<const f32x4_t*>(xa);
     tj.t = reinterpret_cast<f32x4_t*>(ta);
     tj.n4 = qa.B * qa.I / 4;
-    tj.per = round_up(ceil_div(tj.n4, (int64_t)qa.NIB * (qa.O64 / 32)), 256);
+    tj.per = round_up(ceil_div(tj.n4, pack_blocks(qa)), 256);
   }
   const bool bf = qa.esz == 2;
 #define CKAN_PK2(PP, BB) launch_pack2_t<PP, BB>(Ca, pa, qa, tj, Cb_, pb, qb, s)
