@@ -38,7 +38,7 @@ typedef enum ckan_status {
 } ckan_status;
 
 typedef enum ckan_compute {
-  CKAN_COMPUTE_FP32 = 0,      /* fp32 MFMA (v_mfma_f32_32x32x2_f32)                 */
+  CKAN_COMPUTE_FP32 = 0,      /* fp32 results: fp32 MFMA, or fp32 operands as three exact bf16 planes */
   CKAN_COMPUTE_BF16 = 1       /* bf16 MFMA, fp32 accumulate (v_mfma_f32_32x32x16_bf16) */
 } ckan_compute;
 

@@ -55,6 +55,61 @@ __device__ __forceinline__ float split_sum(const float* __restrict__ src, size_t
 // ---------------------------------------------------------------------------
 // Forward
 // ---------------------------------------------------------------------------
+// A wave's NM x NN fragments, rows m0.., fragment columns nbw..: into y with
+// the bias, or, the reduction split over gridDim.z, into this split's partial
+// tile, which k_fwd_reduce adds in order.  nb0, bnf: the block's columns.
+template <int NM, int NN>
+__device__ __forceinline__ void fwd_store_tile(const f32x16_t (&acc)[NM][NN], int64_t m0, int nb0,
+                                               int bnf, int nbw, float* __restrict__ y,
+                                               float* __restrict__ part, const Plan& p,
+                                               const float* __restrict__ bias_f,
+                                               const float* __restrict__ bias_part, int nib,
+                                               float* __restrict__ bias_out, int lane) {
+  const int g = lane >> 5;
+  const bool split = gridDim.z > 1;
+  if (!split) {
+    // nib > 0: the bias from its per-input-block partials (and the first row
+    // of blocks fills the packed bias slot for later forwards)
+    if (nib > 0 && blockIdx.x == 0)
+      for (int idx = threadIdx.x; idx < bnf * 32; idx += 256) {
+        const int o = nb0 * 32 + idx;
+        if (o < p.O32) bias_out[o] = bias_from_parts(bias_part, nib, p.O32, o);
+      }
+#pragma unroll
+    for (int ni = 0; ni < NN; ++ni) {
+      const int o = (nbw + ni) * 32 + (lane & 31);
+      if (o >= p.O) continue;
+      const float bias = nib > 0 ? bias_from_parts(bias_part, nib, p.O32, o) : bias_f[o];
+#pragma unroll
+      for (int mi = 0; mi < NM; ++mi) {
+        const int64_t r0 = m0 + mi * 32;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int64_t r = r0 + acc_row(v, g);
+          if (r < p.B) y[r * p.O + o] = acc[mi][ni][v] + bias;
+        }
+      }
+    }
+    return;
+  }
+#pragma unroll
+  for (int ni = 0; ni < NN; ++ni) {
+    const int nb = nbw + ni;
+    if (nb >= p.NBf) continue;
+    const int o = nb * 32 + (lane & 31);
+#pragma unroll
+    for (int mi = 0; mi < NM; ++mi) {
+      const int64_t r0 = m0 + mi * 32;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int64_t r = r0 + acc_row(v, g);
+        if (r < p.B32)
+          part[((size_t)blockIdx.z * p.B32 + r) * p.O32 + o] = acc[mi][ni][v];
+      }
+    }
+  }
+}
+
 // Block = 4 waves arranged WGM x WGN; wave tile NM x NN fragments of 32x32.
 // The reduction runs over super-groups (SG): SGI inputs = SGK k-blocks.
 // With gridDim.z > 1 the SGs are split over blocks; each block writes its
@@ -212,50 +267,111 @@ k_fwd(const float* __restrict__ tc, const typename Elem<BF>::type* __restrict__ 
     __syncthreads();
   }
 
-  const bool split = gridDim.z > 1;
-  if (!split) {
-    // nib > 0: the bias from its per-input-block partials (and the first row
-    // of blocks fills the packed bias slot for later forwards)
-    if (nib > 0 && blockIdx.x == 0)
-      for (int idx = threadIdx.x; idx < BNF * 32; idx += 256) {
-        const int o = nb0 * 32 + idx;
-        if (o < p.O32) bias_out[o] = bias_from_parts(bias_part, nib, p.O32, o);
-      }
-#pragma unroll
-    for (int ni = 0; ni < NN; ++ni) {
-      const int o = (nb0 + wn * NN + ni) * 32 + (lane & 31);
-      if (o >= p.O) continue;
-      const float bias = nib > 0 ? bias_from_parts(bias_part, nib, p.O32, o) : bias_f[o];
-#pragma unroll
-      for (int mi = 0; mi < NM; ++mi) {
-        const int64_t r0 = m_blk + (wm * NM + mi) * 32;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int64_t r = r0 + acc_row(v, g);
-          if (r < p.B) y[r * p.O + o] = acc[mi][ni][v] + bias;
-        }
-      }
-    }
-    return;
-  }
+  fwd_store_tile<NM, NN>(acc, m_blk + wm * NM * 32, nb0, BNF, nb0 + wn * NN, y, part, p, bias_f,
+                         bias_part, nib, bias_out, lane);
+}
 
-  // split-K: write the partial tile; k_fwd_reduce adds the splits in order
+// The small tiles' forward in split mode: 64 rows x 128 outputs per block,
+// wave w holding output fragment w.  Bound by latency and, at one or two
+// super-groups per block, by the work of each: with the fp32 instruction a
+// k-block took its wave 1024 clk of MFMA, and every wave built all of the
+// basis.  Here a k-block is 12 bf16 MFMAs (384 clk), each wave builds and
+// splits a quarter of a unit's basis fragments (4 k-blocks x 64 rows) into
+// LDS, double-buffered, one barrier per unit, and its coefficient planes, which
+// no other wave reads, go straight to registers one unit ahead.  The five small
+// products are summed apart, as in the large-batch kernel.
+// Measured on the whole call, tanh and reduce included: 300 x 500 -> 300,
+// degree 6: 26.0 -> 21.2 us (error against 64 bits 2.3e-7 -> 1.7e-7).
+template <int P, bool XT>
+__global__ void __launch_bounds__(256)
+k_fwd_split_small(const float* __restrict__ tc, const uint16_t* __restrict__ Cf3,
+                  const float* __restrict__ bias_f, float* __restrict__ y,
+                  float* __restrict__ part, Plan p, int sg_per_split,
+                  const float* __restrict__ bias_part, int nib, float* __restrict__ bias_out,
+                  float* __restrict__ tout) {
+  typedef FwdGroup<P> G;
+  constexpr int FL = kFragLen<kSplit>;
+  constexpr int UPS = G::KBG;  // units of 4 k-blocks per super-group
+  constexpr int TV = 16 / P;   // basis arguments per lane, for 2 k-blocks
+  typedef __attribute__((ext_vector_type(TV))) float tvec_t;
+  static_assert(G::SGK == 4 * UPS && G::LANE_T == 2 * TV * UPS, "a unit is 4 k-blocks");
+  __shared__ __attribute__((aligned(16))) uint16_t lds[2][2][4][FL];  // [buffer][rows / 32][k-block]
+
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int g = lane >> 5;
+  const int64_t m_blk = (int64_t)blockIdx.x * 64;
+  const int nb0 = blockIdx.y * 4, nb = nb0 + wave;
+  const int nsg = p.I_sg / G::SGI;
+  const int u0 = blockIdx.z * sg_per_split * UPS;
+  const int u1 = min(nsg, (int)(blockIdx.z + 1) * sg_per_split) * UPS;
+
+  // the wave's share of the basis: rows mi, k-blocks 2 ks and 2 ks + 1 of a unit
+  const int mi = wave & 1, ks = wave >> 1;
+  const int64_t row = m_blk + mi * 32 + (lane & 31);
+  const bool rvalid = row < p.B;
+  const int64_t toff = (rvalid ? row : 0) * p.I_sg + g * G::LANE_T + ks * TV;
+  auto targ = [&](int u) __attribute__((always_inline)) {  // offset of unit u's arguments
+    return toff + (size_t)(u / UPS) * G::SGI + (u % UPS) * 2 * TV;
+  };
+  // columns past the last fragment read it again; their sums are not stored
+  const uint16_t* brow = Cf3 + (size_t)min(nb, p.NBf - 1) * p.KB * FL;
+
+  tvec_t tn;
+  Frag<kSplit> bn[4];
+  auto load = [&](int u) __attribute__((always_inline)) {
+    tn = *reinterpret_cast<const tvec_t*>(tc + targ(u));
 #pragma unroll
-  for (int ni = 0; ni < NN; ++ni) {
-    const int nb = nb0 + wn * NN + ni;
-    if (nb >= p.NBf) continue;
-    const int o = nb * 32 + (lane & 31);
+    for (int k = 0; k < 4; ++k) bn[k] = load_frag<kSplit>(brow + ((size_t)u * 4 + k) * FL, lane);
+  };
+  auto gen = [&](int u) __attribute__((always_inline)) {
+    float tv[TV], vals[16];
 #pragma unroll
-    for (int mi = 0; mi < NM; ++mi) {
-      const int64_t r0 = m_blk + (wm * NM + mi) * 32;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int64_t r = r0 + acc_row(v, g);
-        if (r < p.B32)
-          part[((size_t)blockIdx.z * p.B32 + r) * p.O32 + o] = acc[mi][ni][v];
-      }
+    for (int e = 0; e < TV; ++e) {
+      if constexpr (XT) tn[e] = input_map(tn[e], p.imap, p.ima, p.imb);
+      tv[e] = rvalid ? tn[e] : 0.0f;
     }
+    if constexpr (XT) {  // the first column block stores the mapped values, each once
+      if (blockIdx.y == 0 && rvalid) *reinterpret_cast<tvec_t*>(tout + targ(u)) = tn;
+    }
+#pragma unroll
+    for (int e = 0; e < TV; ++e) cheb_T<P>(tv[e], vals + e * P);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      // an affine map's argument is unbounded, and its T_d may overflow
+      const Frag<kSplit> f =
+          p.imap ? make_frag_split_any(vals + 8 * h) : make_frag_split(vals + 8 * h);
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        *reinterpret_cast<bf16x8_t*>(&lds[u & 1][mi][2 * ks + h][k * kFragElems + lane * 8]) = f.p[k];
+    }
+  };
+
+  f32x16_t acc[2][1], low[2];
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[m][0][v] = low[m][v] = 0.0f;
+
+  if (u0 < u1) {
+    load(u0);
+    gen(u0);
   }
+  for (int u = u0; u < u1; ++u) {
+    Frag<kSplit> bc[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) bc[k] = bn[k];
+    const bool more = u + 1 < u1;
+    if (more) load(u + 1);
+    __syncthreads();  // unit u's basis written; every wave is done reading unit u - 1's
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      mma_apart(acc[0][0], low[0], load_frag<kSplit>(lds[u & 1][0][k], lane), bc[k], acc[1][0], low[1],
+                load_frag<kSplit>(lds[u & 1][1][k], lane), bc[k]);
+    if (more) gen(u + 1);
+  }
+#pragma unroll
+  for (int m = 0; m < 2; ++m) acc[m][0] += low[m];
+  fwd_store_tile<2, 1>(acc, m_blk, nb0, 4, nb, y, part, p, bias_f, bias_part, nib, bias_out, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -2908,7 +3024,14 @@ FwdChoice choose_fwd(const Plan& p) {
   c.tiles_n = (int)ceil_div(p.NBf, c.bnf);
   const int nsg = p.I_sg / p.SGI;
   const int64_t tiles = (int64_t)c.tiles_m * c.tiles_n;
-  const int target = (c.tile == kFwdBig) ? kChipBlocks : 2 * kChipBlocks;
+  // The split-mode small tile takes one block per CU where that leaves a block
+  // at most 4 super-groups: fewer partials to write and add (300 x 500 -> 300,
+  // degree 6, with the reduce: 22.8 us at two blocks per CU, 20.6 at one; 200 x
+  // 512 -> 512, degree 16: 31.4 / 29.2).  With more super-groups the second
+  // block hides the first one's waits (512 x 1024 -> 1024, degree 8: 75.4 / 80).
+  const bool one_per_cu =
+      c.tile == kFwdBig || (c.tile == kFwdSmall64 && p.split && tiles * nsg <= 4 * kChipBlocks);
+  const int target = one_per_cu ? kChipBlocks : 2 * kChipBlocks;
   int splits = 1;
   if (tiles < target) splits = (int)ceil_div(target, tiles);
   // at least 4 super-groups per split for the large tile; the small-batch
@@ -2986,7 +3109,15 @@ static void fwd_dispatch(const float* x, float* t, const void* packed, float* y,
                              p, c.sg_per_split, bpart, nib_k, bias_out, nullptr);
         break;
       case kFwdSmall64:
-        if (xt)
+        if constexpr (!BF && P >= kSplitMinP) {
+          const uint16_t* cf3 = reinterpret_cast<const uint16_t*>(pk + packed_cf3_offset(p));
+          if (xt)
+            hipLaunchKernelGGL((k_fwd_split_small<P, true>), grid, dim3(256), 0, s, x, cf3, bias, y,
+                               part, p, c.sg_per_split, bpart, nib_k, bias_out, t);
+          else
+            hipLaunchKernelGGL((k_fwd_split_small<P, false>), grid, dim3(256), 0, s, t, cf3, bias, y,
+                               part, p, c.sg_per_split, bpart, nib_k, bias_out, nullptr);
+        } else if (xt)
           hipLaunchKernelGGL((k_fwd<P, BF, 2, 1, 1, 4, true>), grid, dim3(256), 0, s, x, Cf, bias, y,
                              part, p, c.sg_per_split, bpart, nib_k, bias_out, t);
         else

@@ -48,7 +48,10 @@ def _run(x, c, dy):
     (3000, 500, 257, 4),    # dC's wide and narrow tiles with remainders
     (16400, 40, 33, 8),     # many row tiles, one output pair
     (640, 1024, 128, 16),   # the forward reduction split over blocks
-    (130, 70, 500, 10), (300, 300, 96, 6),  # small batches: the fp32 forward, split gradients
+    # small batches: the 64 x 128 forward tile, its reduction whole, split and
+    # split to one super-group, a row and a column of fragments past the end
+    (65, 8, 65, 8), (130, 70, 500, 10), (300, 300, 96, 6), (257, 200, 129, 3), (512, 640, 1000, 7),
+    (65, 8, 100, 16), (100, 16, 97, 4),
 ])
 def test_split_fp32_tilings(B, I, O, deg):
     print(f"split fp32 B={B} I={I} O={O} deg={deg}", flush=True)
