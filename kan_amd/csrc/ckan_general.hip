@@ -606,7 +606,7 @@ __device__ __forceinline__ void gen_dx_body(const T* __restrict__ t, const T* __
 #pragma unroll
         for (int d = 0; d < DM; ++d) {
           if (d > 0 && d == dh) {
-            s[v] += sum * rs[3 * D];
+            s[v] += sum;  // du/dt once, at the store
             sum = T(0);
           }
           if (d < dn) {

@@ -9,6 +9,8 @@ and acos/cos against the recurrence); fp32 1e-5 up to degree 40 and 3e-7 per
 degree above: the three-term recurrence rounds at 2^-24 per step and its steps'
 errors add up coherently for the Jacobi family (2.1e-5 at degree 100 for the
 same recurrence run in plain fp32 FMAs)."""
+import math
+
 import pytest
 import torch
 
@@ -76,3 +78,53 @@ def test_fp64_tilings(B, I, O, deg, family):
 @pytest.mark.parametrize("family", [None, "jacobi"])
 def test_fp32_tilings(B, I, O, deg, family):
     _check(torch.float32, B, I, O, deg, family)
+
+
+def _hermite_case(scaling, domain, deg, low_only, B=90, I=18, O=21):
+    """x, coefficients, dy of a Hermite layer whose every degree counts: H_n
+    (He_n) grows as sqrt(2^n n!) (sqrt(n!)), so coefficient n is divided by it;
+    low_only keeps the degrees below a third."""
+    g = torch.Generator().manual_seed(deg + 100 * low_only)
+    x = torch.randn(B, I, generator=g) * 1.5 if domain is None else torch.rand(B, I, generator=g) * 7 - 2
+    n = torch.arange(deg + 1, dtype=torch.float64)
+    norm = torch.exp(0.5 * (torch.lgamma(n + 1) + (n * math.log(2.0) if scaling == "physicist" else 0)))
+    c = (torch.randn(I, O, deg + 1, generator=g, dtype=torch.float64) / norm).float()
+    if low_only:
+        c[..., deg // 3:] = 0
+    return x, c, torch.randn(B, O, generator=g)
+
+
+# every coefficient's gradient counts likewise: dC's degree n over its norm
+def _hermite_dc_scaled(dc, scaling):
+    n = torch.arange(dc.shape[-1], dtype=torch.float64)
+    norm = torch.exp(0.5 * (torch.lgamma(n + 1) + (n * math.log(2.0) if scaling == "physicist" else 0)))
+    return dc.detach().double().cpu() / norm
+
+
+@pytest.mark.parametrize("deg", [17, 20, 24, 26, 27, 40])  # dx in one chunk to 26, several above
+@pytest.mark.parametrize("scaling", ["physicist", "probabilist"])
+@pytest.mark.parametrize("domain", [None, (-2.0, 5.0)])
+@pytest.mark.parametrize("low_only", [False, True])
+def test_fp32_hermite_every_degree_counts(deg, scaling, domain, low_only):
+    """The Hermite bases are evaluated at 3 t, and dx carries that factor once
+    for every degree.  Tolerance: the fp32 recurrence at |u| <= 3 alone (plain
+    torch in fp32 against fp64, these inputs) is off by at most 9.2e-7."""
+    from kan_amd import HermiteKANLayer
+    print(f"general hermite {scaling} {domain} deg={deg} low={low_only}", flush=True)
+    x, c, dy = _hermite_case(scaling, domain, deg, low_only)
+    m = HermiteKANLayer(c.shape[0], c.shape[1], deg, scaling=scaling, domain=domain,
+                        normalize_domain=True)
+    with torch.no_grad():
+        m.hermite_coeffs.copy_(c)
+    m = m.cuda()
+    xd = x.cuda().requires_grad_(True)
+    y = m(xd)
+    y.backward(dy.cuda())
+    torch.cuda.synchronize()
+    y_ref, dx_ref, dc_ref = fo.family_forward_backward(
+        x.double(), c.double(), dy.double(), "hermite" if scaling == "physicist" else "hermite_e",
+        domain=domain)
+    assert _rel(y, y_ref) <= _tol(torch.float32, deg)
+    assert _rel(xd.grad, dx_ref) <= _tol(torch.float32, deg)
+    assert _rel(_hermite_dc_scaled(m.hermite_coeffs.grad, scaling),
+                _hermite_dc_scaled(dc_ref, scaling)) <= _tol(torch.float32, deg)
