@@ -301,29 +301,37 @@ __device__ __forceinline__ Frag<kSplit> make_frag_split(const float* v) {
   }
   return f;
 }
-// The planes of values a caller handed in (coefficients, dy), which may be
-// infinite, NaN or next to overflow.  A non-finite value goes to the l plane
-// alone: its only product is with the other operand's h plane, so it keeps the
-// sign and the infinity that the fp32 product has (in the h plane it would
-// also meet the m and l planes, whose signs differ).  A finite value whose
-// rounding to bf16 overflows takes the largest finite bf16 instead.
+// The planes of one value that may be infinite, NaN or next to overflow.  An
+// infinite value is +-1 in the h plane and itself in the l plane: l meets only
+// the other operand's h plane, which has that operand's sign (+-1 where it is
+// infinite too), so the product's infinity and sign are the fp32 product's,
+// and the h plane's products are finite beside it.  (Infinite in the h plane,
+// it would also meet the m and l planes, whose signs differ.)  A finite value
+// whose rounding to bf16 overflows is cut toward zero in the h plane.
+__device__ __forceinline__ void split_any(float v, __bf16& h, __bf16& m, __bf16& l) {
+  const uint32_t a = __float_as_uint(v) & 0x7fffffffu;
+  const bool nonfinite = a >= 0x7f800000u;
+  const float s = nonfinite ? copysignf(1.0f, v) : v;
+  const float hf = a >= 0x7f7f8000u ? __uint_as_float(__float_as_uint(s) & 0xffff0000u) : (float)(__bf16)s;
+  const float r = s - hf;
+  h = (__bf16)hf;
+  m = (__bf16)r;
+  l = nonfinite ? (__bf16)v : (__bf16)(r - (float)m);
+}
+// The planes of values a caller handed in (coefficients, dy).
 __device__ __forceinline__ Frag<kSplit> make_frag_split_any(const float* v) {
-  float s[8];
   bool odd = false;
 #pragma unroll
   for (int j = 0; j < 8; ++j) odd |= (__float_as_uint(v[j]) & 0x7fffffffu) >= 0x7f7f8000u;
   if (!odd) return make_frag_split(v);
-#pragma unroll
-  for (int j = 0; j < 8; ++j) s[j] = __builtin_isfinite(v[j]) ? v[j] : 0.0f;
   Frag<kSplit> f;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    const float h = __uint_as_float(__float_as_uint(s[j]) & 0xffff0000u);  // toward zero
-    const float r = s[j] - h;
-    const __bf16 m = (__bf16)r;
-    f.p[0][j] = (__bf16)h;
+    __bf16 h, m, l;
+    split_any(v[j], h, m, l);
+    f.p[0][j] = h;
     f.p[1][j] = m;
-    f.p[2][j] = __builtin_isfinite(v[j]) ? (__bf16)(r - (float)m) : (__bf16)v[j];
+    f.p[2][j] = l;
   }
   return f;
 }

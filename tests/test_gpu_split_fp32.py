@@ -94,3 +94,32 @@ def test_non_finite_and_extreme_values_stay_where_they_were(deg):
         sel = (basis[b].abs() > 0)
         assert torch.equal(got[sel], want[sel])
     assert torch.isfinite(dc[:, [o for o in range(O) if o not in (4, 6)]]).all()
+
+
+@pytest.mark.parametrize("B", [90, 600])
+@pytest.mark.parametrize("deg", [4, 8, 16])
+def test_infinite_coefficient_meets_infinite_gradient(B, deg):
+    """dx where an infinite coefficient meets an infinite upstream gradient:
+    the product's sign and infinity, as the fp32 product gives them.  Every
+    input is near 1 (U_{d-1} > 0 for all degrees there) and the coefficients of
+    output 7 share one sign, so no sum holds two infinities of opposite sign."""
+    print(f"split fp32 inf x inf B={B} deg={deg}", flush=True)
+    I, O = 40, 70
+    x, c, dy = _inputs(B, I, O, deg, 2)
+    x = 2.7 + 0.3 * torch.rand(B, I, generator=torch.Generator().manual_seed(deg))
+    for o, sign in ((7, 1.0), (33, -1.0)):
+        c[:, o] = sign * (c[:, o].abs() + 1e-3)
+        c[3, o, 2] = sign * float("inf")
+    dy[10, 7], dy[20, 7] = float("inf"), float("-inf")
+    dy[30, 33], dy[40, 33] = float("inf"), float("-inf")
+    dy[:, 33] = torch.where(torch.isinf(dy[:, 33]), dy[:, 33], -dy[:, 7].sign() * (dy[:, 33].abs() + 1e-3))
+    dy[[10, 20], 33] = 0.5 * torch.tensor([-1.0, 1.0])
+    dy[[30, 40], 7] = 0.5 * torch.tensor([-1.0, 1.0])
+    _, dx, _ = (v.cpu() for v in _run(x, c, dy))
+    inf = float("inf")
+    assert torch.equal(dx[10], torch.full((I,), inf)) and torch.equal(dx[20], torch.full((I,), -inf))
+    assert torch.equal(dx[30], torch.full((I,), -inf)) and torch.equal(dx[40], torch.full((I,), inf))
+    # input 3 of every other row: the infinite coefficients times a finite gradient
+    assert torch.equal(dx[:, 3], dy[:, 7].sign() * inf)
+    rest = [b for b in range(B) if b not in (10, 20, 30, 40)]
+    assert torch.isfinite(dx[rest][:, [i for i in range(I) if i != 3]]).all()
