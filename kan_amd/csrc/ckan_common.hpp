@@ -307,23 +307,18 @@ __device__ __forceinline__ Frag<kSplit> make_frag_split(const float* v) {
 // infinite too), so the product's infinity and sign are the fp32 product's,
 // and the h plane's products are finite beside it.  (Infinite in the h plane,
 // it would also meet the m and l planes, whose signs differ.)  A finite value
-// whose rounding to bf16 overflows is cut toward zero in the h plane.
+// whose rounding to bf16 overflows has the largest finite bf16 in the h plane.
 __device__ __forceinline__ void split_any(float v, __bf16& h, __bf16& m, __bf16& l) {
-  const uint32_t a = __float_as_uint(v) & 0x7fffffffu;
-  const bool nonfinite = a >= 0x7f800000u;
-  const float s = nonfinite ? copysignf(1.0f, v) : v;
-  const float hf = a >= 0x7f7f8000u ? __uint_as_float(__float_as_uint(s) & 0xffff0000u) : (float)(__bf16)s;
-  const float r = s - hf;
-  h = (__bf16)hf;
-  m = (__bf16)r;
-  l = nonfinite ? (__bf16)v : (__bf16)(r - (float)m);
+  constexpr float kMaxBf16 = 0x1.fep+127f;
+  const bool finite = __builtin_fabsf(v) < __builtin_inff();
+  h = (__bf16)(finite ? __builtin_amdgcn_fmed3f(v, -kMaxBf16, kMaxBf16) : copysignf(1.0f, v));
+  const float r = v - (float)h;  // exact; infinite or NaN as v
+  m = (__bf16)(finite ? r : 0.0f);
+  l = (__bf16)(r - (float)m);
 }
-// The planes of values a caller handed in (coefficients, dy).
-__device__ __forceinline__ Frag<kSplit> make_frag_split_any(const float* v) {
-  bool odd = false;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) odd |= (__float_as_uint(v[j]) & 0x7fffffffu) >= 0x7f7f8000u;
-  if (!odd) return make_frag_split(v);
+// The same for 8 values without a branch, for basis values under an affine
+// map, whose argument is unbounded, made beside the MFMAs.
+__device__ __forceinline__ Frag<kSplit> make_frag_split_far(const float* v) {
   Frag<kSplit> f;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
@@ -334,6 +329,13 @@ __device__ __forceinline__ Frag<kSplit> make_frag_split_any(const float* v) {
     f.p[2][j] = l;
   }
   return f;
+}
+// The planes of values a caller handed in (coefficients, dy).
+__device__ __forceinline__ Frag<kSplit> make_frag_split_any(const float* v) {
+  bool odd = false;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) odd |= (__float_as_uint(v[j]) & 0x7fffffffu) >= 0x7f7f8000u;
+  return odd ? make_frag_split_far(v) : make_frag_split(v);
 }
 
 template <int M> __device__ __forceinline__ Frag<M> make_frag(const float* v);

@@ -339,7 +339,7 @@ k_fwd_split_small(const float* __restrict__ tc, const uint16_t* __restrict__ Cf3
     for (int h = 0; h < 2; ++h) {
       // an affine map's argument is unbounded, and its T_d may overflow
       const Frag<kSplit> f =
-          p.imap ? make_frag_split_any(vals + 8 * h) : make_frag_split(vals + 8 * h);
+          p.imap ? make_frag_split_far(vals + 8 * h) : make_frag_split(vals + 8 * h);
 #pragma unroll
       for (int k = 0; k < 3; ++k)
         *reinterpret_cast<bf16x8_t*>(&lds[u & 1][mi][2 * ks + h][k * kFragElems + lane * 8]) = f.p[k];
@@ -759,8 +759,9 @@ struct FwdSplit {
   static_assert(LDS_BYTES <= 160 * 1024 && B_BYTES % 8192 == 0 && T_BYTES % 8192 == 0, "stage copies");
 };
 
-// Arguments as k_fwd_pipe's.
-template <int P, bool OT, int NN>
+// Arguments as k_fwd_pipe's.  AFF: an affine input map, whose unbounded argument
+// T_d may overflow.
+template <int P, bool OT, int NN, bool AFF>
 __global__ void __launch_bounds__(512)
 k_fwd_split(const float* __restrict__ tc, const uint16_t* __restrict__ Cf3,
             const float* __restrict__ bias_f, float* __restrict__ y, float* __restrict__ part,
@@ -850,7 +851,8 @@ k_fwd_split(const float* __restrict__ tc, const uint16_t* __restrict__ Cf3,
         cheb_T<P>(t, vals + u * P);
       }
 #pragma unroll
-      for (int h = 0; h < KBG; ++h) dst[h] = make_frag_split(vals + 8 * h);
+      for (int h = 0; h < KBG; ++h)
+        dst[h] = AFF ? make_frag_split_far(vals + 8 * h) : make_frag_split(vals + 8 * h);
     };
     auto load_b = [&](int kb, int np, Frag<kSplit> (&dst)[2]) __attribute__((always_inline)) {
 #pragma unroll
@@ -2492,7 +2494,9 @@ template <int P> constexpr int kDcXfBytes = (P + 1) * kMaxD * (int)sizeof(float)
 template <int P, int M, int H, int NN = 0>
 constexpr bool dc_xf_fits() { return DcPipe<P, M, H, NN>::kOk && DcPipe<P, M, H, NN>::LDS_BYTES + kDcXfBytes<P> <= 160 * 1024; }
 
-template <int P, int M, int H_, bool XF = false, int NN_ = 0>
+// AFF (split fp32): an affine input map, whose unbounded argument's T_d may
+// overflow.
+template <int P, int M, int H_, bool XF = false, int NN_ = 0, bool AFF = false>
 __global__ void __launch_bounds__(512)
 k_dc_pipe(const typename Elem<M>::type* __restrict__ dYc, const float* __restrict__ tc,
           const float* __restrict__ colsum_part, float* __restrict__ out, Plan p, int st_per_split,
@@ -2647,6 +2651,10 @@ k_dc_pipe(const typename Elem<M>::type* __restrict__ dYc, const float* __restric
         __bf16 w[3][RPT];
 #pragma unroll
         for (int r = 0; r < RPT; ++r) {
+          if constexpr (AFF) {
+            split_any(b[r], w[0][r], w[1][r], w[2][r]);
+            continue;
+          }
           const __bf16 h = (__bf16)b[r];
           const float rm = b[r] - (float)h;
           const __bf16 m = (__bf16)rm;
@@ -3132,18 +3140,22 @@ static void fwd_dispatch(const float* x, float* t, const void* packed, float* y,
             break;
           }
           const uint16_t* cf3 = reinterpret_cast<const uint16_t*>(pk + packed_cf3_offset(p));
-          auto launch = [&](auto OTc, auto NNc, std::atomic<uint32_t>& flag) {
-            constexpr bool OTv = decltype(OTc)::value;
+          auto launch_aff = [&](auto OTc, auto NNc, auto AFc, std::atomic<uint32_t>& flag) {
+            constexpr bool OTv = decltype(OTc)::value, AFv = decltype(AFc)::value;
             constexpr int NNv = decltype(NNc)::value;
             typedef FwdSplit<P, NNv> KV;
-            ensure_lds_limit(reinterpret_cast<const void*>(&k_fwd_split<P, OTv, NNv>), KV::LDS_BYTES, flag);
-            hipLaunchKernelGGL((k_fwd_split<P, OTv, NNv>), grid, dim3(KV::THREADS),
+            ensure_lds_limit(reinterpret_cast<const void*>(&k_fwd_split<P, OTv, NNv, AFv>), KV::LDS_BYTES, flag);
+            hipLaunchKernelGGL((k_fwd_split<P, OTv, NNv, AFv>), grid, dim3(KV::THREADS),
                                (size_t)KV::LDS_BYTES, s, t, cf3, bias, y, part, p, c.sg_per_split,
                                bpart, nib_k, nib_k > 0 ? bias_out : nullptr);
           };
+          auto launch = [&](auto OTc, auto NNc, std::atomic<uint32_t>* flag) {  // flag[2]
+            if (p.imap) launch_aff(OTc, NNc, std::integral_constant<bool, true>{}, flag[1]);
+            else launch_aff(OTc, NNc, std::integral_constant<bool, false>{}, flag[0]);
+          };
           typedef std::integral_constant<bool, true> OT1;
           typedef std::integral_constant<bool, false> OT0;
-          static std::atomic<uint32_t> lds_split[4];
+          static std::atomic<uint32_t> lds_split[4][2];
           if (c.bnf == 2) {
             if (out_tanh) launch(OT1{}, std::integral_constant<int, 2>{}, lds_split[0]);
             else launch(OT0{}, std::integral_constant<int, 2>{}, lds_split[1]);
@@ -3417,10 +3429,10 @@ BwdLayout bwd_layout(const Plan& p, bool need_dx_arg, bool need_dc_arg) {
   return L;
 }
 
-template <typename K>
-static void dc_pipe_launch(const void* dYc, const float* t, const float* colsum, float* part,
-                           float* dC, DcOut om, const Plan& p, const BwdLayout& L,
-                           hipStream_t s, const BasisXform* xf) {
+template <typename K, bool AFF>
+static void dc_pipe_launch_t(const void* dYc, const float* t, const float* colsum, float* part,
+                             float* dC, DcOut om, const Plan& p, const BwdLayout& L,
+                             hipStream_t s, const BasisXform* xf) {
   constexpr int P = K::PP, M = K::MM, H = K::H, NN = K::NNA;
   typedef typename K::E E;
   const bool split = L.dc_splits > 1;
@@ -3429,18 +3441,28 @@ static void dc_pipe_launch(const void* dYc, const float* t, const float* colsum,
     if (xf && !split) {  // the unsplit launch writes the whole gradient: it maps it
       static std::atomic<uint32_t> lds_xf{0};
       const int lds = K::LDS_BYTES + kDcXfBytes<P>;
-      ensure_lds_limit(reinterpret_cast<const void*>(&k_dc_pipe<P, M, H, true, NN>), lds, lds_xf);
-      hipLaunchKernelGGL((k_dc_pipe<P, M, H, true, NN>), grid, dim3(512), (size_t)lds, s,
+      ensure_lds_limit(reinterpret_cast<const void*>(&k_dc_pipe<P, M, H, true, NN, AFF>), lds, lds_xf);
+      hipLaunchKernelGGL((k_dc_pipe<P, M, H, true, NN, AFF>), grid, dim3(512), (size_t)lds, s,
                          reinterpret_cast<const E*>(dYc), t, colsum, dC, p, L.dc_st_per_split,
                          om, DcXf<true>{*xf});
       return;
     }
   }
   static std::atomic<uint32_t> lds_set{0};
-  ensure_lds_limit(reinterpret_cast<const void*>(&k_dc_pipe<P, M, H, false, NN>), K::LDS_BYTES, lds_set);
-  hipLaunchKernelGGL((k_dc_pipe<P, M, H, false, NN>), grid, dim3(512), K::LDS_BYTES, s,
+  ensure_lds_limit(reinterpret_cast<const void*>(&k_dc_pipe<P, M, H, false, NN, AFF>), K::LDS_BYTES, lds_set);
+  hipLaunchKernelGGL((k_dc_pipe<P, M, H, false, NN, AFF>), grid, dim3(512), K::LDS_BYTES, s,
                      reinterpret_cast<const E*>(dYc), t, colsum, split ? part : dC, p,
                      L.dc_st_per_split, split ? DcOut{kDcStore} : om, DcXf<false>{});
+}
+
+template <typename K>
+static void dc_pipe_launch(const void* dYc, const float* t, const float* colsum, float* part,
+                           float* dC, DcOut om, const Plan& p, const BwdLayout& L,
+                           hipStream_t s, const BasisXform* xf) {
+  if constexpr (K::MM == kSplit) {
+    if (p.imap) return dc_pipe_launch_t<K, true>(dYc, t, colsum, part, dC, om, p, L, s, xf);
+  }
+  dc_pipe_launch_t<K, false>(dYc, t, colsum, part, dC, om, p, L, s, xf);
 }
 
 bool dc_gemm_maps_basis(const Plan& p, const BwdLayout& L) {

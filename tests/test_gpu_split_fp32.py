@@ -123,3 +123,45 @@ def test_infinite_coefficient_meets_infinite_gradient(B, deg):
     assert torch.equal(dx[:, 3], dy[:, 7].sign() * inf)
     rest = [b for b in range(B) if b not in (10, 20, 30, 40)]
     assert torch.isfinite(dx[rest][:, [i for i in range(I) if i != 3]]).all()
+
+
+# B, O: the 64 x 128 forward tile, the 128- and 64-column large ones, both dC tiles
+@pytest.mark.parametrize("B,O", [(300, 70), (600, 70), (600, 40), (1100, 130)])
+@pytest.mark.parametrize("deg,far", [(4, 1e10), (8, 1e5), (16, 140.0)])
+def test_affine_map_basis_overflow(B, O, deg, far):
+    """Under an affine map t is unbounded: at t = ``far`` T_deg alone
+    overflows, and its products are infinite with their sign; where T_deg is
+    finite but above the largest bf16, they are finite.  The same results at
+    every batch size, and no other row or input is touched."""
+    from kan_amd.functional import ChebyKANFunction
+    print(f"split fp32 affine overflow B={B} O={O} deg={deg}", flush=True)
+    I = 40
+    x, c, dy = _inputs(B, I, O, deg, 3)
+    x, dy = x * 0.5, dy.clamp(-1, 1) * 0.5
+    c[4, 5, deg] = float("-inf")
+    near = ((3.3995e38 / 2 ** (deg - 1)) ** (1 / deg))
+    x[17, 4], x[50, 9] = far, near
+    basis = orc.basis_recurrence(x, deg)  # fp32
+    assert torch.isinf(basis[17, 4, deg]) and torch.isfinite(basis[17, 4, :deg]).all()
+    assert 3.3962e38 < basis[50, 9, deg] < 3.4028e38
+    xd, cd = x.cuda().requires_grad_(True), c.cuda().requires_grad_(True)
+    y = ChebyKANFunction.apply(xd, cd, "fp32", None, (1.0, 0.0))  # t = x
+    y.backward(dy.cuda())
+    y, dc = y.detach().cpu(), cd.grad.cpu()
+    cf = c.clone()
+    cf[4, 5, deg] = 0
+    b64 = orc.basis_recurrence(x.double(), deg)
+    y_ref = torch.einsum("bid,iod->bo", b64, cf.double())
+    inf = float("inf")
+    want = c[4, :, deg].sign() * inf
+    assert torch.equal(y[17], want)
+    rows, cols = [b for b in range(B) if b != 17], [o for o in range(O) if o != 5]
+    assert torch.equal(y[rows, 5], -torch.sign(basis[rows, 4, deg]) * inf)
+    assert _rel(y[50][cols], y_ref[50][cols]) <= TOL
+    rows.remove(50)
+    assert _rel(y[rows][:, cols], y_ref[rows][:, cols]) <= TOL
+    assert torch.equal(dc[4, :, deg], dy[17].sign() * inf)
+    assert _rel(dc[9, :, deg], torch.einsum("b,bo->o", b64[:, 9, deg], dy.double())) <= TOL
+    assert torch.isfinite(dc[4, :, :deg]).all() and torch.isfinite(dc[9]).all()
+    ins = [i for i in range(I) if i not in (4, 9)]
+    assert _rel(dc[ins], torch.einsum("bid,bo->iod", b64[:, ins], dy.double())) <= TOL
