@@ -1047,6 +1047,12 @@ bool ckan::layer_out_tanh_ok(const ckan_desc* desc) {
   return fwd_out_tanh_ok(plan_of(desc));
 }
 
+bool ckan::layer_reads_planes(const ckan_desc* desc) {
+  if (validate_desc(desc) != CKAN_OK || general_route(desc)) return false;
+  const Plan p = plan_of(desc);
+  return fwd_reads_planes(p, choose_fwd(p));
+}
+
 bool ckan::pack_pair_fits(const ckan_desc* a, const ckan_desc* b) {
   if (validate_desc(a) != CKAN_OK || validate_desc(b) != CKAN_OK || general_route(a) || general_route(b))
     return false;
@@ -1140,7 +1146,8 @@ bool ckan::self_pack_pair_fits(const ckan_desc* a, const ckan_desc* b) {
   const Plan pa = plan_of(a), pb = plan_of(b);
   const FwdChoice ca = choose_fwd(pa);
   // a's bias as per-input-block partials, summed by the tail
-  return pa.P == pb.P && pa.esz == pb.esz && dc_pack_ok(pa) && dc_pack_ok(pb) && dx_small_ok(pb) &&
+  return pa.P == pb.P && pa.esz == pb.esz && dc_pack_ok(pa) && dc_pack_ok(pb) &&
+         !fwd_reads_planes(pa, ca) && dx_small_ok(pb) && packed_has_cb(pb) &&
          (pa.NIB == 1 || fwd_sums_bias(pa, ca));
 }
 

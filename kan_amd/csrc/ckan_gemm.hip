@@ -2983,6 +2983,10 @@ static bool fwd_pipe_offsets_fit(const Plan& p) {
          (uint64_t)256 * p.I_sg * sizeof(float) < (1ull << 32);
 }
 
+bool fwd_reads_planes(const Plan& p, const FwdChoice& c) {
+  return p.split && (c.tile == kFwdSmall64 || (c.tile == kFwdBig && fwd_pipe_offsets_fit(p)));
+}
+
 // The one-launch small-batch forward needs a block per CU or more: 8-output
 // streams, so at least 2048 outputs.
 constexpr int kFwdColsMinBlocks = 256;
@@ -3134,7 +3138,7 @@ static void fwd_dispatch(const float* x, float* t, const void* packed, float* y,
         break;
       default:
         if constexpr (!BF && P >= kSplitMinP) {
-          if (!fwd_pipe_offsets_fit(p)) {  // per-lane copy offsets are 32-bit
+          if (!fwd_reads_planes(p, c)) {
             hipLaunchKernelGGL((k_fwd<P, BF, 2, 4, 4, 1>), grid, dim3(256), 0, s, t, Cf, bias, y,
                                part, p, c.sg_per_split, bpart, nib_k, bias_out, nullptr);
             break;

@@ -81,6 +81,9 @@ constexpr int kColsTanhRows = 8;
 inline bool fwd_reads_tcache(const FwdChoice& c) {
   return c.tile != kFwdStream32 && !(c.tile == kFwdCols && c.bm <= kColsTanhRows);
 }
+// Whether the forward reads Cf3 (else Cf).  Who rewrites a packed operand in
+// place must write the one that its forward reads (self_pack_pair_fits).
+bool fwd_reads_planes(const Plan& p, const FwdChoice& c);
 // split-K partials [splits][B32][O32] fp32, summed in order by k_fwd_reduce
 inline size_t fwd_ws_bytes(const Plan& p, const FwdChoice& c) {
   if (c.splits <= 1 && !fwd_streaming(c)) return 0;
@@ -316,6 +319,8 @@ int basis_check(const struct ckan_basis_spec* spec, int degree, BasisXform* xf);
 // Whether the layer of desc can take t_ready / out_tanh in pack_forward_ex.
 bool layer_reads_tcache(const struct ckan_desc* desc);
 bool layer_out_tanh_ok(const struct ckan_desc* desc);
+// Whether the layer's forward at desc's batch reads Cf3 (fwd_reads_planes).
+bool layer_reads_planes(const struct ckan_desc* desc);
 // Two consecutive layers a, b of a stack whose forward a stores tanh(y) into
 // b's tanh cache tb: both packs in one launch (b's pack needs nothing of a),
 // then a's forward, then b's (t_ready; out_tanh into outb when outb_tanh).
@@ -341,8 +346,10 @@ int pack2_forward_tail_ce(const struct ckan_desc* da, const void* Ca, void* pka,
 // A two-layer stack trained with cross-entropy whose packed operands the
 // step's dC launch keeps current, so that the step runs no pack:
 // self_pack_pair_fits: pack2_tail_ce_fits, both layers on the small dC path
-// with the packing epilogue (dc_pack_ok), b's dX on the small path, same P and
-// compute type, a's bias summed from its partials by the tail.
+// with the packing epilogue (dc_pack_ok), which writes Cf and Cb only: a's
+// forward reads Cf and b's dX is on the small path, which reads Cb (the planes
+// of both go stale at the first step); same P and compute type, a's bias
+// summed from its partials by the tail.
 // self_pack_layer: the pack that makes `packed` current after C changes other
 // than by a step (creation, a copy into C); the packs of the per-step path
 // without the tanh, so the same bytes.

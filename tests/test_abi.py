@@ -187,6 +187,31 @@ def test_small_backward_needs_no_dc_workspace():
     assert lib.ckan_bwd_workspace_bytes(ctypes.byref(big), 0, 1) > 0
 
 
+def test_self_packed_stack_reads_only_what_its_step_writes():
+    """The executor's two-layer cross-entropy step keeps the packed operands
+    current in its dC launch, which writes Cf and Cb but not the three-plane
+    operands of fp32 layers: the rule that admits a stack admits none whose
+    first layer's forward reads the planes.  Over the rule's whole range of
+    rows and widths, and past it."""
+    lib = ctypes.CDLL(_lib.LIB_PATH)
+    fits = getattr(lib, "_ZN4ckan19self_pack_pair_fitsEPK9ckan_descS2_")
+    planes = getattr(lib, "_ZN4ckan18layer_reads_planesEPK9ckan_desc")
+    fits.restype = planes.restype = ctypes.c_bool
+    admitted = refused_for_planes = 0
+    for B in (1, 32, 64, 65, 100, 128, 255, 256, 257, 300, 512, 513, 1000, 4096):
+        for I in (7, 32, 65, 784, 2048):
+            for O in (1, 10, 32, 33, 64, 65, 96, 128):
+                for deg in range(1, 17):
+                    a, b = _desc(B, I, O, deg), _desc(B, O, 10, deg)
+                    reads = planes(ctypes.byref(a))
+                    assert not (reads and (deg < 3 or B <= 64))
+                    if fits(ctypes.byref(a), ctypes.byref(b)):
+                        admitted += 1
+                        assert not reads, (B, I, O, deg)
+                    refused_for_planes += reads
+    assert admitted > 100 and refused_for_planes > 100
+
+
 def test_small_backward_grid_limit_routes_to_gemm():
     """The small vector-ALU dx puts 8 inputs per block on grid y, the small dC
     8 outputs: past 65535 blocks (524280 inputs / outputs) a layer leaves
