@@ -35,8 +35,8 @@
 // sizes, how far the reduction can be split to fill it.  Against the
 // vector-ALU register tiles that these kernels replaced (which put 64-128
 // blocks on the chip at these sizes), forward / dx / dC:
-//   2048 x 256 -> 256, degree 8, fp64:  483 / 112 / 532 -> 67 / 58 / 51 us
-//   4096 x 256 -> 128, degree 24, fp32: 1013 / 191 / 1534 -> 90 / 78 / 86 us
+//   2048 x 256 -> 256, degree 8, fp64:  483 / 112 / 532 -> 67 / 51 / 51 us
+//   4096 x 256 -> 128, degree 24, fp32: 1013 / 191 / 1534 -> 90 / 75 / 86 us
 // (36-47 TFLOP/s of products in fp64; 74-87 in fp32).
 #include "ckan_kernels.hpp"
 
@@ -436,7 +436,16 @@ k_gen_fwd(const T* __restrict__ t, const T* __restrict__ C, T* __restrict__ y, i
 // bytes a lane in order; else one (input, output) run of degrees per thread,
 // ds = DM.  A second row fragment per wave would halve
 // the LDS reads, which are far from the bound (4 per SIMD round of one matrix
-// instruction each), and spills.
+// instruction each), and spills.  With few outputs or many chunks a wave is bound
+// by its own chain of loads and recurrence steps: t is read ahead of the
+// products, and the recurrences go on from chunk to chunk.  dx alone, us, vector-ALU
+// tiles / t and the recurrences from degree 0 after each chunk / now:
+//   100000 x 64 -> 1, degree 4, fp64:  58 / 75 / 60
+//   16 x 64 -> 64, degree 500, fp64:   1292 / 1518 / 484
+//   16 x 64 -> 64, degree 1024, fp32:  2967 / 1913 / 469
+// Still behind the vector-ALU tiles where most of the 16 input columns are
+// padding: 100000 x 4 -> 4, degree 5, fp64, 19 / 23 / 21 (its dC 32349 -> 1364),
+// 100000 x 1 -> 16, degree 8, 14 / 29 / 27.
 template <int DM> struct GenDxLds {
   static constexpr int Q = (4 * DM + 15) / 32 * 32 + 16;      // 16 (mod 32), >= 4 DM
   static constexpr int S = 4 * Q + (Q % 64 == 16 ? 1 : 3);    // odd, 16 S = Q (mod 64)
@@ -489,9 +498,28 @@ __device__ __forceinline__ void gen_dx_body(const T* __restrict__ t, const T* __
   const T* crun = C + (size_t)(iok ? i0 + (q >> 4) : 0) * O * D;
   T* cdst = buf + (q >> 4) * L::S + ((q >> 2) & 3) * L::Q + (q & 3) * DM;
 
-  T s[4];  // this lane's (b, i) pairs: rows b0 + row(v, g), input i0 + l15
+  // this lane's (b, i) pairs: rows b0 + row(v, g), input i0 + l15; their t is
+  // read up front, ahead of its use after the products
+  T s[4], tv[4];
 #pragma unroll
-  for (int v = 0; v < 4; ++v) s[v] = T(0);
+  for (int v = 0; v < 4; ++v) {
+    const int64_t b = b0 + Mx<T>::row(v, g);
+    tv[v] = b < B && i0 + l15 < I ? t[b * I + i0 + l15] : T(0);
+    s[v] = T(0);
+  }
+  // their recurrences at the chunk's first degree, kept from chunk to chunk
+  // (one chunk: made in place): (up, u) = (U_{n-2}, U_{n-1}) at degree n, from
+  // n = 1; GEN: (pm, pc) = (P_{n-1}, P_n) and their derivatives (qm, qc) in u,
+  // from n = 0
+  constexpr int NR = WHOLE ? 1 : 4;
+  T rp[NR][2], rq[GEN ? NR : 1][2];
+  auto rec0 = [&](int r) __attribute__((always_inline)) {
+    rp[r][0] = T(0);
+    rp[r][1] = T(1);
+    if constexpr (GEN) rq[r][0] = rq[r][1] = T(0);
+  };
+#pragma unroll
+  for (int r = 0; r < NR; ++r) rec0(r);
 
   T pre[WHOLE ? 1 : DM], an[4];
   auto load_step = [&](int ob, int d0, int dn) {
@@ -583,26 +611,12 @@ __device__ __forceinline__ void gen_dx_body(const T* __restrict__ t, const T* __
     const int dh = WHOLE && sizeof(T) == 4 ? (D + 1) / 2 : 0;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const int64_t b = b0 + Mx<T>::row(v, g);
-      const T tv = b < B && i0 + l15 < I ? t[b * I + i0 + l15] : T(0);
+      const int r = WHOLE ? 0 : v;
+      if (WHOLE) rec0(r);
       T sum = T(0);
       if constexpr (GEN) {
-        // (pm, pc) = (P_{n-1}, P_n), (qm, qc) their derivatives in u, from n = 0:
         // P_n' = a_n P_{n-1} + (a_n u + b_n) P_{n-1}' - c_n P_{n-2}'
-        const T u = rs[3 * D] * tv;
-        T pm = T(0), pc = T(1), qm = T(0), qc = T(0);
-        auto step = [&](int n) {
-          asm volatile("" ::: "memory");  // coefficients read per step, not hoisted
-          const int k = n < D ? n : D - 1;
-          const T a_n = rs[k], fn = fma(a_n, u, rs[D + k]), cn = rs[2 * D + k];
-          const T pn = fma(fn, pc, -cn * pm);
-          const T qn = fma(a_n, pc, fma(fn, qc, -cn * qm));
-          pm = pc;
-          pc = pn;
-          qm = qc;
-          qc = qn;
-        };
-        for (int n = 1; n <= d0; ++n) step(n);
+        const T u = rs[3 * D] * tv[v];
 #pragma unroll
         for (int d = 0; d < DM; ++d) {
           if (d > 0 && d == dh) {
@@ -610,20 +624,21 @@ __device__ __forceinline__ void gen_dx_body(const T* __restrict__ t, const T* __
             sum = T(0);
           }
           if (d < dn) {
-            sum = fma(acc[d][v], qc, sum);
-            step(d0 + d + 1);
+            sum = fma(acc[d][v], rq[r][1], sum);
+            asm volatile("" ::: "memory");  // coefficients read per step, not hoisted
+            const int n = d0 + d + 1, k = n < D ? n : D - 1;
+            const T a_n = rs[k], fn = fma(a_n, u, rs[D + k]), cn = rs[2 * D + k];
+            const T pn = fma(fn, rp[r][1], -cn * rp[r][0]);
+            const T qn = fma(a_n, rp[r][1], fma(fn, rq[r][1], -cn * rq[r][0]));
+            rp[r][0] = rp[r][1];
+            rp[r][1] = pn;
+            rq[r][0] = rq[r][1];
+            rq[r][1] = qn;
           }
         }
       } else {
-        // dT_n/dt = n U_{n-1}: (up, u) = (U_{n-2}, U_{n-1}) at degree n, from
-        // (U_{-1}, U_0) at n = 1; degree 0 has no derivative
-        const T t2 = tv + tv;
-        T up = T(0), u = T(1);
-        for (int n = 1; n < d0; ++n) {
-          const T un = fma(t2, u, -up);
-          up = u;
-          u = un;
-        }
+        // dT_n/dt = n U_{n-1}; degree 0 has no derivative
+        const T t2 = tv[v] + tv[v];
         T deg = (T)d0;  // counted in T (exact)
 #pragma unroll
         for (int d = 0; d < DM; ++d) {
@@ -632,10 +647,10 @@ __device__ __forceinline__ void gen_dx_body(const T* __restrict__ t, const T* __
             sum = T(0);
           }
           if (d < dn && (d > 0 || d0 > 0)) {
-            sum = fma(acc[d][v] * deg, u, sum);
-            const T un = fma(t2, u, -up);
-            up = u;
-            u = un;
+            sum = fma(acc[d][v] * deg, rp[r][1], sum);
+            const T un = fma(t2, rp[r][1], -rp[r][0]);
+            rp[r][0] = rp[r][1];
+            rp[r][1] = un;
           }
           deg += T(1);
         }
@@ -662,8 +677,7 @@ __device__ __forceinline__ void gen_dx_body(const T* __restrict__ t, const T* __
   for (int v = 0; v < 4; ++v) {
     const int64_t b = b0 + Mx<T>::row(v, g);
     if (b >= B) continue;
-    const T tv = t[b * I + i0 + l15];
-    const T slope = f.imap ? (T)f.ima : T(1) - tv * tv;
+    const T slope = f.imap ? (T)f.ima : T(1) - tv[v] * tv[v];
     dx[b * I + i0 + l15] = (GEN ? s[v] * rs[3 * D] : s[v]) * slope;  // du/dt = rs[3 D] for a family
   }
 }
