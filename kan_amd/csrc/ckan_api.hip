@@ -126,8 +126,9 @@ inline const float* general_rec(const ckan_desc* d, const void* packed) {
   return reinterpret_cast<const float*>(static_cast<const char*>(packed) + general_rec_offset(d));
 }
 
-// The dimensions that the general kernels take: their 32-bit byte offsets
-// span a few rows of t and dy.
+// The dimensions that the general path takes, well inside what its kernels'
+// 32-bit byte offsets (16 rows of t and dy) span: those of its first kernels'
+// launch grids.
 int general_forward_shape_ok(const ckan_desc* d) {
   if (d->out_dim > 64 * 65535)
     return fail(CKAN_ERR_UNSUPPORTED, "out_dim %d above %d is not supported by the general "

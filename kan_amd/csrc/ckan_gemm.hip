@@ -968,8 +968,9 @@ template <int P, bool BF> struct FwdStream {
 // Waves per SIMD the streaming kernel asks the compiler to fit.  The grid
 // runs 16 waves per CU; at more than 128 registers a lane only 3 fit per
 // SIMD and the last quarter of the waves runs as a second round.  The bf16
-// kernels of degree 8 and 16 fit 4 per SIMD without spilling; the others
-// keep the default (they would spill).
+// kernels of degrees 5-16 fit 4 per SIMD without spilling, but for the one of
+// degrees 5-8 at 33-64 rows, which spills 4 registers; the others keep the
+// default (they would spill more).
 template <int P, bool BF> struct StreamWaves { static constexpr int v = (BF && P >= 8) ? 4 : 1; };
 
 template <int P, bool BF, int NMS, bool TPRE>
@@ -2977,7 +2978,9 @@ k_dc_pipe(const typename Elem<M>::type* __restrict__ dYc, const float* __restric
 static constexpr int kChipBlocks = 256;
 
 // The pipelined forward addresses its copies as a block base plus a per-lane
-// 32-bit offset: up to 4 output fragments of coefficients, 256 tanh rows.
+// 32-bit offset: up to 4 output fragments of coefficients, 256 tanh rows.  (The
+// split one has no such limit on its coefficients; past it those layers, of
+// over half a million inputs, stay on k_fwd.)
 static bool fwd_pipe_offsets_fit(const Plan& p) {
   return (uint64_t)4 * p.KB * kFragElems * p.esz < (1ull << 32) &&
          (uint64_t)256 * p.I_sg * sizeof(float) < (1ull << 32);
@@ -3018,9 +3021,7 @@ FwdChoice choose_fwd(const Plan& p) {
     c.sg_per_split = 4 * spw;
     return c;
   }
-  if (p.B <= 32) {
-    c.tile = kFwdSmall32; c.bm = 32; c.bnf = 4;
-  } else if (p.B <= 64 || (p.B <= 512 && ceil_div(p.B, 256) * ceil_div(p.NBf, 4) < 64)) {
+  if (p.B <= 512 && ceil_div(p.B, 256) * ceil_div(p.NBf, 4) < 64) {
     // at most 2 output fragments: 2 x 2 waves, none idle (config 2's 784 -> 64
     // forward 13.4 -> 10.6 us with the tanh in the kernel)
     if (p.NBf <= 2) {
@@ -3104,14 +3105,6 @@ static void fwd_dispatch(const float* x, float* t, const void* packed, float* y,
     dim3 grid(c.tiles_m, c.tiles_n, c.splits);
     switch (c.tile) {
       // xt: the kernel maps x itself and stores the tanh cache t
-      case kFwdSmall32:
-        if (xt)
-          hipLaunchKernelGGL((k_fwd<P, BF, 1, 1, 1, 4, true>), grid, dim3(256), 0, s, x, Cf, bias, y,
-                             part, p, c.sg_per_split, bpart, nib_k, bias_out, t);
-        else
-          hipLaunchKernelGGL((k_fwd<P, BF, 1, 1, 1, 4>), grid, dim3(256), 0, s, t, Cf, bias, y, part,
-                             p, c.sg_per_split, bpart, nib_k, bias_out, nullptr);
-        break;
       case kFwdSmall64N2:
         if (xt)
           hipLaunchKernelGGL((k_fwd<P, BF, 1, 1, 2, 2, true>), grid, dim3(256), 0, s, x, Cf, bias, y,
@@ -3241,8 +3234,7 @@ bool fwd_sums_bias(const Plan& p, const FwdChoice& c) {
 }
 
 bool fwd_maps_x_ok(const Plan& p, const FwdChoice& c, const float* x) {
-  return (c.tile == kFwdSmall32 || c.tile == kFwdSmall64 || c.tile == kFwdSmall64N2) &&
-         p.I == p.I_sg && p.I % 4 == 0 &&
+  return (c.tile == kFwdSmall64 || c.tile == kFwdSmall64N2) && p.I == p.I_sg && p.I % 4 == 0 &&
          is_al16(x);
 }
 

@@ -203,7 +203,7 @@ struct GenFwd {
   int dc, nch;         // degrees per chunk, chunks
   int dp, s;           // LDS strides (elements)
   int rec_elems;
-  int mblocks, nblocks;
+  int mblocks;
 };
 constexpr int kFwdVecs = 9;  // 16-byte pieces of a WHOLE tile that a thread stages
 template <int NN> __host__ __device__ constexpr int fwd_stride(int dp) {
@@ -913,9 +913,8 @@ static bool gen_fwd_launch(const T* t, const T* C, T* y, int64_t B, int I, int O
   f.wk = wk;
   const int WM = kWaves / wk;
   f.mblocks = (int)((mt + WM - 1) / WM);
-  f.nblocks = (int)nt;
   ensure_lds_limit(reinterpret_cast<const void*>(&k_gen_fwd<T, NM, NN, WHOLE>), kMaxLds, lds_done);
-  hipLaunchKernelGGL((k_gen_fwd<T, NM, NN, WHOLE>), dim3((unsigned)f.mblocks * f.nblocks), dim3(512),
+  hipLaunchKernelGGL((k_gen_fwd<T, NM, NN, WHOLE>), dim3((unsigned)f.mblocks * (unsigned)nt), dim3(512),
                      (size_t)bytes(wk), s, t, C, y, B, I, O, D, f, rec);
   return true;
 }

@@ -69,8 +69,12 @@ def _backward_workspace(device: torch.device, desc, need_dx: bool, need_dc: bool
 # own operands for its backward.  Code that writes the coefficients through a
 # raw pointer (a C-ABI call) must advance the version itself, as kan_amd.optim
 # does (torch.autograd.graph.increment_version).  Entries die with their tensor; one packed
-# buffer per live coefficient tensor stays allocated (2 I O P bytes in bf16,
-# about 4 I O P in fp32).  clear_pack_cache() drops them all.
+# buffer per live coefficient tensor stays allocated: with P the degree padded
+# to 2, 4, 8 or 16, 4 I O P bytes in bf16; in fp32 8 I O P at degrees 1-2 and
+# 16 I O P at degrees 3-16 (20 I O P at up to 64 outputs), where the operands of
+# the large-batch products are held as three bf16 planes beside the fp32 ones;
+# above degree 16 the size of the fp32 coefficients.  clear_pack_cache() drops
+# them all.
 # Entries are keyed by id(tensor) and hold a weak reference to the tensor
 # (checked by identity on lookup; a tensor's == is elementwise, so weak-keyed
 # dictionaries cannot hold tensors) whose callback drops the entry.

@@ -76,7 +76,7 @@ def test_descriptor_validation(field, value, code):
 
 
 def test_high_degree_sizes_and_limits():
-    """Degrees 17..1024 run on the vector-ALU kernels: the packed buffer is C
+    """Degrees 17..1024 run on the general kernels: the packed buffer is C
     as fp32 [I, O, D] followed, at the next 256-byte boundary, by the basis
     recurrence block (3 D + 2 floats); the input-map cache has row pitch I; no
     workspace."""
@@ -93,7 +93,7 @@ def test_high_degree_sizes_and_limits():
             assert lib.ckan_tcache_elems(d) == B * I
             assert lib.ckan_fwd_workspace_bytes(d) == 0
             assert lib.ckan_bwd_workspace_bytes(d, 1, 1) == 0
-    # the vector-ALU backward puts 8 inputs per block on grid y: in_dim <= 524280
+    # the general backward takes in_dim <= 524280
     big = _lib.make_desc(4, 524288, 2, 20, 0, 0)
     assert lib.ckan_backward(big, 256, 256, 256, 256, 256, 0, None, 0, None) == _lib.CKAN_ERR_UNSUPPORTED
     assert b"524280" in lib.ckan_last_error()

@@ -190,12 +190,12 @@ def _derivatives_graph(x, c, order):
 
 @pytest.mark.parametrize("B,I,O,deg,order", [
     (64, 8, 6, 14, 3),      # degree 17 derivative layer: the row-by-row operator
-    (100, 12, 10, 20, 1),   # degree 20 layer (vector-ALU forward)
+    (100, 12, 10, 20, 1),   # degree 20 layer (general forward)
     (50, 6, 5, 40, 2),
 ])
 def test_long_derivative_series_fp32(B, I, O, deg, order):
     """Past degree + order 16 the derivative coefficients come from the
-    row-by-row device operator and the derivative layer runs the vector-ALU
+    row-by-row device operator and the derivative layer runs the general
     forward: values, coefficient and input gradients, and the Jacobian."""
     print(f"long derivative series B={B} I={I} O={O} deg={deg} order={order}", flush=True)
     torch.manual_seed(B + deg)

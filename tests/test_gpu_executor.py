@@ -611,7 +611,7 @@ FAMILY_STACKS = [
     ([20, 16, 12, 6], [("jacobi", 4, 0.5, -0.3), ("hermite", 5, "physicist", None, 0.01),
                        ("cheb", 3)], None),
     # a finite-domain Hermite first layer (affine map), He_n, and a Jacobi
-    # layer above degree 16 (vector-ALU recurrence, optimizer fused)
+    # layer above degree 16 (its own recurrence, optimizer fused)
     ([10, 14, 8, 5], [("hermite", 4, "physicist", (-2.0, 2.0), 0.02),
                       ("hermite", 3, "probabilist", None, 0.2), ("jacobi", 20, 1.0, 1.0)],
      (-2.0, 2.0)),

@@ -1,9 +1,10 @@
 """GPU parity of ChebyKAN layers above degree 16 (the reference layer takes
 any degree: kan/layers/chebykan.py:21-51, kan/basis/chebyshev.py:78-101).
 
-Those layers run on the vector-ALU kernels in fp32, the degree axis in
-chunks of 17 (the cases below cover one chunk and a remainder of 1, whole
-chunks, several chunks with a short last one, degree 256, and up to 1024, the largest served).  The oracle runs in fp64 here: the fp32 acos/cos of the reference's
+Those layers run on the general kernels in fp32, the degree axis in even
+chunks of at most 17 (forward, dC) or 27 (dx) degrees (the cases below cover
+one chunk, several with a short last one, degree 256, and up to 1024, the
+largest served).  The oracle runs in fp64 here: the fp32 acos/cos of the reference's
 default path itself drifts by about d * 6e-8 at degree d, so the fp64 form is
 the honest yardstick.
 
@@ -189,7 +190,7 @@ def test_high_degree_executor_matches_oracle(optimizer):
     ex.close()
 
 
-# Jacobi / Hermite layers above degree 16: the vector-ALU kernels run the
+# Jacobi / Hermite layers above degree 16: the general kernels run the
 # family's own three-term recurrence (coefficients from the packed buffer's
 # recurrence block) and differentiate it for dx, so dC comes out in the
 # family's basis directly.  Oracle: the reference's op order
@@ -256,7 +257,7 @@ def test_high_degree_family_bf16_request_runs_fp32():
 def test_high_degree_hermite_finite_domain(scaling, B, I, O, deg):
     """HermiteKANLayer(domain=(lo, hi), normalize_domain=True) above degree
     16: the affine map onto [-3, 3] (kan/basis/hermite.py:102-112) runs in the
-    vector-ALU input-map launch, dx takes its constant chain factor; the
+    general path's input-map launch, dx takes its constant chain factor; the
     coefficient gradient accumulates over two backward calls."""
     import kan_amd
     from oracle import family_oracle as fo

@@ -61,12 +61,14 @@ def test_split_fp32_tilings(B, I, O, deg):
         assert _rel(got, want) <= TOL
 
 
+@pytest.mark.parametrize("B", [300, 600])  # the 64 x 128 forward tile, the large ones
 @pytest.mark.parametrize("deg", [4, 8, 16])
-def test_non_finite_and_extreme_values_stay_where_they_were(deg):
+def test_non_finite_and_extreme_values_stay_where_they_were(B, deg):
     """An infinite coefficient or upstream gradient reaches exactly the results
     that the fp32 products reach, with their sign; values next to overflow and
     far below 1 keep their precision."""
-    B, I, O = 600, 40, 70
+    print(f"split fp32 non-finite B={B} deg={deg}", flush=True)
+    I, O = 40, 70
     x, c, dy = _inputs(B, I, O, deg, 1)
     x = x.abs() * 0.3 + 0.05
     big = torch.finfo(torch.float32).max
