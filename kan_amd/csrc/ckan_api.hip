@@ -126,22 +126,13 @@ inline const float* general_rec(const ckan_desc* d, const void* packed) {
   return reinterpret_cast<const float*>(static_cast<const char*>(packed) + general_rec_offset(d));
 }
 
-// The dimensions that the general path takes, well inside what its kernels'
-// 32-bit byte offsets (16 rows of t and dy) span: those of its first kernels'
-// launch grids.
-int general_forward_shape_ok(const ckan_desc* d) {
-  if (d->out_dim > 64 * 65535)
-    return fail(CKAN_ERR_UNSUPPORTED, "out_dim %d above %d is not supported by the general "
-                "forward (degree above 16 or fp64)", d->out_dim, 64 * 65535);
-  return CKAN_OK;
-}
+// The inputs that the general backward takes (those of its first kernels'
+// launch grid).  Its kernels' 32-bit byte offsets span 16 rows of t and dy, far
+// past every dimension that validate_desc lets through.
 int general_backward_shape_ok(const ckan_desc* d) {
   if ((d->in_dim + 7) / 8 > 65535)
     return fail(CKAN_ERR_UNSUPPORTED, "in_dim %d above 524280 is not supported by the general "
                 "backward (degree above 16 or fp64)", d->in_dim);
-  if (d->out_dim > 128 * 65535)
-    return fail(CKAN_ERR_UNSUPPORTED, "out_dim %d above %d is not supported by the general "
-                "backward (degree above 16 or fp64)", d->out_dim, 128 * 65535);
   return CKAN_OK;
 }
 
@@ -389,7 +380,6 @@ int ckan_forward(const ckan_desc* desc, const float* x, const void* packed, floa
   if (!aligned16(packed) || !aligned16(t_cache))
     return fail(CKAN_ERR_INVALID_ARG, "packed and t_cache must be 16-byte aligned");
   if (general_route(desc)) {
-    if ((rc = general_forward_shape_ok(desc))) return rc;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     ProfScope ps("fwd_general", s);
     launch_forward_general<float>(x, static_cast<const float*>(packed), y, t_cache, desc->batch,
@@ -559,7 +549,6 @@ int forward_f64_impl(const ckan_desc* desc, const double* rec, const double* x,
   if ((rc = require_tanh_map(desc, "fp64 path"))) return rc;
   if (desc->batch == 0) return CKAN_OK;
   if (!x || !coeffs || !y || !t_cache) return fail(CKAN_ERR_INVALID_ARG, "x/coeffs/y/t_cache is NULL");
-  if ((rc = general_forward_shape_ok(desc))) return rc;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   ProfScope ps("fwd_f64", s);
   launch_forward_general<double>(x, coeffs, y, t_cache, desc->batch, desc->in_dim,
